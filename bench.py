@@ -180,16 +180,9 @@ def algorithmic_bytes(name, n, P, M_total, launches_per_sub, substeps, iters_tot
     return None
 
 
-def band_kernel_name(fp64):
-    """Template name of the MIC(0) band kernel the library runs for one precision."""
-    from ctypes import byref, c_int, c_void_p
-    from ffengine import pybindings as pb
-    from ffengine.ffengine import ffengine as lib
-    f = lib.FFAMD_mic0_band_shape
-    pb.init_lib_func(f, [c_int, c_void_p, c_void_p, c_void_p], None)
-    k, bt = c_int(), c_int()
-    pb.execute_lib_func(f, [1 if fp64 else 0, byref(k), byref(bt)])
-    return "micBandKernel<%s, %d, %d>" % ("double" if fp64 else "float", k.value, bt.value)
+def sweep_kernel_name(fp64):
+    """Template name of the MIC(0) sweep kernel the library runs for one precision (forward and backward launches)."""
+    return "columnSweepKernel<%s>" % ("double" if fp64 else "float")
 
 
 def measured_traffic(kernel):
@@ -665,8 +658,8 @@ def main():
     ap.add_argument("--cpu-substeps", type=int, default=3, help="cpu-calibration: timed substeps per engine")
     ap.add_argument("--no-cpu", action="store_true")
     ap.add_argument("--schedule", type=int, default=None, choices=[2, 4, 5],
-                    help="MIC(0) application: 2 = bands of hyperplanes, 4 = line pipeline, 5 = the bands "
-                         "replayed from a HIP graph (default: the engine's)")
+                    help="MIC(0) application: 2 = columns of lines, 4 = line pipeline, 5 = bands of hyperplanes from a "
+                         "replayed graph (default: the engine's)")
     ap.add_argument("--modes", default="fp64,mixed,mixed-reliable,fp32-preconditioner",
                     help="comma list of PCG modes: fp64, mixed (FP32 PCG restarted in FP64 refinement), "
                          "mixed-reliable (FP32 PCG with FP64 reliable updates), fp32-preconditioner (FP64 "
@@ -761,7 +754,7 @@ def main():
     launches = max(kt[dom]["launches"], 1)
     traffic, kname = None, dom
     if dom == "mic0_apply":
-        kname = band_kernel_name(main_mode == "fp64")
+        kname = sweep_kernel_name(main_mode == "fp64")
         traffic = measured_traffic(kname)
     # algorithmic HBM bytes / time of every kernel group that has a byte model
     # (SpMV, the transfers, the preconditioner, ...), as a fraction of 8 TB/s

@@ -1277,7 +1277,7 @@ int FFAMD_mic0_apply(int ni, int nj, int nk, double dx, double dt, const float *
         checkGrid(ni, nj, nk, dx);
         if (precision != 0 && precision != 1) throw std::domain_error("precision must be 0 (FP64) or 1 (FP32)");
         if (schedule < 0 || schedule > 4)
-            throw std::domain_error("schedule must be 0 (hyperplanes), 1 (tiles), 2 (bands), 3 (bands, device "
+            throw std::domain_error("schedule must be 0 (hyperplanes), 1 (tiles), 2 (columns), 3 (bands, device "
                                     "tile check) or 4 (line pipeline)");
         ff::Grid g{ni, nj, nk, dx};
         Scratch sc;

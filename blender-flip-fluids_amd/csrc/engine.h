@@ -155,7 +155,7 @@ public:
         _ps.setWarmStart(on);
     }
     bool getPressureSolverWarmStart() const { return _warmStart; }
-    // the MIC(0) application's schedule: 2 = bands of hyperplanes, 4 = the line pipeline
+    // the MIC(0) application's schedule: 2 = columns, 4 = the line pipeline, 5 = bands from a graph
     void setPressureSolverPreconditionerSchedule(int schedule) { _ps.setSchedule(schedule); }
     int getPressureSolverPreconditionerSchedule() const { return _ps.schedule(); }
     // constant viscosity (fluidsimulation.cpp:2565-2601, 303-312): the first

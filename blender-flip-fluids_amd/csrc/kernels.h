@@ -8,6 +8,7 @@
 
 #include <vector>
 
+#include "column_types.h"
 #include "ffdevice.h"
 #include "pencil_types.h"
 
@@ -318,7 +319,7 @@ struct PressureSys {
     int *rowOf;     // N+1 (exclusive scan of mask)
     int *rows;      // M: flat cell of each row (k,j,i order)
     int *cellRow;   // N: row of each cell, or -1
-    double *rhs, *diag, *ox, *oy, *oz, *mx, *my, *mz;  // M
+    double *rhs, *diag, *ox, *oy, *oz;  // M: off-diagonals toward +x/+y/+z
     int *nbr;       // 6M: -x,+x,-y,+y,-z,+z row ids or -1
     double *invdiag, *lx, *ly, *lz;  // M: MIC(0) factor (L entries toward +x/+y/+z)
     double *lmx, *lmy, *lmz;         // M: L entries of the -x/-y/-z neighbour rows toward the row
@@ -326,16 +327,11 @@ struct PressureSys {
     float *flmx, *flmy, *flmz;
     MicRec<double> *recFwd, *recBwd;  // M: band-sweep records (FP64)
     MicRec<float> *frecFwd, *frecBwd;  // M: band-sweep records (FP32 copies)
-    float *fdiag, *fox, *foy, *foz, *fmx, *fmy, *fmz;
     int *levelCount;  // L+1
     int *levelStart;  // L+1
     int *levelFill;   // L
     int *levelRows;   // M: rows grouped by i+j+k
-    // row bits of each 32-cell word of every (j, k) line along i, and the row
-    // of the word's first liquid cell (nj*nk lines x nw words; SpMV and the
-    // line-pipeline sweeps find neighbour rows in them)
-    LineWord *words;
-    int nw, ni, nj, nk;
+    int ni, nj, nk;
     int m;
     int nLevels;
 };
@@ -351,7 +347,9 @@ void pressureAssemble(Grid g, double dt, const float *u, const float *v, const f
                       const float *wu, const float *wv, const float *ww, const float *phi,
                       PressureSys &S, hipStream_t s, SolidTerms solid = SolidTerms{},
                       TensionView tension = TensionView{});
+// rows per hyperplane and their prefix sum; and the rows grouped by hyperplane
 void pressureLevels(Grid g, PressureSys &S, int *scanScratch, hipStream_t s);
+void pressureLevelRows(Grid g, PressureSys &S, hipStream_t s);
 // MIC(0) factor and application z = (L L^T)^-1 r; hyperplane-by-hyperplane
 // launches driven by the host copy of the level table
 void mic0Factor(PressureSys &S, const int *hLevelStart, hipStream_t s);
@@ -400,16 +398,12 @@ void mic0ApplyBands(Grid g, const PressureSys &S, const BandPlan &plan, const in
                     const double *r, double *y, double *z, hipStream_t s);
 void mic0ApplyBandsF(Grid g, const PressureSys &S, const BandPlan &plan, const int *tileLo, const int *tileHi,
                      const float *r, float *y, float *z, hipStream_t s);
-void spmv(const PressureSys &S, const double *x, double *y, hipStream_t s);
-void spmvF(const PressureSys &S, const float *x, float *y, hipStream_t s);
+// (vectors: in any one order)
 // y += (float)(sign * num/den) * x   (device scalars; den may be null -> scalar = num)
 void axpyFloatStep(double *y, const double *x, size_t n, const double *num, const double *den,
                    double sign, hipStream_t s);
 void axpyFloatStepF(float *y, const float *x, size_t n, const double *num, const double *den,
                     double sign, hipStream_t s);
-// q = A s and *sq = s . q (the dot in the dot()/dotf() order)
-void spmvDot(const PressureSys &S, const double *s, double *q, double *partial, double *sq, hipStream_t st);
-void spmvDotF(const PressureSys &S, const float *s, float *q, double *partial, double *sq, hipStream_t st);
 // a = (float)(num/den); x += a * s; r -= a * q; *rmax = |r|_inf (the absMax order);
 // rf (optional) receives (float)r; rmaxHost (optional) a mapped host copy of *rmax
 void pcgStep(double *x, const double *s, double *r, const double *q, size_t n, const double *num,
@@ -425,9 +419,6 @@ void widenAxpyStep(double *z, const float *zf, const double *s, size_t n, const 
 // x += (double)(float)(sign * num/den) * (double)p   (FP64 x, FP32 p)
 void axpyMixed(double *x, const float *p, size_t n, const double *num, const double *den, double sign,
                hipStream_t s);
-// r = b - A x (FP64 true residual)
-void residual(const PressureSys &S, const double *b, const double *x, double *r, hipStream_t s);
-void pressureToGrid(Grid g, const PressureSys &S, const double *x, float *p, hipStream_t s);
 void castToFloat(const double *a, float *b, size_t n, hipStream_t s);
 void addFloatToDouble(double *x, const float *d, size_t n, hipStream_t s);
 void mic0ToFloat(PressureSys &S, hipStream_t s);
@@ -455,11 +446,67 @@ size_t sampleBuckets(Grid g, int dir);
 void sampleAdjoint(Grid g, int dir, int np, const float *px, const float *py, const float *pz, const float *vbar,
                    int *key, int *slot, int *counts, int *offsets, int *perm, int *scanScratch, float *out,
                    hipStream_t s);
-// rhs[r] = cells[rows[r]];  cells[rows[r]] = x[r] (other cells untouched)
+// rhs[r] = cells[rows[r]]
 void gatherRows(const PressureSys &S, const double *cells, double *rhs, hipStream_t s);
-// x[r] = (double)cells[rows[r]] (a float cell grid onto the rows)
-void gatherRowsF(const PressureSys &S, const float *cells, double *x, hipStream_t s);
-void scatterRows(const PressureSys &S, const double *x, double *cells, hipStream_t s);
+
+// ---- the pressure system in the column layout (kernels_column.hip) ----
+// The layout of the current system (column_types.h) and the sweeps' exchange
+// buffers; the device buffers are owned by the caller.
+struct ColumnPlan {
+    int ncj = 0, nck = 0, ntj = 0, ntk = 0;  // columns and tiles along j and k
+    size_t maxSlices = 0, exJWords = 0, exKWords = 0;  // buffer sizes for the grid
+    int exSteps = 0;                         // hyperplanes a column can span
+    int slices = 0;                          // of the current system
+    ColumnRange *cols = nullptr;             // ncj * nck
+    int *order = nullptr;                    // tiles by PJ + PK
+    int *total = nullptr;                    // the slice count columnRanges found
+    SliceLinks *links = nullptr;             // maxSlices
+    int *slotRow = nullptr;                  // COL_SLICE maxSlices: row of each slot or -1
+    unsigned *exJ = nullptr, *exK = nullptr; // exchange words, cleared once
+    unsigned *counter = nullptr;             // ticket counter, cleared once
+    int *error = nullptr;                    // raised by a wait past waitTicks
+    unsigned base = 0, epoch = 0;            // counter value and last epoch used
+    long long waitTicks = 0;                 // longest wait in wall-clock ticks
+    size_t slots() const { return (size_t)slices * COL_SLICE; }
+};
+// matrix, right-hand side and MIC(0) records in slots (zeros where no row is)
+struct ColumnSys {
+    double *rhs, *diag, *ox, *oy, *oz;
+    float *fdiag, *fox, *foy, *foz;    // FP32 copies of the matrix
+    MicRec<double> *recFwd, *recBwd;
+    MicRec<float> *frecFwd, *frecBwd;  // FP32 copies of the factor
+};
+void columnShape(Grid g, ColumnPlan &cp);
+// tiles by PJ+PK, then PJ (the forward sweep's dependency order)
+void columnOrder(const ColumnPlan &cp, std::vector<int> &order);
+// the columns' ranges and slots for the pressure cells in mask; *cp.total
+// receives the slice count, which the caller reads into cp.slices
+void columnRanges(Grid g, const int *mask, ColumnPlan &cp, hipStream_t s);
+// links, slot rows, matrix and right-hand side from the assembled rows;
+// floats: the FP32 copies of the matrix too
+void columnFill(Grid g, const PressureSys &S, ColumnPlan &cp, ColumnSys &C, bool floats, hipStream_t s);
+// the sweeps' records from the rows' factor (invdiag, lx, ly, lz)
+void columnRecords(const PressureSys &S, const ColumnPlan &cp, ColumnSys &C, bool fp64, hipStream_t s);
+template <class T>
+void slotsFromRows(const ColumnPlan &cp, const T *rows, T *slots, hipStream_t s);
+template <class T>
+void rowsFromSlots(const ColumnPlan &cp, const T *slots, T *rows, hipStream_t s);
+// the rows' cells of a float grid onto the slots; and the slots onto the rows'
+// cells (other cells untouched)
+void slotsFromCells(const PressureSys &S, const ColumnPlan &cp, const float *cells, double *slots, hipStream_t s);
+template <class T>
+void cellsFromSlots(const PressureSys &S, const ColumnPlan &cp, const double *slots, T *cells, hipStream_t s);
+// q = A s and *sq = s . q (the dot in the dot()/dotf() order of the slots)
+void columnSpmvDot(const ColumnPlan &cp, const ColumnSys &C, const double *s, double *q, double *partial, double *sq,
+                   hipStream_t st);
+void columnSpmvDotF(const ColumnPlan &cp, const ColumnSys &C, const float *s, float *q, double *partial, double *sq,
+                    hipStream_t st);
+// r = b - A x
+void columnResidual(const ColumnPlan &cp, const ColumnSys &C, const double *b, const double *x, double *r,
+                    hipStream_t st);
+// z = (L L^T)^-1 r, y = the forward result (slots, distinct from r and z)
+void columnApply(ColumnPlan &cp, const ColumnSys &C, const double *r, double *y, double *z, hipStream_t s);
+void columnApplyF(ColumnPlan &cp, const ColumnSys &C, const float *r, float *y, float *z, hipStream_t s);
 
 // ---- MIC(0) application as a line pipeline (kernels_pencil.hip) ----
 // Pencils of 16 x 16 (j, k) lines along i, one workgroup each, one launch per

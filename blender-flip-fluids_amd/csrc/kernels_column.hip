@@ -1,0 +1,404 @@
+// kernels_column.hip -- the pressure system in the column layout
+// (column_types.h): building the layout and its matrix, the fused matrix
+// product, and the MIC(0) application as one launch per triangular sweep
+// (column_sweep.h).
+//
+// Why this layout: the rows' own order (k, j, i) gives a sweep 64 lines to
+// gather from per hyperplane and a neighbour id per term.  In columns a wave's
+// operands of one hyperplane are one slice of consecutive slots, and every
+// neighbour is at a fixed place of an adjacent slice, so the sweeps and the
+// product load whole slices at addresses known ahead of time.  The price is
+// the slots without rows: 22 hyperplanes of skew per column and the gaps.
+#include <stdexcept>
+#include <vector>
+
+#include "kernels.h"
+
+#include "column_hw.h"
+#include "column_sweep.h"
+
+namespace ff {
+
+namespace {
+
+// steps whose operands, and whose neighbours' words, are in flight
+constexpr int CPF = 6;
+template <class T>
+constexpr int CPX = sizeof(T) == 8 ? 4 : 3;
+constexpr int EMPTY_LO = 0x3fffffff;
+
+int ceilDiv(int a, int b) { return (a + b - 1) / b; }
+
+// lowest and highest hyperplane of the pressure cells of each column: one
+// workgroup per column, a wave per line
+__global__ __launch_bounds__(256) void columnRangeKernel(Grid g, const int *mask, int ncj, ColumnRange *cols) {
+    __shared__ int sLo[4], sHi[4];
+    const int ni = g.ni, nj = g.nj, nk = g.nk;
+    const int J0 = (blockIdx.x % ncj) * COL_J, K0 = (blockIdx.x / ncj) * COL_K;
+    const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
+    int lo = EMPTY_LO, hi = -1;
+    for (int line = wave; line < COL_SLICE; line += 4) {
+        const int j = J0 + line % COL_J, k = K0 + line / COL_J;
+        if (j >= nj || k >= nk) continue;
+        const int *m = mask + (size_t)ni * (j + (size_t)nj * k);
+        for (int i = lane; i < ni; i += 64)
+            if (m[i]) {
+                lo = min(lo, i + j + k);
+                hi = max(hi, i + j + k);
+            }
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        lo = min(lo, __shfl_xor(lo, o, 64));
+        hi = max(hi, __shfl_xor(hi, o, 64));
+    }
+    if (lane == 0) {
+        sLo[wave] = lo;
+        sHi[wave] = hi;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0)
+        cols[blockIdx.x] = ColumnRange{min(min(sLo[0], sLo[1]), min(sLo[2], sLo[3])),
+                                       max(max(sHi[0], sHi[1]), max(sHi[2], sHi[3])), 0, 0};
+}
+
+// the columns' slots in column order (one workgroup) and the total slice count
+__global__ __launch_bounds__(1024) void columnScanKernel(ColumnRange *cols, int nc, int *totalSlices) {
+    __shared__ int s[1024];
+    const int t = threadIdx.x, per = (nc + 1023) / 1024;
+    int sum = 0;
+    for (int q = 0; q < per; q++) {
+        const int c = t * per + q;
+        if (c < nc && cols[c].hi >= cols[c].lo) sum += cols[c].hi - cols[c].lo + 1;
+    }
+    s[t] = sum;
+    __syncthreads();
+    for (int off = 1; off < 1024; off <<= 1) {
+        const int add = t >= off ? s[t - off] : 0;
+        __syncthreads();
+        s[t] += add;
+        __syncthreads();
+    }
+    int run = s[t] - sum;
+    for (int q = 0; q < per; q++) {
+        const int c = t * per + q;
+        if (c >= nc || cols[c].hi < cols[c].lo) continue;
+        cols[c].base = COL_SLICE * (run - cols[c].lo);
+        run += cols[c].hi - cols[c].lo + 1;
+    }
+    if (t == 1023) *totalSlices = s[t];
+}
+
+// the slices' links: one workgroup per column
+__global__ __launch_bounds__(256) void columnLinksKernel(const ColumnRange *cols, int ncj, int nck, SliceLinks *links) {
+    const int c = blockIdx.x, cj = c % ncj, ck = c / ncj;
+    const ColumnRange own = cols[c], none{EMPTY_LO, -1, 0, 0};
+    const ColumnRange jm = cj > 0 ? cols[c - 1] : none, jp = cj + 1 < ncj ? cols[c + 1] : none;
+    const ColumnRange km = ck > 0 ? cols[c - ncj] : none, kp = ck + 1 < nck ? cols[c + ncj] : none;
+    auto at = [](const ColumnRange &r, int h) { return h >= r.lo && h <= r.hi ? r.base + COL_SLICE * h : -1; };
+    for (int h = own.lo + (int)threadIdx.x; h <= own.hi; h += 256)
+        links[(own.base + COL_SLICE * h) / COL_SLICE] =
+            SliceLinks{at(own, h - 1), at(own, h + 1), at(jm, h - 1), at(jp, h + 1),
+                       at(km, h - 1),  at(kp, h + 1),  c,             h};
+}
+
+// slot -> row, and the matrix and right-hand side in slots; two slices per
+// workgroup
+template <class T>
+__global__ __launch_bounds__(256) void columnFillKernel(Grid g, PressureSys S, int slices, const SliceLinks *links,
+                                                        int ncj, int *slotRow, double *rhs, double *diag, double *ox,
+                                                        double *oy, double *oz, T *fdiag, T *fox, T *foy, T *foz) {
+    const int slice = blockIdx.x * (256 / COL_SLICE) + threadIdx.x / COL_SLICE, place = threadIdx.x % COL_SLICE;
+    if (slice >= slices) return;
+    const int c = links[slice].col, h = links[slice].h;
+    const int j = (c % ncj) * COL_J + columnLineJ(place), k = (c / ncj) * COL_K + columnLineK(place), i = h - j - k;
+    int r = -1;
+    if (j < g.nj && k < g.nk && i >= 0 && i < g.ni) r = S.cellRow[i + (size_t)g.ni * (j + (size_t)g.nj * k)];
+    const size_t e = (size_t)slice * COL_SLICE + place;
+    const bool has = r >= 0;
+    const double d = has ? S.diag[r] : 0.0, x = has ? S.ox[r] : 0.0, y = has ? S.oy[r] : 0.0, z = has ? S.oz[r] : 0.0;
+    slotRow[e] = r;
+    rhs[e] = has ? S.rhs[r] : 0.0;
+    diag[e] = d;
+    ox[e] = x;
+    oy[e] = y;
+    oz[e] = z;
+    if (fdiag) {
+        fdiag[e] = (T)d;
+        fox[e] = (T)x;
+        foy[e] = (T)y;
+        foz[e] = (T)z;
+    }
+}
+
+// the sweeps' records from the factor's rows: forward the L entries of the
+// -x/-y/-z neighbour rows toward the row, backward the row's own
+template <class T>
+__global__ void columnRecordsKernel(PressureSys S, size_t slots, const int *slotRow, MicRec<T> *fwd, MicRec<T> *bwd) {
+    const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (e >= slots) return;
+    const int r = slotRow[e];
+    MicRec<T> f{T(0), T(0), T(0), T(0)}, b = f;
+    if (r >= 0) {
+        const int *nb = S.nbr + (size_t)6 * r;
+        f.inv = b.inv = (T)S.invdiag[r];
+        f.a = nb[0] >= 0 ? (T)S.lx[nb[0]] : T(0);
+        f.b = nb[2] >= 0 ? (T)S.ly[nb[2]] : T(0);
+        f.c = nb[4] >= 0 ? (T)S.lz[nb[4]] : T(0);
+        b.a = (T)S.lx[r];
+        b.b = (T)S.ly[r];
+        b.c = (T)S.lz[r];
+    }
+    fwd[e] = f;
+    bwd[e] = b;
+}
+
+template <class T>
+__global__ void slotsFromRowsKernel(size_t slots, const int *slotRow, const T *rows, T *out) {
+    const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (e < slots) out[e] = slotRow[e] >= 0 ? rows[slotRow[e]] : T(0);
+}
+template <class T>
+__global__ void rowsFromSlotsKernel(size_t slots, const int *slotRow, const T *in, T *rows) {
+    const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (e < slots && slotRow[e] >= 0) rows[slotRow[e]] = in[e];
+}
+// cells' values at the slots' rows (a float grid), and back
+__global__ void slotsFromCellsKernel(size_t slots, const int *slotRow, const int *rows, const float *cells, double *out) {
+    const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (e < slots) out[e] = slotRow[e] >= 0 ? (double)cells[rows[slotRow[e]]] : 0.0;
+}
+template <class T>
+__global__ void cellsFromSlotsKernel(size_t slots, const int *slotRow, const int *rows, const double *x, T *cells) {
+    const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (e < slots && slotRow[e] >= 0) cells[rows[slotRow[e]]] = (T)x[e];
+}
+
+// (A x) of one slot in the reference's order (sparsematrix.h:174-215: -z, -y,
+// -x, diagonal, +x, +y, +z).  The -x/-y/-z coefficients are the neighbour
+// slots' +x/+y/+z ones (the assembly computes both from the shared face by
+// the same expression).  A missing neighbour's term is left out.
+template <class T>
+struct ColumnMatrix {
+    const T *diag, *ox, *oy, *oz;
+};
+template <class T>
+__device__ __forceinline__ T columnProduct(const SliceLinks &L, size_t e, int place, const ColumnMatrix<T> &A,
+                                           const T *__restrict__ x) {
+    const int lj = columnLineJ(place), lk = columnLineK(place);
+    // first slot of the neighbour's slice and the place in it
+    const int bym = lj > 0 ? L.im : L.jm, byp = lj < COL_J - 1 ? L.ip : L.jp;
+    const int bzm = lk > 0 ? L.im : L.km, bzp = lk < COL_K - 1 ? L.ip : L.kp;
+    const bool hxm = L.im >= 0, hxp = L.ip >= 0, hym = bym >= 0, hyp = byp >= 0, hzm = bzm >= 0, hzp = bzp >= 0;
+    const int exm = hxm ? L.im + place : (int)e, exp = hxp ? L.ip + place : (int)e;
+    const int eym = hym ? bym + columnPlace(lj + COL_J - 1, lk) : (int)e;
+    const int eyp = hyp ? byp + columnPlace(lj + 1, lk) : (int)e;
+    const int ezm = hzm ? bzm + columnPlace(lj, lk + COL_K - 1) : (int)e;
+    const int ezp = hzp ? bzp + columnPlace(lj, lk + 1) : (int)e;
+    const T cmz = A.oz[ezm], cmy = A.oy[eym], cmx = A.ox[exm], cd = A.diag[e], cox = A.ox[e], coy = A.oy[e],
+            coz = A.oz[e];
+    const T xzm = x[ezm], xym = x[eym], xxm = x[exm], xr = x[e], xxp = x[exp], xyp = x[eyp], xzp = x[ezp];
+    T s = 0;
+    if (hzm) s += cmz * xzm;
+    if (hym) s += cmy * xym;
+    if (hxm) s += cmx * xxm;
+    s += cd * xr;
+    if (hxp) s += cox * xxp;
+    if (hyp) s += coy * xyp;
+    if (hzp) s += coz * xzp;
+    return s;
+}
+
+// q = A s with the partials of s . q, over the spans of the reductions (a span
+// is whole slices, a wave handles half a slice at a time)
+static_assert(REDUCE_THREADS % COL_SLICE == 0 && COL_SLICE % 64 == 0, "spans are whole slices, slices whole waves");
+constexpr int COL_SPMV_PARTS = 4;
+template <class T>
+__global__ __launch_bounds__(REDUCE_THREADS) void columnSpmvDotKernel(size_t slots, const SliceLinks *links,
+                                                                      ColumnMatrix<T> A, const T *__restrict__ x,
+                                                                      T *__restrict__ y, double *partial) {
+    const unsigned L = reduceLogicalBlock();
+    const size_t span = reduceSpan(slots, gridDim.x);
+    const size_t lo = (size_t)L * span, hi = lo + span < slots ? lo + span : slots;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / 64), lane = threadIdx.x % 64;
+    double acc = 0.0;
+    for (size_t b = lo + (size_t)wave * 64; b < hi; b += COL_SPMV_PARTS * REDUCE_THREADS) {
+        T s[COL_SPMV_PARTS];
+#pragma unroll
+        for (int u = 0; u < COL_SPMV_PARTS; u++) {
+            size_t e = b + (size_t)u * REDUCE_THREADS;
+            if (e >= hi) e = b;
+            s[u] = columnProduct<T>(links[e / COL_SLICE], e + lane, (int)(e % COL_SLICE) + lane, A, x);
+        }
+#pragma unroll
+        for (int u = 0; u < COL_SPMV_PARTS; u++) {
+            const size_t e = b + (size_t)u * REDUCE_THREADS + lane;
+            if (b + (size_t)u * REDUCE_THREADS < hi) {
+                y[e] = s[u];
+                acc += (double)x[e] * (double)s[u];
+            }
+        }
+    }
+    acc = reduceFold<0>(acc);
+    if (threadIdx.x == 0) partial[L] = acc;
+}
+
+// y = A x (b null) or y = b - A x
+template <class T>
+__global__ __launch_bounds__(256) void columnResidualKernel(size_t slots, const SliceLinks *links, ColumnMatrix<T> A,
+                                                            const T *b, const T *x, T *y) {
+    const unsigned g = gridDim.x, lb = g % XCDS == 0 ? (blockIdx.x % XCDS) * (g / XCDS) + blockIdx.x / XCDS : blockIdx.x;
+    const size_t e0 = (size_t)lb * 256 + (size_t)__builtin_amdgcn_readfirstlane((int)threadIdx.x / 64) * 64;
+    const int lane = threadIdx.x % 64;
+    if (e0 >= slots) return;
+    const T s = columnProduct<T>(links[e0 / COL_SLICE], e0 + lane, (int)(e0 % COL_SLICE) + lane, A, x);
+    y[e0 + lane] = b ? b[e0 + lane] - s : s;
+}
+
+template <class T, bool FWD>
+__global__ __launch_bounds__(COL_LANES *COL_WAVES) void columnSweepKernel(ColumnArgs<T, MicRec<T>> a) {
+    columnSweep<T, MicRec<T>, CPF, CPX<T>, FWD>(a, (int)threadIdx.x);
+}
+
+template <class T>
+void columnSweeps(ColumnPlan &cp, const T *r, T *y, T *z, const MicRec<T> *fwd, const MicRec<T> *bwd, hipStream_t st) {
+    ColumnArgs<T, MicRec<T>> a;
+    a.ncj = cp.ncj;
+    a.nck = cp.nck;
+    a.ntj = cp.ntj;
+    a.ntk = cp.ntk;
+    a.cols = cp.cols;
+    a.order = cp.order;
+    a.exJ = cp.exJ;
+    a.exK = cp.exK;
+    a.exSteps = cp.exSteps;
+    a.counter = cp.counter;
+    a.error = cp.error;
+    a.waitTicks = cp.waitTicks;
+    const dim3 grid(cp.ntj * cp.ntk), block(COL_LANES * COL_WAVES);
+    for (int sweep = 0; sweep < 2; sweep++) {
+        a.base = cp.base;
+        if (++cp.epoch == 0) cp.epoch = 1;  // 0 tags the cleared buffer
+        a.epoch = cp.epoch;
+        cp.base += grid.x;
+        a.in = sweep == 0 ? r : y;
+        a.out = sweep == 0 ? y : z;
+        a.rec = sweep == 0 ? fwd : bwd;
+        if (sweep == 0)
+            hipLaunchKernelGGL((columnSweepKernel<T, true>), grid, block, 0, st, a);
+        else
+            hipLaunchKernelGGL((columnSweepKernel<T, false>), grid, block, 0, st, a);
+    }
+    hipCheck(hipGetLastError(), "MIC(0) column sweep launch");
+}
+
+unsigned slotBlocks(size_t n) { return (unsigned)((n + 255) / 256); }
+
+}  // namespace
+
+void columnShape(Grid g, ColumnPlan &cp) {
+    cp.ncj = ceilDiv(g.nj, COL_J);
+    cp.nck = ceilDiv(g.nk, COL_K);
+    cp.ntj = cp.ncj;
+    cp.ntk = ceilDiv(cp.nck, COL_WAVES);
+    cp.exSteps = g.ni + COL_SKEW;
+    cp.maxSlices = (size_t)cp.ncj * cp.nck * cp.exSteps;
+    // four 32-bit parts: a double's two words
+    cp.exJWords = (size_t)cp.ncj * cp.ntk * COL_WAVES * cp.exSteps * COL_K * 4;
+    cp.exKWords = (size_t)cp.ntj * cp.ntk * cp.exSteps * COL_J * 4;
+}
+
+void columnOrder(const ColumnPlan &cp, std::vector<int> &order) {
+    order.clear();
+    for (int d = 0; d <= cp.ntj + cp.ntk - 2; d++)
+        for (int pj = 0; pj < cp.ntj; pj++)
+            if (d - pj >= 0 && d - pj < cp.ntk) order.push_back(pj + (d - pj) * cp.ntj);
+}
+
+void columnRanges(Grid g, const int *mask, ColumnPlan &cp, hipStream_t s) {
+    hipLaunchKernelGGL(columnRangeKernel, dim3(cp.ncj * cp.nck), dim3(256), 0, s, g, mask, cp.ncj, cp.cols);
+    hipLaunchKernelGGL(columnScanKernel, dim3(1), dim3(1024), 0, s, cp.cols, cp.ncj * cp.nck, cp.total);
+}
+
+void columnFill(Grid g, const PressureSys &S, ColumnPlan &cp, ColumnSys &C, bool floats, hipStream_t s) {
+    if (cp.slices == 0) return;
+    hipLaunchKernelGGL(columnLinksKernel, dim3(cp.ncj * cp.nck), dim3(256), 0, s, cp.cols, cp.ncj, cp.nck, cp.links);
+    hipLaunchKernelGGL(columnFillKernel<float>, dim3(slotBlocks(cp.slots())), dim3(256), 0, s, g, S, cp.slices, cp.links,
+                       cp.ncj, cp.slotRow, C.rhs, C.diag, C.ox, C.oy, C.oz, floats ? C.fdiag : nullptr, C.fox, C.foy,
+                       C.foz);
+}
+
+void columnRecords(const PressureSys &S, const ColumnPlan &cp, ColumnSys &C, bool fp64, hipStream_t s) {
+    if (cp.slices == 0) return;
+    if (fp64)
+        hipLaunchKernelGGL(columnRecordsKernel<double>, dim3(slotBlocks(cp.slots())), dim3(256), 0, s, S, cp.slots(),
+                           cp.slotRow, C.recFwd, C.recBwd);
+    else
+        hipLaunchKernelGGL(columnRecordsKernel<float>, dim3(slotBlocks(cp.slots())), dim3(256), 0, s, S, cp.slots(),
+                           cp.slotRow, C.frecFwd, C.frecBwd);
+}
+
+template <class T>
+void slotsFromRows(const ColumnPlan &cp, const T *rows, T *slots, hipStream_t s) {
+    if (cp.slices == 0) return;
+    hipLaunchKernelGGL(slotsFromRowsKernel<T>, dim3(slotBlocks(cp.slots())), dim3(256), 0, s, cp.slots(), cp.slotRow,
+                       rows, slots);
+}
+template <class T>
+void rowsFromSlots(const ColumnPlan &cp, const T *slots, T *rows, hipStream_t s) {
+    if (cp.slices == 0) return;
+    hipLaunchKernelGGL(rowsFromSlotsKernel<T>, dim3(slotBlocks(cp.slots())), dim3(256), 0, s, cp.slots(), cp.slotRow,
+                       slots, rows);
+}
+template void slotsFromRows<float>(const ColumnPlan &, const float *, float *, hipStream_t);
+template void slotsFromRows<double>(const ColumnPlan &, const double *, double *, hipStream_t);
+template void rowsFromSlots<float>(const ColumnPlan &, const float *, float *, hipStream_t);
+template void rowsFromSlots<double>(const ColumnPlan &, const double *, double *, hipStream_t);
+
+void slotsFromCells(const PressureSys &S, const ColumnPlan &cp, const float *cells, double *slots, hipStream_t s) {
+    if (cp.slices == 0) return;
+    hipLaunchKernelGGL(slotsFromCellsKernel, dim3(slotBlocks(cp.slots())), dim3(256), 0, s, cp.slots(), cp.slotRow,
+                       S.rows, cells, slots);
+}
+template <class T>
+void cellsFromSlots(const PressureSys &S, const ColumnPlan &cp, const double *slots, T *cells, hipStream_t s) {
+    if (cp.slices == 0) return;
+    hipLaunchKernelGGL(cellsFromSlotsKernel<T>, dim3(slotBlocks(cp.slots())), dim3(256), 0, s, cp.slots(), cp.slotRow,
+                       S.rows, slots, cells);
+}
+template void cellsFromSlots<float>(const PressureSys &, const ColumnPlan &, const double *, float *, hipStream_t);
+template void cellsFromSlots<double>(const PressureSys &, const ColumnPlan &, const double *, double *, hipStream_t);
+
+template <class T>
+static void launchColumnSpmvDot(const ColumnPlan &cp, ColumnMatrix<T> A, const T *x, T *y, double *partial, double *sq,
+                                hipStream_t st) {
+    if (cp.slices == 0) return;
+    const int nb = reduceBlocks(cp.slots());
+    hipLaunchKernelGGL(columnSpmvDotKernel<T>, dim3(nb), dim3(REDUCE_THREADS), 0, st, cp.slots(), cp.links, A, x, y,
+                       partial);
+    reduceFinish(partial, nb, sq, false, st);
+}
+void columnSpmvDot(const ColumnPlan &cp, const ColumnSys &C, const double *x, double *y, double *partial, double *sq,
+                   hipStream_t st) {
+    launchColumnSpmvDot<double>(cp, ColumnMatrix<double>{C.diag, C.ox, C.oy, C.oz}, x, y, partial, sq, st);
+}
+void columnSpmvDotF(const ColumnPlan &cp, const ColumnSys &C, const float *x, float *y, double *partial, double *sq,
+                    hipStream_t st) {
+    launchColumnSpmvDot<float>(cp, ColumnMatrix<float>{C.fdiag, C.fox, C.foy, C.foz}, x, y, partial, sq, st);
+}
+void columnResidual(const ColumnPlan &cp, const ColumnSys &C, const double *b, const double *x, double *r,
+                    hipStream_t st) {
+    if (cp.slices == 0) return;
+    const unsigned nb = (slotBlocks(cp.slots()) + XCDS - 1) / XCDS * XCDS;
+    hipLaunchKernelGGL(columnResidualKernel<double>, dim3(nb), dim3(256), 0, st, cp.slots(), cp.links,
+                       ColumnMatrix<double>{C.diag, C.ox, C.oy, C.oz}, b, x, r);
+}
+
+void columnApply(ColumnPlan &cp, const ColumnSys &C, const double *r, double *y, double *z, hipStream_t s) {
+    if (cp.slices > 0) columnSweeps<double>(cp, r, y, z, C.recFwd, C.recBwd, s);
+}
+void columnApplyF(ColumnPlan &cp, const ColumnSys &C, const float *r, float *y, float *z, hipStream_t s) {
+    if (cp.slices > 0) columnSweeps<float>(cp, r, y, z, C.frecFwd, C.frecBwd, s);
+}
+
+}  // namespace ff

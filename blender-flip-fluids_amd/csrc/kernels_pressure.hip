@@ -1,7 +1,7 @@
 // kernels_pressure.hip -- the variational pressure solve of the FLIP substep:
 // pressure-cell rows, divergence and 7-point ghost-fluid assembly, the MIC(0)
-// factor, its hyperplane-scheduled triangular solves, SpMV and the PCG vector
-// ops.
+// factor, its hyperplane-scheduled triangular solves and the PCG vector ops.
+// (The solver's matrix product and sweeps: kernels_column.hip.)
 //
 // Rows keep the reference's order (interior liquid cells in k,j,i order,
 // pressuresolver.cpp:118-159).  The factor and both triangular sweeps depend
@@ -129,11 +129,10 @@ __global__ void assembleKernel(Grid g, double dt, const float *u, const float *v
     }
     diag = fmax(diag, 0.0);
     S.diag[r] = diag;
-    S.mx[r] = off[0];
+    // the -x/-y/-z entries are the neighbour rows' +x/+y/+z ones: both rows
+    // compute -(weight / rho) * dt / dx^2 from the shared face
     S.ox[r] = off[1];
-    S.my[r] = off[2];
     S.oy[r] = off[3];
-    S.mz[r] = off[4];
     S.oz[r] = off[5];
 }
 
@@ -242,191 +241,6 @@ __global__ void backwardLevelKernel(const int *nbr, const T *invdiag, const T *l
     z[i] = x * invdiag[i];
 }
 
-// FixedSparseMatrix multiply (sparsematrix.h:174-215): ascending column order
-// (A x)[r] with the terms added in ascending column order: -z, -y, -x, diag,
-// +x, +y, +z.  Every load is issued up front (an absent neighbour reads x[r]
-// and its term is skipped by a select), so the row costs one round trip.
-// The -x/-y/-z coefficients are read as the neighbour rows' +x/+y/+z ones:
-// the assembly computes both from the same face by the same expression, so
-// they are the same bits, and those rows were just read by nearby threads
-// (mx, my, mz are kept for the other users of the matrix).
-// Row r's product with the 7-point matrix, (A x)_r, in the reference's order
-// (sparsematrix.h:174-215 over the row's entries by column: -z, -y, -x,
-// diagonal, +x, +y, +z).  The -x/-y/-z coefficients are the neighbour rows'
-// +x/+y/+z entries (the same bits: both sides assemble -(weight / rho) * dt /
-// dx^2 from the shared face).  A missing neighbour's term is left out, as
-// SparseMatrix leaves out absent entries.
-struct RowTopo {
-    int m;
-    const int *nbr;  // 6 per row: -x, +x, -y, +y, -z, +z rows or -1
-};
-
-template <class T>
-__device__ inline T rowProduct(int r, const RowTopo &t, const T *diag, const T *ox, const T *oy, const T *oz,
-                               const T *x) {
-    const int *nb = t.nbr + 6 * (size_t)r;
-    const int n0 = nb[0], n1 = nb[1], n2 = nb[2], n3 = nb[3], n4 = nb[4], n5 = nb[5];
-    const int a0 = n0 >= 0 ? n0 : r, a1 = n1 >= 0 ? n1 : r, a2 = n2 >= 0 ? n2 : r, a3 = n3 >= 0 ? n3 : r,
-              a4 = n4 >= 0 ? n4 : r, a5 = n5 >= 0 ? n5 : r;
-    const T cmz = oz[a4], cmy = oy[a2], cmx = ox[a0], cd = diag[r], cox = ox[r], coy = oy[r], coz = oz[r];
-    const T x4 = x[a4], x2 = x[a2], x0 = x[a0], xr = x[r], x1 = x[a1], x3 = x[a3], x5 = x[a5];
-    T s = 0;
-    if (n4 >= 0) s += cmz * x4;
-    if (n2 >= 0) s += cmy * x2;
-    if (n0 >= 0) s += cmx * x0;
-    s += cd * xr;
-    if (n1 >= 0) s += cox * x1;
-    if (n3 >= 0) s += coy * x3;
-    if (n5 >= 0) s += coz * x5;
-    return s;
-}
-
-// one row per thread; blocks renumbered so that each die streams one
-// contiguous eighth of the rows (its neighbour rows then sit in its L2)
-__device__ inline int dieRow() {
-    const unsigned b = blockIdx.x, g = gridDim.x;
-    const unsigned lb = g % XCDS == 0 ? (b % XCDS) * (g / XCDS) + b / XCDS : b;
-    return (int)(lb * blockDim.x + threadIdx.x);
-}
-
-template <class T>
-__global__ void spmvKernel(RowTopo t, const T *diag, const T *ox, const T *oy, const T *oz, const T *x, T *y) {
-    const int r = dieRow();
-    if (r >= t.m) return;
-    y[r] = rowProduct<T>(r, t, diag, ox, oy, oz, x);
-}
-
-// U rows' products at once: the neighbour lists of all U rows are loaded
-// before their values, so a thread keeps U lookups in flight.  Indices of
-// absent neighbours are clamped to the row itself (a valid address) and their
-// terms left out, as in rowProduct.
-template <class T, int U>
-__device__ inline void rowProducts(const int (&r)[U], const RowTopo &t, const T *__restrict__ diag,
-                                   const T *__restrict__ ox, const T *__restrict__ oy, const T *__restrict__ oz,
-                                   const T *__restrict__ x, T (&out)[U]) {
-    int nb[U][6];
-#pragma unroll
-    for (int u = 0; u < U; u++)
-#pragma unroll
-        for (int q = 0; q < 6; q++) nb[u][q] = t.nbr[6 * (size_t)r[u] + q];
-#pragma unroll
-    for (int u = 0; u < U; u++) {
-        const int q = r[u];
-        const int n0 = nb[u][0], n1 = nb[u][1], n2 = nb[u][2], n3 = nb[u][3], n4 = nb[u][4], n5 = nb[u][5];
-        const int a0 = n0 >= 0 ? n0 : q, a1 = n1 >= 0 ? n1 : q, a2 = n2 >= 0 ? n2 : q, a3 = n3 >= 0 ? n3 : q,
-                  a4 = n4 >= 0 ? n4 : q, a5 = n5 >= 0 ? n5 : q;
-        const T cmz = oz[a4], cmy = oy[a2], cmx = ox[a0], cd = diag[q], cox = ox[q], coy = oy[q], coz = oz[q];
-        const T x4 = x[a4], x2 = x[a2], x0 = x[a0], xr = x[q], x1 = x[a1], x3 = x[a3], x5 = x[a5];
-        T s = 0;
-        if (n4 >= 0) s += cmz * x4;
-        if (n2 >= 0) s += cmy * x2;
-        if (n0 >= 0) s += cmx * x0;
-        s += cd * xr;
-        if (n1 >= 0) s += cox * x1;
-        if (n3 >= 0) s += coy * x3;
-        if (n5 >= 0) s += coz * x5;
-        out[u] = s;
-    }
-}
-
-// Neighbour lookup of the fused SpMV: the rows' six neighbour ids (RowTopo,
-// the default) or, built with -DFF_SPMV_WORDS=1, the rows' cells and the line
-// words (WordTopo: 4 B per row instead of 24, one more dependent load; it
-// measured slower at 256^3, 148 ms against 107 ms of SpMV per 10 substeps).
-#ifndef FF_SPMV_WORDS
-#define FF_SPMV_WORDS 0
-#endif
-// The rows' neighbours found from the rows' cells and the line words (no
-// per-row neighbour ids): bit i%32 of word i/32 of line (j, k) marks a
-// pressure cell, whose row is the word's base plus the marked cells below it
-// in the word.  Rows lie on interior cells, so every neighbour cell is inside
-// the grid.
-struct WordTopo {
-    int m, ni, nj, nw;
-    const int *rows;  // flat cell of each row, (k*nj + j)*ni + i
-    const LineWord *words;
-};
-
-__device__ inline int wordRow(const LineWord *__restrict__ words, size_t line, int nw, int i) {
-    const LineWord w = words[line * nw + (i >> 5)];
-    const unsigned bit = 1u << (i & 31);
-    return (w.bits & bit) ? w.base + __builtin_popcount(w.bits & (bit - 1u)) : -1;
-}
-
-template <class T, int U>
-__device__ inline void rowProducts(const int (&r)[U], const WordTopo &t, const T *__restrict__ diag,
-                                    const T *__restrict__ ox, const T *__restrict__ oy, const T *__restrict__ oz,
-                                    const T *__restrict__ x, T (&out)[U]) {
-    int cell[U];
-#pragma unroll
-    for (int u = 0; u < U; u++) cell[u] = t.rows[r[u]];
-    int nb[U][6];
-#pragma unroll
-    for (int u = 0; u < U; u++) {
-        const int c = cell[u], i = c % t.ni, line = c / t.ni;
-        const size_t nj = (size_t)t.nj;
-        nb[u][0] = wordRow(t.words, line, t.nw, i - 1);
-        nb[u][1] = wordRow(t.words, line, t.nw, i + 1);
-        nb[u][2] = wordRow(t.words, line - 1, t.nw, i);
-        nb[u][3] = wordRow(t.words, line + 1, t.nw, i);
-        nb[u][4] = wordRow(t.words, line - nj, t.nw, i);
-        nb[u][5] = wordRow(t.words, line + nj, t.nw, i);
-    }
-#pragma unroll
-    for (int u = 0; u < U; u++) {
-        const int q = r[u];
-        const int n0 = nb[u][0], n1 = nb[u][1], n2 = nb[u][2], n3 = nb[u][3], n4 = nb[u][4], n5 = nb[u][5];
-        const int a0 = n0 >= 0 ? n0 : q, a1 = n1 >= 0 ? n1 : q, a2 = n2 >= 0 ? n2 : q, a3 = n3 >= 0 ? n3 : q,
-                  a4 = n4 >= 0 ? n4 : q, a5 = n5 >= 0 ? n5 : q;
-        const T cmz = oz[a4], cmy = oy[a2], cmx = ox[a0], cd = diag[q], cox = ox[q], coy = oy[q], coz = oz[q];
-        const T x4 = x[a4], x2 = x[a2], x0 = x[a0], xr = x[q], x1 = x[a1], x3 = x[a3], x5 = x[a5];
-        T s = 0;
-        if (n4 >= 0) s += cmz * x4;
-        if (n2 >= 0) s += cmy * x2;
-        if (n0 >= 0) s += cmx * x0;
-        s += cd * xr;
-        if (n1 >= 0) s += cox * x1;
-        if (n3 >= 0) s += coy * x3;
-        if (n5 >= 0) s += coz * x5;
-        out[u] = s;
-    }
-}
-
-// SpMV over the rows of the reduction spans, with each thread's partial of
-// s . q in the order of the standalone dot product (its rows in ascending
-// order, SPMV_ROWS at a time)
-constexpr int SPMV_ROWS = 4;
-template <class T, class Topo>
-__global__ __launch_bounds__(REDUCE_THREADS) void spmvDotKernel(Topo t, const T *__restrict__ diag,
-                                                                const T *__restrict__ ox, const T *__restrict__ oy,
-                                                                const T *__restrict__ oz, const T *__restrict__ x,
-                                                                T *__restrict__ y, double *partial) {
-    const unsigned L = reduceLogicalBlock();
-    const size_t span = reduceSpan((size_t)t.m, gridDim.x);
-    const size_t lo = (size_t)L * span, hi = lo + span < (size_t)t.m ? lo + span : (size_t)t.m;
-    double acc = 0.0;
-    for (size_t b = lo + threadIdx.x; b < hi; b += SPMV_ROWS * REDUCE_THREADS) {
-        int r[SPMV_ROWS];
-        bool ok[SPMV_ROWS];
-#pragma unroll
-        for (int u = 0; u < SPMV_ROWS; u++) {
-            const size_t q = b + (size_t)u * REDUCE_THREADS;
-            ok[u] = q < hi;
-            r[u] = (int)(ok[u] ? q : b);
-        }
-        T s[SPMV_ROWS];
-        rowProducts<T, SPMV_ROWS>(r, t, diag, ox, oy, oz, x, s);
-#pragma unroll
-        for (int u = 0; u < SPMV_ROWS; u++)
-            if (ok[u]) {
-                y[r[u]] = s[u];
-                acc += (double)x[r[u]] * (double)s[u];
-            }
-    }
-    acc = reduceFold<0>(acc);
-    if (threadIdx.x == 0) partial[L] = acc;
-}
-
 // x += a s; r -= a q with a the float-rounded step, and the partial max |r|
 template <class TX, class T>
 __global__ __launch_bounds__(REDUCE_THREADS) void pcgStepKernel(TX *x, const T *s, T *r, const T *q, size_t n,
@@ -447,14 +261,6 @@ __global__ __launch_bounds__(REDUCE_THREADS) void pcgStepKernel(TX *x, const T *
     }
     acc = reduceFold<1>(acc);
     if (threadIdx.x == 0) partial[L] = acc;
-}
-
-// r = b - A x
-__global__ void residualKernel(RowTopo t, const double *diag, const double *ox, const double *oy,
-                               const double *oz, const double *b, const double *x, double *r) {
-    const int q = dieRow();
-    if (q >= t.m) return;
-    r[q] = b[q] - rowProduct<double>(q, t, diag, ox, oy, oz, x);
 }
 
 // BLAS::addScaled(float alpha, ...) (blaswrapper.h:128-157): the step length
@@ -496,18 +302,6 @@ __global__ void gatherRowsKernel(int m, const int *rows, const double *cells, do
     int r = blockIdx.x * blockDim.x + threadIdx.x;
     if (r < m) rhs[r] = cells[rows[r]];
 }
-__global__ void gatherRowsFKernel(int m, const int *rows, const float *cells, double *x) {
-    int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r < m) x[r] = (double)cells[rows[r]];
-}
-__global__ void scatterRowsKernel(int m, const int *rows, const double *x, double *cells) {
-    int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r < m) cells[rows[r]] = x[r];
-}
-__global__ void toGridKernel(int m, const int *rows, const double *x, float *p) {
-    int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r < m) p[rows[r]] = (float)x[r];
-}
 __global__ void castKernel(const double *a, float *b, size_t n) {
     size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (q < n) b[q] = (float)a[q];
@@ -540,10 +334,13 @@ void pressureAssemble(Grid g, double dt, const float *u, const float *v, const f
 void pressureLevels(Grid g, PressureSys &S, int *scanScratch, hipStream_t s) {
     S.nLevels = g.ni + g.nj + g.nk - 2;
     hipCheck(hipMemsetAsync(S.levelCount, 0, sizeof(int) * (S.nLevels + 1), s), "hipMemsetAsync");
-    hipCheck(hipMemsetAsync(S.levelFill, 0, sizeof(int) * S.nLevels, s), "hipMemsetAsync");
     if (S.m > 0)
         hipLaunchKernelGGL(levelCountKernel, dim3(blocksFor(S.m, TPB)), dim3(TPB), 0, s, g, S);
     exclusiveScan(S.levelCount, S.levelStart, S.nLevels, scanScratch, s);
+}
+
+void pressureLevelRows(Grid g, PressureSys &S, hipStream_t s) {
+    hipCheck(hipMemsetAsync(S.levelFill, 0, sizeof(int) * S.nLevels, s), "hipMemsetAsync");
     if (S.m > 0)
         hipLaunchKernelGGL(levelScatterKernel, dim3(blocksFor(S.m, TPB)), dim3(TPB), 0, s, g, S);
 }
@@ -586,24 +383,6 @@ void mic0ApplyF(const PressureSys &S, const int *hs, const float *r, float *z, h
     micApply<float>(S, hs, S.finvdiag, S.flx, S.fly, S.flz, r, z, s);
 }
 
-static RowTopo topo(const PressureSys &S) { return RowTopo{S.m, S.nbr}; }
-// one row per thread over whole runs of XCDS blocks (so dieRow renumbers them)
-static unsigned dieBlocks(size_t m) {
-    const unsigned b = blocksFor(m, TPB);
-    return (b + XCDS - 1) / XCDS * XCDS;
-}
-
-void spmv(const PressureSys &S, const double *x, double *y, hipStream_t s) {
-    if (S.m == 0) return;
-    hipLaunchKernelGGL(spmvKernel<double>, dim3(dieBlocks(S.m)), dim3(TPB), 0, s, topo(S), S.diag, S.ox, S.oy,
-                       S.oz, x, y);
-}
-void spmvF(const PressureSys &S, const float *x, float *y, hipStream_t s) {
-    if (S.m == 0) return;
-    hipLaunchKernelGGL(spmvKernel<float>, dim3(dieBlocks(S.m)), dim3(TPB), 0, s, topo(S), S.fdiag, S.fox, S.foy,
-                       S.foz, x, y);
-}
-
 void axpyFloatStep(double *y, const double *x, size_t n, const double *num, const double *den,
                    double sign, hipStream_t s) {
     if (n == 0) return;
@@ -613,28 +392,6 @@ void axpyFloatStepF(float *y, const float *x, size_t n, const double *num, const
                     double sign, hipStream_t s) {
     if (n == 0) return;
     hipLaunchKernelGGL(axpyStepKernel<float>, dim3(blocksFor(n, TPB)), dim3(TPB), 0, s, y, x, n, num, den, sign);
-}
-
-template <class T>
-static void launchSpmvDot(const PressureSys &S, const T *diag, const T *ox, const T *oy, const T *oz, const T *x,
-                          T *y, double *partial, double *sq, hipStream_t st) {
-    const int nb = reduceBlocks(S.m);
-#if FF_SPMV_WORDS
-    WordTopo t{S.m, S.ni, S.nj, S.nw, S.rows, S.words};
-#else
-    RowTopo t = topo(S);
-#endif
-    hipLaunchKernelGGL((spmvDotKernel<T, decltype(t)>), dim3(nb), dim3(REDUCE_THREADS), 0, st, t, diag, ox, oy, oz,
-                       x, y, partial);
-    reduceFinish(partial, nb, sq, false, st);
-}
-void spmvDot(const PressureSys &S, const double *x, double *y, double *partial, double *sq, hipStream_t st) {
-    if (S.m == 0) return;
-    launchSpmvDot<double>(S, S.diag, S.ox, S.oy, S.oz, x, y, partial, sq, st);
-}
-void spmvDotF(const PressureSys &S, const float *x, float *y, double *partial, double *sq, hipStream_t st) {
-    if (S.m == 0) return;
-    launchSpmvDot<float>(S, S.fdiag, S.fox, S.foy, S.foz, x, y, partial, sq, st);
 }
 
 template <class TX, class T>
@@ -672,29 +429,9 @@ void axpyMixed(double *x, const float *p, size_t n, const double *num, const dou
     hipLaunchKernelGGL(axpyMixedKernel, dim3(blocksFor(n, TPB)), dim3(TPB), 0, s, x, p, n, num, den, sign);
 }
 
-void residual(const PressureSys &S, const double *b, const double *x, double *r, hipStream_t s) {
-    if (S.m == 0) return;
-    hipLaunchKernelGGL(residualKernel, dim3(dieBlocks(S.m)), dim3(TPB), 0, s, topo(S), S.diag, S.ox, S.oy, S.oz, b,
-                       x, r);
-}
-
-void pressureToGrid(Grid g, const PressureSys &S, const double *x, float *p, hipStream_t s) {
-    size_t n = (size_t)g.ni * g.nj * g.nk;
-    hipCheck(hipMemsetAsync(p, 0, sizeof(float) * n, s), "hipMemsetAsync");
-    if (S.m > 0) hipLaunchKernelGGL(toGridKernel, dim3(blocksFor(S.m, TPB)), dim3(TPB), 0, s, S.m, S.rows, x, p);
-}
-
 void gatherRows(const PressureSys &S, const double *cells, double *rhs, hipStream_t s) {
     if (S.m == 0) return;
     hipLaunchKernelGGL(gatherRowsKernel, dim3(blocksFor(S.m, TPB)), dim3(TPB), 0, s, S.m, S.rows, cells, rhs);
-}
-void gatherRowsF(const PressureSys &S, const float *cells, double *x, hipStream_t s) {
-    if (S.m == 0) return;
-    hipLaunchKernelGGL(gatherRowsFKernel, dim3(blocksFor(S.m, TPB)), dim3(TPB), 0, s, S.m, S.rows, cells, x);
-}
-void scatterRows(const PressureSys &S, const double *x, double *cells, hipStream_t s) {
-    if (S.m == 0) return;
-    hipLaunchKernelGGL(scatterRowsKernel, dim3(blocksFor(S.m, TPB)), dim3(TPB), 0, s, S.m, S.rows, x, cells);
 }
 void castToFloat(const double *a, float *b, size_t n, hipStream_t s) {
     if (n == 0) return;
@@ -710,13 +447,6 @@ void mic0ToFloat(PressureSys &S, hipStream_t s) {
     castToFloat(S.lx, S.flx, m, s);
     castToFloat(S.ly, S.fly, m, s);
     castToFloat(S.lz, S.flz, m, s);
-    castToFloat(S.diag, S.fdiag, m, s);
-    castToFloat(S.ox, S.fox, m, s);
-    castToFloat(S.oy, S.foy, m, s);
-    castToFloat(S.oz, S.foz, m, s);
-    castToFloat(S.mx, S.fmx, m, s);
-    castToFloat(S.my, S.fmy, m, s);
-    castToFloat(S.mz, S.fmz, m, s);
 }
 
 }  // namespace ff

@@ -57,17 +57,18 @@ public:
     // the surface tension terms of the following solves' divergence (status
     // null: none)
     void setTension(TensionView t) { _tension = t; }
-    // the solver's MIC(0) application: 2 = bands of hyperplanes, 4 = the
-    // line pipeline (two launches per application), 5 = the bands of one
-    // application replayed from a HIP graph captured once per solve
+    // the solver's MIC(0) application: 2 = columns of lines, one launch per
+    // sweep; 4 = the line pipeline on the row order (two launches per
+    // application), 5 = bands of hyperplanes on the row order, replayed from a
+    // HIP graph captured once per solve
     void setSchedule(int schedule);
     int schedule() const { return _sched; }
     const std::vector<int> &levelTable() const { return _hLevelStart; }
     // one preconditioner application z = (L L^T)^-1 r on the current factor
-    // (after solve()); FP64 or the FP32 copy.  schedule 0 = one launch per
-    // hyperplane, 1 = tile wavefront (switched off: raises an error),
-    // 2 = bands of hyperplanes, 3 = the same bands with the tile ranges
-    // checked on the device instead of passed in the launches, 4 = the line
+    // (after solve()); FP64 or the FP32 copy; r and z in row order.
+    // schedule 0 = one launch per hyperplane, 1 = tile wavefront (switched
+    // off: raises an error), 2 = columns (the solver's), 3 = bands of
+    // hyperplanes with the tile ranges checked on the device, 4 = the line
     // pipeline.
     void applyPreconditioner(const double *r, double *z, int schedule, hipStream_t s);
     void applyPreconditionerF(const float *r, float *z, int schedule, hipStream_t s);
@@ -77,9 +78,16 @@ public:
 private:
     Grid _g{};
     PressureSys _S{};
-    void *_block = nullptr;  // one allocation for everything
+    void *_block = nullptr;     // one allocation for the system, its columns and the vectors
+    void *_rowBlock = nullptr;  // and one for the row-ordered schedules, made when one is used
+    ColumnPlan _cp;
+    ColumnSys _C{};
+    // the PCG's vectors, in slots
     double *_x = nullptr, *_r = nullptr, *_z = nullptr, *_s = nullptr, *_y = nullptr;
     float *_fr = nullptr, *_fz = nullptr, *_fs = nullptr, *_fd = nullptr, *_fq = nullptr, *_fy = nullptr;
+    // an application's operands in row order (row-ordered schedules and dots)
+    double *_rowR = nullptr, *_rowY = nullptr, *_rowZ = nullptr;
+    float *_rowFR = nullptr, *_rowFY = nullptr, *_rowFZ = nullptr;
     double *_partial = nullptr, *_scal = nullptr;
     double *_hostScal = nullptr, *_hostScalDev = nullptr;  // mapped pinned host slot and its device alias
     std::vector<int> _hLevelStart;
@@ -93,12 +101,17 @@ private:
     KernelTimers *_t = nullptr;
     KernelTimers _noTimers;
     int _levelLaunches = 0, _bandLaunches = 0;
-    PencilPlan _pp;  // line-pipeline buffers (inside _block)
+    PencilPlan _pp;  // line-pipeline buffers (inside _rowBlock)
     int _sched = 2;
     // z = M^-1 r with the solver's schedule (y: forward result)
     void precond(const double *r, double *y, double *z, hipStream_t s);
     void precondF(const float *r, float *y, float *z, hipStream_t s);
-    int applyLaunches() const { return _sched == 4 ? 2 : _bandLaunches; }
+    int applyLaunches() const { return _sched == 5 ? _bandLaunches : 2; }
+    size_t maxRows() const;
+    void ensureRowSchedules();
+    void prepareRowSchedule(int schedule, bool fp64, hipStream_t s);
+    void factor(bool fp64, hipStream_t st);
+    void rowDot(const double *a, const double *b, double *out, hipStream_t st);
     // schedule 5: executable graphs of the band launches for the (r, z)
     // pairs of the current solve's applications (the PCG's z alternates
     // between two buffers), dropped when a new system is assembled

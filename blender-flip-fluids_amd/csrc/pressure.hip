@@ -13,8 +13,21 @@ void hipCheck(hipError_t e, const char *what);
 PressureSolver::~PressureSolver() {
     dropGraphs();
     if (_block) (void)hipFree(_block);
+    if (_rowBlock) (void)hipFree(_rowBlock);
     if (_hostScal) (void)hipHostFree(_hostScal);
 }
+
+namespace {
+// consecutive 256-byte aligned parts of one allocation
+struct Carver {
+    size_t bytes = 0;
+    size_t take(size_t n) {
+        const size_t off = bytes;
+        bytes += (n + 255) / 256 * 256;
+        return off;
+    }
+};
+}  // namespace
 
 void PressureSolver::allocate(Grid g) {
     _g = g;
@@ -23,126 +36,175 @@ void PressureSolver::allocate(Grid g) {
         hipCheck(hipHostGetDevicePointer((void **)&_hostScalDev, _hostScal, 0), "hipHostGetDevicePointer");
     }
     if (_block) (void)hipFree(_block);
+    if (_rowBlock) (void)hipFree(_rowBlock);
+    _block = _rowBlock = nullptr;
     const size_t N = (size_t)g.ni * g.nj * g.nk;
-    // pressure rows live on interior cells only
-    const size_t M = (size_t)std::max(g.ni - 2, 1) * std::max(g.nj - 2, 1) * std::max(g.nk - 2, 1);
-    const size_t L = (size_t)g.ni + g.nj + g.nk;
-    size_t bytes = 0;
-    auto take = [&](size_t nbytes) {
-        size_t off = bytes;
-        bytes += (nbytes + 255) / 256 * 256;
-        return off;
-    };
-    size_t oMask = take(4 * (N + 1)), oRowOf = take(4 * (N + 1)), oRows = take(4 * M), oNbr = take(24 * M);
-    size_t oCellRow = take(4 * N);
-    {
-        int ti, tj, tk;
-        micTileCounts(g, std::min(micTileDepth(true), micTileDepth(false)), ti, tj, tk);
-        _maxTiles = ti * tj * tk;
-    }
-    size_t oOrder = take(4 * (size_t)_maxTiles), oTileRows = take(4 * (size_t)_maxTiles);
-    size_t oFlags = take(4 * (size_t)_maxTiles), oCounter = take(4), oError = take(4);
+    const size_t M = maxRows(), L = (size_t)g.ni + g.nj + g.nk;
+    Carver b;
+    size_t oMask = b.take(4 * (N + 1)), oRowOf = b.take(4 * (N + 1)), oRows = b.take(4 * M), oNbr = b.take(24 * M);
+    size_t oCellRow = b.take(4 * N), oError = b.take(4);
     _bandTilesMax = std::max(mic0BandTiles(g, true), mic0BandTiles(g, false));
-    size_t oTileLo = take(4 * (size_t)_bandTilesMax), oTileHi = take(4 * (size_t)_bandTilesMax);
-    size_t oLc = take(4 * (L + 1)), oLs = take(4 * (L + 1)), oLf = take(4 * L), oLr = take(4 * M);
-    size_t oD[15], oF[14];
-    for (auto &o : oD) o = take(8 * M);
-    for (auto &o : oF) o = take(4 * M);
-    size_t oV[5], oFV[6];
-    for (auto &o : oV) o = take(8 * M);
-    for (auto &o : oFV) o = take(4 * M);
-    size_t oRec64[2], oRec32[2];
-    for (auto &o : oRec64) o = take(sizeof(MicRec<double>) * M);
-    for (auto &o : oRec32) o = take(sizeof(MicRec<float>) * M);
-    pencilShape(g, _pp.npj, _pp.npk, _pp.nw);
-    _pp.np = _pp.npj * _pp.npk;
-    size_t oPOrder = take(4 * (size_t)_pp.np), oPWords = take(sizeof(LineWord) * (size_t)g.nj * g.nk * _pp.nw);
-    const size_t exWords = pencilExchangeWords(g);
-    size_t oPEx = take(8 * exWords), oPCounter = take(4);
-    size_t oPart = take(8 * 1024), oScal = take(8 * 16);
-    hipCheck(hipMalloc(&_block, bytes), "hipMalloc pressure");
-    char *b = (char *)_block;
-    _S.mask = (int *)(b + oMask);
-    _S.rowOf = (int *)(b + oRowOf);
-    _S.rows = (int *)(b + oRows);
-    _S.nbr = (int *)(b + oNbr);
-    _S.levelCount = (int *)(b + oLc);
-    _S.levelStart = (int *)(b + oLs);
-    _S.levelFill = (int *)(b + oLf);
-    _S.levelRows = (int *)(b + oLr);
-    _S.cellRow = (int *)(b + oCellRow);
-    _ms.order = (int *)(b + oOrder);
-    _ms.tileRows = (int *)(b + oTileRows);
-    _ms.flags = (int *)(b + oFlags);
-    _ms.counter = (int *)(b + oCounter);
-    _ms.error = (int *)(b + oError);
-    _tileLo = (int *)(b + oTileLo);
-    _tileHi = (int *)(b + oTileHi);
+    size_t oTileLo = b.take(4 * (size_t)_bandTilesMax), oTileHi = b.take(4 * (size_t)_bandTilesMax);
+    size_t oLc = b.take(4 * (L + 1)), oLs = b.take(4 * (L + 1));
+    size_t oD[9];
+    for (auto &o : oD) o = b.take(8 * M);
+    columnShape(g, _cp);
+    const size_t E = _cp.maxSlices * COL_SLICE;
+    size_t oCols = b.take(sizeof(ColumnRange) * (size_t)_cp.ncj * _cp.nck);
+    size_t oOrder = b.take(4 * (size_t)_cp.ntj * _cp.ntk);
+    size_t oLinks = b.take(sizeof(SliceLinks) * _cp.maxSlices), oSlotRow = b.take(4 * E), oTotal = b.take(4);
+    size_t oExJ = b.take(4 * _cp.exJWords), oExK = b.take(4 * _cp.exKWords), oCounter = b.take(4);
+    size_t oC[5], oCF[4], oV[5], oFV[6];
+    for (auto &o : oC) o = b.take(8 * E);
+    for (auto &o : oCF) o = b.take(4 * E);
+    for (auto &o : oV) o = b.take(8 * E);
+    for (auto &o : oFV) o = b.take(4 * E);
+    // one solve's sweeps are of one precision: the FP32 records share the FP64 ones' place
+    size_t oRec[2];
+    for (auto &o : oRec) o = b.take(sizeof(MicRec<double>) * E);
+    size_t oPart = b.take(8 * 1024), oScal = b.take(8 * 16);
+    hipCheck(hipMalloc(&_block, b.bytes), "hipMalloc pressure");
+    char *m = (char *)_block;
+    _S.mask = (int *)(m + oMask);
+    _S.rowOf = (int *)(m + oRowOf);
+    _S.rows = (int *)(m + oRows);
+    _S.nbr = (int *)(m + oNbr);
+    _S.levelCount = (int *)(m + oLc);
+    _S.levelStart = (int *)(m + oLs);
+    _S.cellRow = (int *)(m + oCellRow);
+    _tileLo = (int *)(m + oTileLo);
+    _tileHi = (int *)(m + oTileHi);
     _hTileLo.assign(_bandTilesMax, 0);
     _hTileHi.assign(_bandTilesMax, 0);
-    double *d[15];
-    for (int q = 0; q < 15; q++) d[q] = (double *)(b + oD[q]);
+    double *d[9];
+    for (int q = 0; q < 9; q++) d[q] = (double *)(m + oD[q]);
     _S.rhs = d[0]; _S.diag = d[1]; _S.ox = d[2]; _S.oy = d[3]; _S.oz = d[4];
-    _S.mx = d[5]; _S.my = d[6]; _S.mz = d[7]; _S.invdiag = d[8];
-    _S.lx = d[9]; _S.ly = d[10]; _S.lz = d[11];
-    _S.lmx = d[12]; _S.lmy = d[13]; _S.lmz = d[14];
-    float *f[14];
-    for (int q = 0; q < 14; q++) f[q] = (float *)(b + oF[q]);
-    _S.finvdiag = f[0]; _S.flx = f[1]; _S.fly = f[2]; _S.flz = f[3];
-    _S.fdiag = f[4]; _S.fox = f[5]; _S.foy = f[6]; _S.foz = f[7];
-    _S.fmx = f[8]; _S.fmy = f[9]; _S.fmz = f[10];
-    _S.flmx = f[11]; _S.flmy = f[12]; _S.flmz = f[13];
-    _S.recFwd = (MicRec<double> *)(b + oRec64[0]);
-    _S.recBwd = (MicRec<double> *)(b + oRec64[1]);
-    _S.frecFwd = (MicRec<float> *)(b + oRec32[0]);
-    _S.frecBwd = (MicRec<float> *)(b + oRec32[1]);
-    _x = (double *)(b + oV[0]); _r = (double *)(b + oV[1]); _z = (double *)(b + oV[2]); _s = (double *)(b + oV[3]);
-    _y = (double *)(b + oV[4]);
-    _fr = (float *)(b + oFV[0]); _fz = (float *)(b + oFV[1]); _fs = (float *)(b + oFV[2]);
-    _fd = (float *)(b + oFV[3]); _fq = (float *)(b + oFV[4]); _fy = (float *)(b + oFV[5]);
-    _pp.order = (int *)(b + oPOrder);
-    _pp.words = (LineWord *)(b + oPWords);
-    _S.words = _pp.words;
-    _S.nw = _pp.nw;
+    _S.invdiag = d[5]; _S.lx = d[6]; _S.ly = d[7]; _S.lz = d[8];
+    _cp.cols = (ColumnRange *)(m + oCols);
+    _cp.order = (int *)(m + oOrder);
+    _cp.links = (SliceLinks *)(m + oLinks);
+    _cp.slotRow = (int *)(m + oSlotRow);
+    _cp.total = (int *)(m + oTotal);
+    _cp.exJ = (unsigned *)(m + oExJ);
+    _cp.exK = (unsigned *)(m + oExK);
+    _cp.counter = (unsigned *)(m + oCounter);
+    _cp.error = (int *)(m + oError);
+    _cp.base = _cp.epoch = 0;
+    _cp.slices = 0;
+    _C.rhs = (double *)(m + oC[0]); _C.diag = (double *)(m + oC[1]);
+    _C.ox = (double *)(m + oC[2]); _C.oy = (double *)(m + oC[3]); _C.oz = (double *)(m + oC[4]);
+    _C.fdiag = (float *)(m + oCF[0]); _C.fox = (float *)(m + oCF[1]);
+    _C.foy = (float *)(m + oCF[2]); _C.foz = (float *)(m + oCF[3]);
+    _C.recFwd = (MicRec<double> *)(m + oRec[0]); _C.recBwd = (MicRec<double> *)(m + oRec[1]);
+    _C.frecFwd = (MicRec<float> *)(m + oRec[0]); _C.frecBwd = (MicRec<float> *)(m + oRec[1]);
+    _x = (double *)(m + oV[0]); _r = (double *)(m + oV[1]); _z = (double *)(m + oV[2]); _s = (double *)(m + oV[3]);
+    _y = (double *)(m + oV[4]);
+    _fr = (float *)(m + oFV[0]); _fz = (float *)(m + oFV[1]); _fs = (float *)(m + oFV[2]);
+    _fd = (float *)(m + oFV[3]); _fq = (float *)(m + oFV[4]); _fy = (float *)(m + oFV[5]);
     _S.ni = g.ni;
     _S.nj = g.nj;
     _S.nk = g.nk;
-    _pp.ex = (unsigned long long *)(b + oPEx);
-    _pp.counter = (unsigned *)(b + oPCounter);
-    _pp.error = _ms.error;
-    _pp.base = 0;
-    _pp.epoch = 0;
     {
+        // epoch 0 marks a word no launch has published; the counter starts at
+        // 0.  The copy comes last: it waits for the fills, which the solver's
+        // own stream would not.
+        hipCheck(hipMemset(_cp.exJ, 0, 4 * _cp.exJWords), "clear exchange words");
+        hipCheck(hipMemset(_cp.exK, 0, 4 * _cp.exKWords), "clear exchange words");
+        hipCheck(hipMemset(_cp.counter, 0, 4), "clear ticket counter");
         std::vector<int> order;
-        pencilOrder(g, order);
-        hipCheck(hipMemcpy(_pp.order, order.data(), sizeof(int) * order.size(), hipMemcpyHostToDevice),
-                 "H2D pencil order");
-        // epoch 0 marks a word no launch has published; the counter starts at 0
-        hipCheck(hipMemset(_pp.ex, 0, 8 * exWords), "clear exchange words");
-        hipCheck(hipMemset(_pp.counter, 0, 4), "clear ticket counter");
+        columnOrder(_cp, order);
+        hipCheck(hipMemcpy(_cp.order, order.data(), sizeof(int) * order.size(), hipMemcpyHostToDevice),
+                 "H2D tile order");
     }
-    _partial = (double *)(b + oPart);
-    _scal = (double *)(b + oScal);
+    _partial = (double *)(m + oPart);
+    _scal = (double *)(m + oScal);
     _S.m = 0;
     _S.nLevels = g.ni + g.nj + g.nk - 2;
-    int dev = 0, cus = 0;
+    int dev = 0, wallKHz = 0;
+    hipCheck(hipGetDevice(&dev), "hipGetDevice");
+    hipCheck(hipDeviceGetAttribute(&wallKHz, hipDeviceAttributeWallClockRate, dev), "device attribute");
+    _cp.waitTicks = 2000LL * std::max(wallKHz, 1);  // 2 s
+}
+
+size_t PressureSolver::maxRows() const {
+    // pressure rows live on interior cells only
+    return (size_t)std::max(_g.ni - 2, 1) * std::max(_g.nj - 2, 1) * std::max(_g.nk - 2, 1);
+}
+
+// The buffers of the row-ordered schedules, made when one of them is first
+// used.
+void PressureSolver::ensureRowSchedules() {
+    if (_rowBlock) return;
+    const Grid g = _g;
+    const size_t M = maxRows(), L = (size_t)g.ni + g.nj + g.nk;
+    int ti, tj, tk;
+    micTileCounts(g, std::min(micTileDepth(true), micTileDepth(false)), ti, tj, tk);
+    _maxTiles = ti * tj * tk;
+    Carver b;
+    size_t oOrder = b.take(4 * (size_t)_maxTiles), oTileRows = b.take(4 * (size_t)_maxTiles);
+    size_t oFlags = b.take(4 * (size_t)_maxTiles), oCounter = b.take(4);
+    size_t oLf = b.take(4 * L), oLr = b.take(4 * M);
+    size_t oD[6], oF[10];
+    for (auto &o : oD) o = b.take(8 * M);
+    for (auto &o : oF) o = b.take(4 * M);
+    size_t oRec64[2], oRec32[2];
+    for (auto &o : oRec64) o = b.take(sizeof(MicRec<double>) * M);
+    for (auto &o : oRec32) o = b.take(sizeof(MicRec<float>) * M);
+    pencilShape(g, _pp.npj, _pp.npk, _pp.nw);
+    _pp.np = _pp.npj * _pp.npk;
+    size_t oPOrder = b.take(4 * (size_t)_pp.np), oPWords = b.take(sizeof(LineWord) * (size_t)g.nj * g.nk * _pp.nw);
+    const size_t exWords = pencilExchangeWords(g);
+    size_t oPEx = b.take(8 * exWords), oPCounter = b.take(4);
+    int dev = 0, cus = 0, lds = 0;
     hipCheck(hipGetDevice(&dev), "hipGetDevice");
     hipCheck(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev), "device attribute");
-    _ms.grid = std::max(cus, 1);
-    int wallKHz = 0;
-    hipCheck(hipDeviceGetAttribute(&wallKHz, hipDeviceAttributeWallClockRate, dev), "device attribute");
-    _ms.waitTicks = 2000LL * std::max(wallKHz, 1);  // 2 s
-    _pp.waitTicks = _ms.waitTicks;
-    int lds = 0;
     hipCheck(hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev), "device attribute");
-    if ((size_t)lds < pencilLdsBytes(g) + 8448)
-        throw std::runtime_error("the MIC(0) line pipeline needs " + std::to_string(pencilLdsBytes(g) + 8448) +
+    const size_t pencilLds = pencilLdsBytes(g) + 8448;
+    if ((size_t)lds < pencilLds)
+        throw std::runtime_error("the MIC(0) line pipeline needs " + std::to_string(pencilLds) +
                                  " bytes of LDS per workgroup at this grid size; the device offers " +
                                  std::to_string(lds));
     if ((size_t)lds < micTileLds(true))
         throw std::runtime_error("the MIC(0) tile kernel needs " + std::to_string(micTileLds(true)) +
                                  " bytes of LDS per workgroup; the device offers " + std::to_string(lds));
+    hipCheck(hipMalloc(&_rowBlock, b.bytes), "hipMalloc pressure (row schedules)");
+    char *m = (char *)_rowBlock;
     _ms.g = g;
+    _ms.order = (int *)(m + oOrder);
+    _ms.tileRows = (int *)(m + oTileRows);
+    _ms.flags = (int *)(m + oFlags);
+    _ms.counter = (int *)(m + oCounter);
+    _ms.error = _cp.error;
+    _ms.grid = std::max(cus, 1);
+    _ms.waitTicks = _cp.waitTicks;
+    _S.levelFill = (int *)(m + oLf);
+    _S.levelRows = (int *)(m + oLr);
+    double *d[6];
+    for (int q = 0; q < 6; q++) d[q] = (double *)(m + oD[q]);
+    _S.lmx = d[0]; _S.lmy = d[1]; _S.lmz = d[2];
+    _rowR = d[3]; _rowY = d[4]; _rowZ = d[5];
+    float *f[10];
+    for (int q = 0; q < 10; q++) f[q] = (float *)(m + oF[q]);
+    _S.finvdiag = f[0]; _S.flx = f[1]; _S.fly = f[2]; _S.flz = f[3];
+    _S.flmx = f[4]; _S.flmy = f[5]; _S.flmz = f[6];
+    _rowFR = f[7]; _rowFY = f[8]; _rowFZ = f[9];
+    _S.recFwd = (MicRec<double> *)(m + oRec64[0]);
+    _S.recBwd = (MicRec<double> *)(m + oRec64[1]);
+    _S.frecFwd = (MicRec<float> *)(m + oRec32[0]);
+    _S.frecBwd = (MicRec<float> *)(m + oRec32[1]);
+    _pp.order = (int *)(m + oPOrder);
+    _pp.words = (LineWord *)(m + oPWords);
+    _pp.ex = (unsigned long long *)(m + oPEx);
+    _pp.counter = (unsigned *)(m + oPCounter);
+    _pp.error = _cp.error;
+    _pp.waitTicks = _cp.waitTicks;
+    _pp.base = _pp.epoch = 0;
+    hipCheck(hipMemset(_pp.ex, 0, 8 * exWords), "clear exchange words");
+    hipCheck(hipMemset(_pp.counter, 0, 4), "clear ticket counter");
+    std::vector<int> order;
+    pencilOrder(g, order);
+    hipCheck(hipMemcpy(_pp.order, order.data(), sizeof(int) * order.size(), hipMemcpyHostToDevice),
+             "H2D pencil order");
 }
 
 // Non-empty tiles of the preconditioner's tile wavefront, listed by tile
@@ -186,7 +248,7 @@ void PressureSolver::enqueueTileRanges(bool fp64, hipStream_t s) {
 
 void PressureSolver::checkError(hipStream_t s) {
     int e = 0;
-    hipCheck(hipMemcpyAsync(&e, _ms.error, sizeof(int), hipMemcpyDeviceToHost, s), "D2H error word");
+    hipCheck(hipMemcpyAsync(&e, _cp.error, sizeof(int), hipMemcpyDeviceToHost, s), "D2H error word");
     hipCheck(hipStreamSynchronize(s), "sync");
     if (e) throw std::runtime_error("MIC(0) preconditioner: a wait for a neighbour's results exceeded its time limit");
 }
@@ -194,7 +256,7 @@ void PressureSolver::checkError(hipStream_t s) {
 void PressureSolver::setSchedule(int schedule) {
     if (schedule != 2 && schedule != 4 && schedule != 5)
         throw std::domain_error(
-            "the solver's preconditioner schedule must be 2 (bands), 4 (line pipeline) or 5 (bands from a graph)");
+            "the solver's preconditioner schedule must be 2 (columns), 4 (line pipeline) or 5 (bands from a graph)");
     _sched = schedule;
 }
 
@@ -243,62 +305,91 @@ void PressureSolver::graphApply(const T *r, T *y, T *z, hipStream_t s) {
     hipCheck(hipGraphLaunch(slot->exec, s), "launch the band graph");
 }
 
+// the row-ordered schedules' operands of the current factor
+void PressureSolver::prepareRowSchedule(int schedule, bool fp64, hipStream_t s) {
+    ensureRowSchedules();
+    if (!fp64) mic0ToFloat(_S, s);
+    mic0LowerEntries(_S, fp64, s);
+    if (schedule == 4) {
+        pencilLineWords(_g, _S, _pp, s);
+    } else if (schedule == 0) {
+        pressureLevelRows(_g, _S, s);
+    } else if (schedule != 1) {
+        const bool host = schedule != 3;
+        mic0BandPlan(_g, _S, _hLevelStart.data(), fp64, host ? _hTileLo.data() : nullptr,
+                     host ? _hTileHi.data() : nullptr, _plan);
+        _bandLaunches = (int)_plan.l0.size();
+    }
+    dropGraphs();  // recorded with the previous system's plan
+}
+
 void PressureSolver::precond(const double *r, double *y, double *z, hipStream_t s) {
+    if (_sched == 2) {
+        columnApply(_cp, _C, r, y, z, s);
+        return;
+    }
+    rowsFromSlots(_cp, r, _rowR, s);
     if (_sched == 4)
-        pencilApply(_g, _S, _pp, r, y, z, s);
-    else if (_sched == 5)
-        graphApply(r, y, z, s);
+        pencilApply(_g, _S, _pp, _rowR, _rowY, _rowZ, s);
     else
-        mic0ApplyBands(_g, _S, _plan, _tileLo, _tileHi, r, y, z, s);
+        graphApply(_rowR, _rowY, _rowZ, s);
+    slotsFromRows(_cp, _rowZ, z, s);
 }
 void PressureSolver::precondF(const float *r, float *y, float *z, hipStream_t s) {
+    if (_sched == 2) {
+        columnApplyF(_cp, _C, r, y, z, s);
+        return;
+    }
+    rowsFromSlots(_cp, r, _rowFR, s);
     if (_sched == 4)
-        pencilApplyF(_g, _S, _pp, r, y, z, s);
-    else if (_sched == 5)
-        graphApply(r, y, z, s);
+        pencilApplyF(_g, _S, _pp, _rowFR, _rowFY, _rowFZ, s);
     else
-        mic0ApplyBandsF(_g, _S, _plan, _tileLo, _tileHi, r, y, z, s);
+        graphApply(_rowFR, _rowFY, _rowFZ, s);
+    slotsFromRows(_cp, _rowFZ, z, s);
 }
 
 void PressureSolver::applyPreconditioner(const double *r, double *z, int schedule, hipStream_t s) {
+    if (schedule == 2) {
+        columnRecords(_S, _cp, _C, true, s);
+        slotsFromRows(_cp, r, _r, s);
+        columnApply(_cp, _C, _r, _y, _z, s);
+        rowsFromSlots(_cp, _z, z, s);
+        return;
+    }
+    prepareRowSchedule(schedule, true, s);
     if (schedule == 4) {
-        pencilLineWords(_g, _S, _pp, s);
-        pencilApply(_g, _S, _pp, r, _y, z, s);
+        pencilApply(_g, _S, _pp, r, _rowY, z, s);
     } else if (schedule == 1) {
         buildSchedule(true, s);
         micApplyTiles(_S, _ms, r, z, s);
-    } else if (schedule == 2 || schedule == 3) {
-        enqueueTileRanges(true, s);
-        hipCheck(hipStreamSynchronize(s), "sync");
-        const bool host = schedule == 2;
-        mic0BandPlan(_g, _S, _hLevelStart.data(), true, host ? _hTileLo.data() : nullptr,
-                     host ? _hTileHi.data() : nullptr, _plan);
-        mic0ApplyBands(_g, _S, _plan, _tileLo, _tileHi, r, _y, z, s);
+    } else if (schedule == 3) {
+        mic0ApplyBands(_g, _S, _plan, _tileLo, _tileHi, r, _rowY, z, s);
     } else {
         mic0Apply(_S, _hLevelStart.data(), r, z, s);
     }
 }
 void PressureSolver::applyPreconditionerF(const float *r, float *z, int schedule, hipStream_t s) {
+    if (schedule == 2) {
+        columnRecords(_S, _cp, _C, false, s);
+        slotsFromRows(_cp, r, _fr, s);
+        columnApplyF(_cp, _C, _fr, _fy, _fz, s);
+        rowsFromSlots(_cp, _fz, z, s);
+        return;
+    }
+    prepareRowSchedule(schedule, false, s);
     if (schedule == 4) {
-        pencilLineWords(_g, _S, _pp, s);
-        pencilApplyF(_g, _S, _pp, r, _fy, z, s);
+        pencilApplyF(_g, _S, _pp, r, _rowFY, z, s);
     } else if (schedule == 1) {
         buildSchedule(false, s);
         micApplyTilesF(_S, _ms, r, z, s);
-    } else if (schedule == 2 || schedule == 3) {
-        enqueueTileRanges(false, s);
-        hipCheck(hipStreamSynchronize(s), "sync");
-        const bool host = schedule == 2;
-        mic0BandPlan(_g, _S, _hLevelStart.data(), false, host ? _hTileLo.data() : nullptr,
-                     host ? _hTileHi.data() : nullptr, _plan);
-        mic0ApplyBandsF(_g, _S, _plan, _tileLo, _tileHi, r, _fy, z, s);
+    } else if (schedule == 3) {
+        mic0ApplyBandsF(_g, _S, _plan, _tileLo, _tileHi, r, _rowFY, z, s);
     } else {
         mic0ApplyF(_S, _hLevelStart.data(), r, z, s);
     }
 }
 
-// Reads one device scalar.  (The solver's band schedule never raises the tile
-// wavefront's error word; applyPreconditioner checks it for that schedule.)
+// Reads one device scalar.
 double PressureSolver::hostScalar(const double *d, hipStream_t s) {
     double h = 0.0;
     hipCheck(hipMemcpyAsync(&h, d, sizeof(double), hipMemcpyDeviceToHost, s), "D2H scalar");
@@ -325,13 +416,15 @@ PressureResult PressureSolver::solve(double dt, const float *u, const float *v, 
     if (cellSolution)
         hipCheck(hipMemsetAsync(cellSolution, 0, sizeof(double) * (size_t)_g.ni * _g.nj * _g.nk, s), "memset");
     _t = timers ? timers : &_noTimers;
-    hipCheck(hipMemsetAsync(_ms.error, 0, sizeof(int), s), "memset error word");
+    hipCheck(hipMemsetAsync(_cp.error, 0, sizeof(int), s), "memset error word");
     _t->begin(T_ASSEMBLE, s);
     const size_t N = (size_t)_g.ni * _g.nj * _g.nk;
     pressureMask(_g, phi, _S.mask, s);
     exclusiveScan(_S.mask, _S.rowOf, N, scanScratch, s);
+    columnRanges(_g, _S.mask, _cp, s);
     int m = 0;
     hipCheck(hipMemcpyAsync(&m, _S.rowOf + N, sizeof(int), hipMemcpyDeviceToHost, s), "D2H");
+    hipCheck(hipMemcpyAsync(&_cp.slices, _cp.total, sizeof(int), hipMemcpyDeviceToHost, s), "D2H");
     hipCheck(hipStreamSynchronize(s), "sync");
     _S.m = m;
     res.unknowns = m;
@@ -339,7 +432,7 @@ PressureResult PressureSolver::solve(double dt, const float *u, const float *v, 
     pressureAssemble(_g, dt, u, v, w, wu, wv, ww, phi, _S, s, _solid, _tension);
     if (cellRhs) gatherRows(_S, cellRhs, _S.rhs, s);
     pressureLevels(_g, _S, scanScratch, s);
-    if (m > 0) pencilLineWords(_g, _S, _pp, s);  // SpMV and the line pipeline find neighbour rows in them
+    columnFill(_g, _S, _cp, _C, mode == 1 || mode == 2, s);
     _t->end(T_ASSEMBLE, s);
     _hLevelStart.resize(_S.nLevels + 1);
     hipCheck(hipMemcpyAsync(_hLevelStart.data(), _S.levelStart, sizeof(int) * (_S.nLevels + 1),
@@ -347,7 +440,7 @@ PressureResult PressureSolver::solve(double dt, const float *u, const float *v, 
     enqueueTileRanges(mode == 0, s);
     double maxAbs = 0.0;
     if (m > 0) {
-        absMax(_S.rhs, m, _partial, _scal + 1, s);
+        absMax(_C.rhs, _cp.slots(), _partial, _scal + 1, s);
         maxAbs = hostScalar(_scal + 1, s);  // also waits for the level table and the tile ranges
     } else {
         hipCheck(hipStreamSynchronize(s), "sync");
@@ -355,9 +448,6 @@ PressureResult PressureSolver::solve(double dt, const float *u, const float *v, 
     res.rhsInf = maxAbs;
     if (afterAssembly) hipCheck(hipEventRecord(afterAssembly, s), "event");
     _levelLaunches = mic0FactorBandLaunches(_S, _hLevelStart.data());
-    mic0BandPlan(_g, _S, _hLevelStart.data(), mode == 0, _hTileLo.data(), _hTileHi.data(), _plan);
-    _bandLaunches = (int)_plan.l0.size();
-    dropGraphs();  // recorded with the previous system's plan
     // The forward solve skips a right-hand side below the tolerance as an
     // absolute threshold, as the reference does (pressuresolver.cpp:69-75).  A
     // given right-hand side (the adjoint's) is solved unless it is exactly 0,
@@ -377,8 +467,9 @@ PressureResult PressureSolver::solve(double dt, const float *u, const float *v, 
                 : mode == 2 ? pcgReliable(tol, maxIter, maxAbs, innerTol, iters, resid, s)
                             : pcgPrecond32(tol, maxIter, maxAbs, iters, resid, s);
     checkError(s);
-    pressureToGrid(_g, _S, _x, pressure, s);
-    if (cellSolution) scatterRows(_S, _x, cellSolution, s);
+    hipCheck(hipMemsetAsync(pressure, 0, sizeof(float) * N, s), "memset");
+    cellsFromSlots(_S, _cp, _x, pressure, s);
+    if (cellSolution) cellsFromSlots(_S, _cp, _x, cellSolution, s);
     float e = (float)resid;
     res.success = conv || (iters == maxIter && e < 1.0);
     res.iterations = iters;
@@ -389,29 +480,44 @@ PressureResult PressureSolver::solve(double dt, const float *u, const float *v, 
 // PCGSolver<double>::solve (pcgsolver.h:268-322): x0 = 0, MIC(0), float step
 // lengths, |r|_inf stop test against min(tol * |b|_inf, 1.0)
 void PressureSolver::initialGuess(hipStream_t st) {
-    const int m = _S.m;
+    const size_t n = _cp.slots();
     if (_warm && _prevPressure) {
-        gatherRowsF(_S, _prevPressure, _x, st);
-        residual(_S, _S.rhs, _x, _r, st);
+        slotsFromCells(_S, _cp, _prevPressure, _x, st);
+        columnResidual(_cp, _C, _C.rhs, _x, _r, st);
     } else {
-        hipCheck(hipMemcpyAsync(_r, _S.rhs, sizeof(double) * m, hipMemcpyDeviceToDevice, st), "copy");
-        hipCheck(hipMemsetAsync(_x, 0, sizeof(double) * m, st), "memset");
+        hipCheck(hipMemcpyAsync(_r, _C.rhs, sizeof(double) * n, hipMemcpyDeviceToDevice, st), "copy");
+        hipCheck(hipMemsetAsync(_x, 0, sizeof(double) * n, st), "memset");
     }
+}
+
+// MIC(0) factor and the operands of the solver's sweeps in fp64 or FP32
+void PressureSolver::factor(bool fp64, hipStream_t st) {
+    _t->begin(T_MIC0_FACTOR, st, _levelLaunches + 2);
+    mic0FactorBands(_g, _S, _hLevelStart.data(), _hTileLo.data(), _hTileHi.data(), _tileLo, _tileHi, st);
+    mic0LFactor(_S, st);
+    if (_sched == 2)
+        columnRecords(_S, _cp, _C, fp64, st);
+    else
+        prepareRowSchedule(_sched, fp64, st);
+    _t->end(T_MIC0_FACTOR, st);
+}
+
+// a . b in the reference's summation order: over the rows
+void PressureSolver::rowDot(const double *a, const double *b, double *out, hipStream_t st) {
+    ensureRowSchedules();
+    rowsFromSlots(_cp, a, _rowR, st);
+    rowsFromSlots(_cp, b, _rowY, st);
+    dotReference(_rowR, _rowY, _S.m, _refDots, _partial, out, st);
 }
 
 bool PressureSolver::pcgFP64(double tolFactor, int maxIter, double resid0, int &iters, double &resid,
                              hipStream_t st) {
-    const int m = _S.m;
-    const int *hs = _hLevelStart.data();
+    const size_t n = _cp.slots();
     if (tolFactor < 1e-30) tolFactor = 1e-30;
     initialGuess(st);
     resid = resid0;
     double tol = tolFactor * resid;
-    _t->begin(T_MIC0_FACTOR, st, _levelLaunches + 2);
-    mic0FactorBands(_g, _S, hs, _hTileLo.data(), _hTileHi.data(), _tileLo, _tileHi, st);
-    mic0LFactor(_S, st);
-    mic0LowerEntries(_S, true, st);
-    _t->end(T_MIC0_FACTOR, st);
+    factor(true, st);
     _t->begin(T_MIC0_APPLY, st, applyLaunches());
     precond(_r, _y, _z, st);
     _t->end(T_MIC0_APPLY, st);
@@ -419,9 +525,9 @@ bool PressureSolver::pcgFP64(double tolFactor, int maxIter, double resid0, int &
     // dot products: the reference's order, or the deterministic tree
     auto dotp = [&](const double *a, const double *b, double *out) {
         if (_refDots > 0)
-            dotReference(a, b, m, _refDots, _partial, out, st);
+            rowDot(a, b, out, st);
         else
-            dot(a, b, m, _partial, out, st);
+            dot(a, b, n, _partial, out, st);
     };
     dotp(_z, _r, rho);
     double hrho = hostScalar(rho, st);
@@ -429,19 +535,19 @@ bool PressureSolver::pcgFP64(double tolFactor, int maxIter, double resid0, int &
         iters = 0;
         return false;
     }
-    hipCheck(hipMemcpyAsync(_s, _z, sizeof(double) * m, hipMemcpyDeviceToDevice, st), "copy");
+    hipCheck(hipMemcpyAsync(_s, _z, sizeof(double) * n, hipMemcpyDeviceToDevice, st), "copy");
     double *s = _s, *z = _z;
     int it;
     for (it = 0; it < maxIter; it++) {
         _t->begin(T_SPMV, st);
         if (_refDots > 0) {
-            spmv(_S, s, z, st);
-            dotReference(s, z, m, _refDots, _partial, sz, st);
+            columnResidual(_cp, _C, nullptr, s, z, st);
+            rowDot(s, z, sz, st);
         } else {
-            spmvDot(_S, s, z, _partial, sz, st);
+            columnSpmvDot(_cp, _C, s, z, _partial, sz, st);
         }
         _t->end(T_SPMV, st);
-        pcgStep(_x, s, _r, z, m, rho, sz, _partial, rn, st, nullptr, _hostScalDev);
+        pcgStep(_x, s, _r, z, n, rho, sz, _partial, rn, st, nullptr, _hostScalDev);
         resid = mappedResidual(st);
         if (resid <= std::min(tol, 1.0)) {
             iters = it + 1;
@@ -452,7 +558,7 @@ bool PressureSolver::pcgFP64(double tolFactor, int maxIter, double resid0, int &
         _t->end(T_MIC0_APPLY, st);
         dotp(z, _r, rhoNew);
         // beta = rhoNew / rho; z += (float)beta * s; then s <-> z
-        axpyFloatStep(z, s, m, rhoNew, rho, 1.0, st);
+        axpyFloatStep(z, s, n, rhoNew, rho, 1.0, st);
         std::swap(s, z);
         std::swap(rho, rhoNew);
     }
@@ -467,38 +573,32 @@ bool PressureSolver::pcgFP64(double tolFactor, int maxIter, double resid0, int &
 // iteration follows the FP64 solve except for the preconditioner's rounding.
 bool PressureSolver::pcgPrecond32(double tolFactor, int maxIter, double resid0, int &iters, double &resid,
                                   hipStream_t st) {
-    const int m = _S.m;
-    const int *hs = _hLevelStart.data();
+    const size_t n = _cp.slots();
     if (tolFactor < 1e-30) tolFactor = 1e-30;
     initialGuess(st);
     resid = resid0;
     double tol = tolFactor * resid;
-    _t->begin(T_MIC0_FACTOR, st, _levelLaunches + 2);
-    mic0FactorBands(_g, _S, hs, _hTileLo.data(), _hTileHi.data(), _tileLo, _tileHi, st);
-    mic0LFactor(_S, st);
-    _t->end(T_MIC0_FACTOR, st);
-    mic0ToFloat(_S, st);
-    mic0LowerEntries(_S, false, st);
-    castToFloat(_r, _fr, m, st);
+    factor(false, st);
+    castToFloat(_r, _fr, n, st);
     _t->begin(T_MIC0_APPLY, st, applyLaunches());
     precondF(_fr, _fy, _fz, st);
     _t->end(T_MIC0_APPLY, st);
     double *rho = _scal + 2, *rhoNew = _scal + 3, *sz = _scal + 4, *rn = _scal + 5;
-    dotfd(_fz, _r, m, _partial, rho, st);
+    dotfd(_fz, _r, n, _partial, rho, st);
     double hrho = hostScalar(rho, st);
     if (hrho == 0 || hrho != hrho) {
         iters = 0;
         return false;
     }
-    hipCheck(hipMemsetAsync(_s, 0, sizeof(double) * m, st), "memset");
-    addFloatToDouble(_s, _fz, m, st);
+    hipCheck(hipMemsetAsync(_s, 0, sizeof(double) * n, st), "memset");
+    addFloatToDouble(_s, _fz, n, st);
     double *s = _s, *z = _z;
     int it;
     for (it = 0; it < maxIter; it++) {
         _t->begin(T_SPMV, st);
-        spmvDot(_S, s, z, _partial, sz, st);
+        columnSpmvDot(_cp, _C, s, z, _partial, sz, st);
         _t->end(T_SPMV, st);
-        pcgStep(_x, s, _r, z, m, rho, sz, _partial, rn, st, _fr, _hostScalDev);
+        pcgStep(_x, s, _r, z, n, rho, sz, _partial, rn, st, _fr, _hostScalDev);
         resid = mappedResidual(st);
         if (resid <= std::min(tol, 1.0)) {
             iters = it + 1;
@@ -507,9 +607,9 @@ bool PressureSolver::pcgPrecond32(double tolFactor, int maxIter, double resid0, 
         _t->begin(T_MIC0_APPLY, st, applyLaunches());
         precondF(_fr, _fy, _fz, st);
         _t->end(T_MIC0_APPLY, st);
-        dotfd(_fz, _r, m, _partial, rhoNew, st);
+        dotfd(_fz, _r, n, _partial, rhoNew, st);
         // beta = rhoNew / rho; z = (double)fz + (float)beta * s; then s <-> z
-        widenAxpyStep(z, _fz, s, m, rhoNew, rho, st);
+        widenAxpyStep(z, _fz, s, n, rhoNew, rho, st);
         std::swap(s, z);
         std::swap(rho, rhoNew);
     }
@@ -524,54 +624,48 @@ bool PressureSolver::pcgPrecond32(double tolFactor, int maxIter, double resid0, 
 // reference's |r|_inf <= min(tol * |b|_inf, 1.0), on the true residual.
 bool PressureSolver::pcgMixed(double tolFactor, int maxIter, double resid0, double innerRel, int &iters,
                               double &resid, hipStream_t st) {
-    const int m = _S.m;
-    const int *hs = _hLevelStart.data();
+    const size_t n = _cp.slots();
     if (tolFactor < 1e-30) tolFactor = 1e-30;
     double tol = std::min(tolFactor * resid0, 1.0);
-    hipCheck(hipMemcpyAsync(_r, _S.rhs, sizeof(double) * m, hipMemcpyDeviceToDevice, st), "copy");
-    hipCheck(hipMemsetAsync(_x, 0, sizeof(double) * m, st), "memset");
-    _t->begin(T_MIC0_FACTOR, st, _levelLaunches + 2);
-    mic0FactorBands(_g, _S, hs, _hTileLo.data(), _hTileHi.data(), _tileLo, _tileHi, st);
-    mic0LFactor(_S, st);
-    _t->end(T_MIC0_FACTOR, st);
-    mic0ToFloat(_S, st);
-    mic0LowerEntries(_S, false, st);
+    hipCheck(hipMemcpyAsync(_r, _C.rhs, sizeof(double) * n, hipMemcpyDeviceToDevice, st), "copy");
+    hipCheck(hipMemsetAsync(_x, 0, sizeof(double) * n, st), "memset");
+    factor(false, st);
     double *rho = _scal + 2, *rhoNew = _scal + 3, *sz = _scal + 4, *rn = _scal + 5;
     resid = resid0;
     iters = 0;
     int outer = 0;
     while (resid > tol && iters < maxIter && outer < 100) {
         outer++;
-        castToFloat(_r, _fr, m, st);
-        absMaxf(_fr, m, _partial, rn, st);
+        castToFloat(_r, _fr, n, st);
+        absMaxf(_fr, n, _partial, rn, st);
         double innerTol = innerRel * hostScalar(rn, st);
-        hipCheck(hipMemsetAsync(_fd, 0, sizeof(float) * m, st), "memset");
+        hipCheck(hipMemsetAsync(_fd, 0, sizeof(float) * n, st), "memset");
         _t->begin(T_MIC0_APPLY, st, applyLaunches());
         precondF(_fr, _fy, _fz, st);
         _t->end(T_MIC0_APPLY, st);
-        dotf(_fz, _fr, m, _partial, rho, st);
+        dotf(_fz, _fr, n, _partial, rho, st);
         double hrho = hostScalar(rho, st);
         if (hrho == 0 || hrho != hrho) return false;
-        hipCheck(hipMemcpyAsync(_fs, _fz, sizeof(float) * m, hipMemcpyDeviceToDevice, st), "copy");
+        hipCheck(hipMemcpyAsync(_fs, _fz, sizeof(float) * n, hipMemcpyDeviceToDevice, st), "copy");
         float *s = _fs, *z = _fz;
         while (iters < maxIter) {
             _t->begin(T_SPMV, st);
-            spmvDotF(_S, s, _fq, _partial, sz, st);
+            columnSpmvDotF(_cp, _C, s, _fq, _partial, sz, st);
             _t->end(T_SPMV, st);
-            pcgStepF(_fd, s, _fr, _fq, m, rho, sz, _partial, rn, st, _hostScalDev);
+            pcgStepF(_fd, s, _fr, _fq, n, rho, sz, _partial, rn, st, _hostScalDev);
             iters++;
             if (mappedResidual(st) <= innerTol) break;
             _t->begin(T_MIC0_APPLY, st, applyLaunches());
             precondF(_fr, _fy, z, st);
             _t->end(T_MIC0_APPLY, st);
-            dotf(z, _fr, m, _partial, rhoNew, st);
-            axpyFloatStepF(z, s, m, rhoNew, rho, 1.0, st);
+            dotf(z, _fr, n, _partial, rhoNew, st);
+            axpyFloatStepF(z, s, n, rhoNew, rho, 1.0, st);
             std::swap(s, z);
             std::swap(rho, rhoNew);
         }
-        addFloatToDouble(_x, _fd, m, st);
-        residual(_S, _S.rhs, _x, _r, st);
-        absMax(_r, m, _partial, rn, st);
+        addFloatToDouble(_x, _fd, n, st);
+        columnResidual(_cp, _C, _C.rhs, _x, _r, st);
+        absMax(_r, n, _partial, rn, st);
         resid = hostScalar(rn, st);
     }
     return resid <= tol;
@@ -588,59 +682,53 @@ bool PressureSolver::pcgMixed(double tolFactor, int maxIter, double resid0, doub
 // restarted.  Iterations counts every FP32 PCG step.
 bool PressureSolver::pcgReliable(double tolFactor, int maxIter, double resid0, double delta, int &iters,
                                  double &resid, hipStream_t st) {
-    const int m = _S.m;
-    const int *hs = _hLevelStart.data();
+    const size_t n = _cp.slots();
     if (tolFactor < 1e-30) tolFactor = 1e-30;
     const double tol = std::min(tolFactor * resid0, 1.0);
-    hipCheck(hipMemsetAsync(_x, 0, sizeof(double) * m, st), "memset");
-    _t->begin(T_MIC0_FACTOR, st, _levelLaunches + 2);
-    mic0FactorBands(_g, _S, hs, _hTileLo.data(), _hTileHi.data(), _tileLo, _tileHi, st);
-    mic0LFactor(_S, st);
-    _t->end(T_MIC0_FACTOR, st);
-    mic0ToFloat(_S, st);
-    mic0LowerEntries(_S, false, st);
+    hipCheck(hipMemsetAsync(_x, 0, sizeof(double) * n, st), "memset");
+    factor(false, st);
     double *rho = _scal + 2, *rhoNew = _scal + 3, *sz = _scal + 4, *rn = _scal + 5;
-    castToFloat(_S.rhs, _fr, m, st);
+    castToFloat(_C.rhs, _fr, n, st);
     double sinceUpdate = resid0;
     resid = resid0;
     iters = 0;
     _t->begin(T_MIC0_APPLY, st, applyLaunches());
     precondF(_fr, _fy, _fz, st);
     _t->end(T_MIC0_APPLY, st);
-    dotf(_fz, _fr, m, _partial, rho, st);
+    dotf(_fz, _fr, n, _partial, rho, st);
     double hrho = hostScalar(rho, st);
     if (hrho == 0 || hrho != hrho) return false;
-    hipCheck(hipMemcpyAsync(_fs, _fz, sizeof(float) * m, hipMemcpyDeviceToDevice, st), "copy");
+    hipCheck(hipMemcpyAsync(_fs, _fz, sizeof(float) * n, hipMemcpyDeviceToDevice, st), "copy");
     float *s = _fs, *z = _fz;
     bool trueKnown = true;  // resid holds the true residual of the current x
     while (iters < maxIter) {
         _t->begin(T_SPMV, st);
-        spmvDotF(_S, s, _fq, _partial, sz, st);
+        columnSpmvDotF(_cp, _C, s, _fq, _partial, sz, st);
         _t->end(T_SPMV, st);
-        pcgStepMixed(_x, s, _fr, _fq, m, rho, sz, _partial, rn, st, _hostScalDev);
+        pcgStepMixed(_x, s, _fr, _fq, n, rho, sz, _partial, rn, st, _hostScalDev);
         iters++;
         trueKnown = false;
         const double rf = mappedResidual(st);
         if (rf <= delta * sinceUpdate || rf <= tol) {
-            residual(_S, _S.rhs, _x, _r, st);
-            absMax(_r, m, _partial, rn, st);
+            columnResidual(_cp, _C, _C.rhs, _x, _r, st);
+            absMax(_r, n, _partial, rn, st);
             resid = hostScalar(rn, st);
             trueKnown = true;
             if (resid <= tol) return true;
-            castToFloat(_r, _fr, m, st);
+            castToFloat(_r, _fr, n, st);
             sinceUpdate = resid;
         }
         _t->begin(T_MIC0_APPLY, st, applyLaunches());
         precondF(_fr, _fy, z, st);
         _t->end(T_MIC0_APPLY, st);
-        dotf(z, _fr, m, _partial, rhoNew, st);
-        axpyFloatStepF(z, s, m, rhoNew, rho, 1.0, st);
+        dotf(z, _fr, n, _partial, rhoNew, st);
+        axpyFloatStepF(z, s, n, rhoNew, rho, 1.0, st);
         std::swap(s, z);
         std::swap(rho, rhoNew);
     }
     if (!trueKnown) {
-        residual(_S, _S.rhs, _x, _r, st);
-        absMax(_r, m, _partial, rn, st);
+        columnResidual(_cp, _C, _C.rhs, _x, _r, st);
+        absMax(_r, n, _partial, rn, st);
         resid = hostScalar(rn, st);
     }
     return resid <= tol;

@@ -340,9 +340,10 @@ class FluidSimulation(object):
         pb.execute_lib_func(f, [self(), 1 if enabled else 0])
 
     def set_pressure_solver_preconditioner_schedule(self, schedule):
-        """Schedule of the MIC(0) application: 2 = bands of hyperplanes,
-        4 = the line pipeline (one launch per triangular sweep), 5 = the bands
-        recorded once per solve as a HIP graph and replayed; same bits."""
+        """Schedule of the MIC(0) application: 2 = columns of lines (one launch
+        per triangular sweep, the default), 4 = the line pipeline on the row
+        order, 5 = bands of hyperplanes on the row order, recorded once per
+        solve as a HIP graph and replayed; same bits."""
         f = lib.FluidSimulation_set_pressure_solver_preconditioner_schedule
         pb.init_lib_func(f, [c_void_p, c_int, c_void_p], None)
         pb.execute_lib_func(f, [self(), int(schedule)])

@@ -224,10 +224,11 @@ void FluidSimulation_set_pressure_solver_warm_start(FluidSimulation *obj, int en
 int FluidSimulation_get_pressure_solver_warm_start(FluidSimulation *obj, int *err);
 /* Schedule of the MIC(0) preconditioner application (no counterpart in the
  * reference, whose triangular solves are serial loops, pcgsolver.h:211-241):
- * 2 = bands of i+j+k hyperplanes, one launch per band; 4 = the line
- * pipeline, one launch per triangular sweep; 5 = the bands of schedule 2
- * recorded once per solve as a HIP graph and replayed per application.  All
- * give the same bits. */
+ * 2 (default) = columns of lines, one launch per triangular sweep; 4 = the line pipeline on
+ * the row order, one launch per triangular sweep; 5 = bands of hyperplanes on
+ * the row order, recorded once per solve as a HIP graph and replayed.  All give
+ * the same bits; 4 and 5 convert between the solver's layout and the row order
+ * around each application. */
 void FluidSimulation_set_pressure_solver_preconditioner_schedule(FluidSimulation *obj, int schedule,
                                                                  int *err);
 int FluidSimulation_get_pressure_solver_preconditioner_schedule(FluidSimulation *obj, int *err);
@@ -478,10 +479,9 @@ int FFAMD_pressure_system(int isize, int jsize, int ksize, double dx, double dt,
  * 0 = FP64, 1 = the FP32 copy of the factor used by the mixed-precision solve
  * (r rounded to float, z widened).  schedule 0 = one launch per hyperplane,
  * 1 = the tile-wavefront kernel, which is switched off and fails with an
- * error, 2 = bands of hyperplanes (the solver's: the launches name the tiles
- * that hold rows of their band), 3 = the same bands with each workgroup
- * reading its tile's hyperplane range on the device (used when the tiles
- * outnumber what a launch can list), 4 = the line pipeline (pencils of
+ * error, 2 = columns of 16 x 8 lines along i, one launch per triangular sweep
+ * (the solver's), 3 = bands of hyperplanes with each workgroup reading its
+ * tile's hyperplane range on the device, 4 = the line pipeline (pencils of
  * 16 x 16 lines along i, one launch per triangular sweep).  The inputs must give a non-zero
  * divergence.  Returns M. */
 int FFAMD_mic0_apply(int isize, int jsize, int ksize, double dx, double dt, const float *u,

@@ -1,0 +1,50 @@
+"""The MIC(0) application in the column layout (csrc/kernels_column.hip, the
+solver's schedule) against the oracle's serial sweeps (FP64) and a
+hyperplane-vectorised FP32 restatement, bit for bit, where its split into
+columns of 16 x 8 lines, tiles of two of them and rounds of steps can go
+wrong: sides around the multiples of those, one line of cells, columns and
+tiles without rows between ones with rows, scattered rows."""
+import numpy as np
+import pytest
+
+import oracle_lib as O
+from ffengine import kernels as K
+from test_gpu_kernels import _mic_sweeps, same_bits, say
+
+pytestmark = pytest.mark.gpu
+
+
+def _liquid(kind, n3, rng):
+    ni, nj, nk = n3
+    k, j, i = np.meshgrid(np.arange(nk), np.arange(nj), np.arange(ni), indexing="ij")
+    if kind == "full":
+        wet = np.ones((nk, nj, ni), bool)
+    elif kind == "scattered":
+        wet = rng.random((nk, nj, ni)) < 0.3
+    elif kind == "islands":  # two blocks with empty columns and tiles between
+        wet = ((j < 5) & (k < 6)) | ((j >= nj - 6) & (k >= nk - 7) & (i > ni // 2))
+    else:  # "layer": every column spans few hyperplanes, at different heights
+        wet = (j + 2 * k) // 3 % 11 == i % 11
+    return np.where(wet, np.float32(-0.4), np.float32(0.3)).astype(np.float32) / max(n3)
+
+
+@pytest.mark.parametrize("kind", ["full", "scattered", "islands", "layer"])
+@pytest.mark.parametrize("n3", [(3, 3, 3), (5, 17, 9), (9, 16, 33), (40, 33, 8), (31, 15, 47), (130, 18, 34), (7, 70, 20)])
+def test_column_sweeps_bitexact(n3, kind):
+    rng = np.random.default_rng(sum(n3) + len(kind))
+    dx, dt = 1.0 / max(n3), 1.0 / 120.0
+    ni, nj, nk = n3
+    phi = _liquid(kind, n3, rng)
+    weights = O.face_weights(n3, O.solid_box_phi(n3, dx))
+    uvw = [rng.standard_normal(s).astype(np.float32) for s in ((nk, nj, ni + 1), (nk, nj + 1, ni), (nk + 1, nj, ni))]
+    sysm = O.pressure_system(n3, dx, dt, uvw, weights, phi)
+    m = len(sysm["rows"])
+    if m == 0:
+        pytest.skip("no rows")
+    r = rng.standard_normal(m)
+    say(f"column sweeps {n3} {kind}: {m} rows")
+    z = K.mic0_apply(n3, dx, dt, uvw, weights, phi, r, precision=0, schedule=2)
+    assert same_bits(z, O.apply_mic0(sysm, r))
+    f = K.mic0_apply(n3, dx, dt, uvw, weights, phi, r, precision=1, schedule=2)
+    # the call adds the widened FP32 result to zeros: -0 comes back as +0
+    assert same_bits(f.astype(np.float32), _mic_sweeps(sysm, n3, r, np.float32) + np.float32(0))
