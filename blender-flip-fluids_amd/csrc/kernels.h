@@ -143,9 +143,29 @@ __device__ inline double reduceFold(double v) {
     for (int q = 1; q < REDUCE_THREADS / 64; q++) acc = OP == 0 ? acc + waves[q] : fmax(acc, waves[q]);
     return acc;
 }
-// outHost (optional): device alias of mapped pinned host memory that also
-// receives the result
-void reduceFinish(const double *partial, int nb, double *out, bool isMax, hipStream_t s, double *outHost = nullptr);
+// the partials of a dot product only (reduceBlocks(n) of them), for a kernel
+// that folds them itself
+void dotPartials(const double *a, const double *b, size_t n, double *partial, hipStream_t s);
+void dotfPartials(const float *a, const float *b, size_t n, double *partial, hipStream_t s);
+void dotfdPartials(const float *a, const double *b, size_t n, double *partial, hipStream_t s);
+// The largest of nb partials, stored by one thread to mapped host memory in
+// one access that the host can see before the kernel ends (any block of up to
+// 1024 threads, whole waves).
+__device__ inline void publishMax(const double *partial, int nb, double *host) {
+    __shared__ double waves[16];
+    double v = 0.0;
+    for (int i = threadIdx.x; i < nb; i += blockDim.x) v = fmax(v, partial[i]);
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl_xor(v, off, 64));
+    if ((threadIdx.x & 63) == 0) waves[threadIdx.x >> 6] = v;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (unsigned q = 1; q < blockDim.x / 64; q++) v = fmax(v, waves[q]);
+        __hip_atomic_store((unsigned long long *)host, (unsigned long long)__double_as_longlong(v), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+void publishMaximum(const double *partial, int nb, double *host, hipStream_t s);
 
 // ---- setup (kernels_setup.hip) ----
 void solidBoxPhi(Grid g, float *phiNodes, hipStream_t s);
@@ -398,27 +418,22 @@ void mic0ApplyBands(Grid g, const PressureSys &S, const BandPlan &plan, const in
                     const double *r, double *y, double *z, hipStream_t s);
 void mic0ApplyBandsF(Grid g, const PressureSys &S, const BandPlan &plan, const int *tileLo, const int *tileHi,
                      const float *r, float *y, float *z, hipStream_t s);
-// (vectors: in any one order)
-// y += (float)(sign * num/den) * x   (device scalars; den may be null -> scalar = num)
-void axpyFloatStep(double *y, const double *x, size_t n, const double *num, const double *den,
-                   double sign, hipStream_t s);
-void axpyFloatStepF(float *y, const float *x, size_t n, const double *num, const double *den,
-                    double sign, hipStream_t s);
-// a = (float)(num/den); x += a * s; r -= a * q; *rmax = |r|_inf (the absMax order);
-// rf (optional) receives (float)r; rmaxHost (optional) a mapped host copy of *rmax
-void pcgStep(double *x, const double *s, double *r, const double *q, size_t n, const double *num,
-             const double *den, double *partial, double *rmax, hipStream_t st, float *rf = nullptr,
-             double *rmaxHost = nullptr);
-void pcgStepF(float *x, const float *s, float *r, const float *q, size_t n, const double *num,
-              const double *den, double *partial, double *rmax, hipStream_t st, double *rmaxHost = nullptr);
-void pcgStepMixed(double *x, const float *s, float *r, const float *q, size_t n, const double *num,
-                  const double *den, double *partial, double *rmax, hipStream_t st, double *rmaxHost = nullptr);
-// z = (double)zf + (double)(float)(num/den) * s   (FP32 zf, FP64 z and s)
-void widenAxpyStep(double *z, const float *zf, const double *s, size_t n, const double *num, const double *den,
+// (vectors: in any one order; values of a reduction as its nb partials)
+// a = (float)(rho / sum sq); x += a * s; r -= a * q; rmax: the partials of
+// |r|_inf, reduceBlocks(n) of them; rf (optional) receives (float)r
+void pcgStep(double *x, const double *s, double *r, const double *q, size_t n, const double *rho, const double *sq,
+             int nsq, double *rmax, hipStream_t st, float *rf = nullptr);
+void pcgStepF(float *x, const float *s, float *r, const float *q, size_t n, const double *rho, const double *sq, int nsq,
+              double *rmax, hipStream_t st);
+void pcgStepMixed(double *x, const float *s, float *r, const float *q, size_t n, const double *rho, const double *sq,
+                  int nsq, double *rmax, hipStream_t st);
+// *rhoNew = sum zr; z += (float)(rhoNew / rho) * s  (Widen: z = (double)zf + ...)
+void pcgDirection(double *z, const double *s, size_t n, const double *zr, int nzr, const double *rho, double *rhoNew,
+                  hipStream_t st);
+void pcgDirectionF(float *z, const float *s, size_t n, const double *zr, int nzr, const double *rho, double *rhoNew,
                    hipStream_t st);
-// x += (double)(float)(sign * num/den) * (double)p   (FP64 x, FP32 p)
-void axpyMixed(double *x, const float *p, size_t n, const double *num, const double *den, double sign,
-               hipStream_t s);
+void pcgDirectionWiden(double *z, const float *zf, const double *s, size_t n, const double *zr, int nzr,
+                       const double *rho, double *rhoNew, hipStream_t st);
 void castToFloat(const double *a, float *b, size_t n, hipStream_t s);
 void addFloatToDouble(double *x, const float *d, size_t n, hipStream_t s);
 void mic0ToFloat(PressureSys &S, hipStream_t s);
@@ -496,17 +511,28 @@ void rowsFromSlots(const ColumnPlan &cp, const T *slots, T *rows, hipStream_t s)
 void slotsFromCells(const PressureSys &S, const ColumnPlan &cp, const float *cells, double *slots, hipStream_t s);
 template <class T>
 void cellsFromSlots(const PressureSys &S, const ColumnPlan &cp, const double *slots, T *cells, hipStream_t s);
-// q = A s and *sq = s . q (the dot in the dot()/dotf() order of the slots)
-void columnSpmvDot(const ColumnPlan &cp, const ColumnSys &C, const double *s, double *q, double *partial, double *sq,
+// q = A s and the partials of s . q (reduceBlocks(cp.slots()) of them, in the
+// dot()/dotf() order of the slots)
+void columnSpmvDot(const ColumnPlan &cp, const ColumnSys &C, const double *s, double *q, double *partial,
                    hipStream_t st);
-void columnSpmvDotF(const ColumnPlan &cp, const ColumnSys &C, const float *s, float *q, double *partial, double *sq,
-                    hipStream_t st);
+void columnSpmvDotF(const ColumnPlan &cp, const ColumnSys &C, const float *s, float *q, double *partial, hipStream_t st);
 // r = b - A x
 void columnResidual(const ColumnPlan &cp, const ColumnSys &C, const double *b, const double *x, double *r,
                     hipStream_t st);
-// z = (L L^T)^-1 r, y = the forward result (slots, distinct from r and z)
-void columnApply(ColumnPlan &cp, const ColumnSys &C, const double *r, double *y, double *z, hipStream_t s);
-void columnApplyF(ColumnPlan &cp, const ColumnSys &C, const float *r, float *y, float *z, hipStream_t s);
+// y = L^-1 r, then z = L^-T y (slots, r, y and z distinct).  Before it the
+// forward launch's first workgroup publishes the largest of rmax's partials to
+// host (publishMax), where rmax is given.
+struct ColumnPublish {
+    const double *rmax = nullptr;
+    int n = 0;
+    double *host = nullptr;
+};
+void columnForward(ColumnPlan &cp, const ColumnSys &C, const double *r, double *y, hipStream_t s,
+                   ColumnPublish pub = ColumnPublish{});
+void columnForward(ColumnPlan &cp, const ColumnSys &C, const float *r, float *y, hipStream_t s,
+                   ColumnPublish pub = ColumnPublish{});
+void columnBackward(ColumnPlan &cp, const ColumnSys &C, const double *y, double *z, hipStream_t s);
+void columnBackward(ColumnPlan &cp, const ColumnSys &C, const float *y, float *z, hipStream_t s);
 
 // ---- MIC(0) application as a line pipeline (kernels_pencil.hip) ----
 // Pencils of 16 x 16 (j, k) lines along i, one workgroup each, one launch per

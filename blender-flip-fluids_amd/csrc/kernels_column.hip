@@ -256,39 +256,25 @@ __global__ __launch_bounds__(256) void columnResidualKernel(size_t slots, const 
 }
 
 template <class T, bool FWD>
-__global__ __launch_bounds__(COL_LANES *COL_WAVES) void columnSweepKernel(ColumnArgs<T, MicRec<T>> a) {
+__global__ __launch_bounds__(COL_LANES *COL_WAVES) void columnSweepKernel(ColumnArgs<T, MicRec<T>> a,
+                                                                          ColumnPublish pub) {
+    if (pub.rmax && blockIdx.x == 0) {
+        publishMax(pub.rmax, pub.n, pub.host);
+        return;
+    }
     columnSweep<T, MicRec<T>, CPF, CPX<T>, FWD>(a, (int)threadIdx.x);
 }
 
-template <class T>
-void columnSweeps(ColumnPlan &cp, const T *r, T *y, T *z, const MicRec<T> *fwd, const MicRec<T> *bwd, hipStream_t st) {
-    ColumnArgs<T, MicRec<T>> a;
-    a.ncj = cp.ncj;
-    a.nck = cp.nck;
-    a.ntj = cp.ntj;
-    a.ntk = cp.ntk;
-    a.cols = cp.cols;
-    a.order = cp.order;
-    a.exJ = cp.exJ;
-    a.exK = cp.exK;
-    a.exSteps = cp.exSteps;
-    a.counter = cp.counter;
-    a.error = cp.error;
-    a.waitTicks = cp.waitTicks;
-    const dim3 grid(cp.ntj * cp.ntk), block(COL_LANES * COL_WAVES);
-    for (int sweep = 0; sweep < 2; sweep++) {
-        a.base = cp.base;
-        if (++cp.epoch == 0) cp.epoch = 1;  // 0 tags the cleared buffer
-        a.epoch = cp.epoch;
-        cp.base += grid.x;
-        a.in = sweep == 0 ? r : y;
-        a.out = sweep == 0 ? y : z;
-        a.rec = sweep == 0 ? fwd : bwd;
-        if (sweep == 0)
-            hipLaunchKernelGGL((columnSweepKernel<T, true>), grid, block, 0, st, a);
-        else
-            hipLaunchKernelGGL((columnSweepKernel<T, false>), grid, block, 0, st, a);
-    }
+template <class T, bool FWD>
+void columnSweepLaunch(ColumnPlan &cp, const T *in, T *out, const MicRec<T> *rec, ColumnPublish pub, hipStream_t st) {
+    const unsigned tiles = (unsigned)cp.ntj * cp.ntk;
+    if (++cp.epoch == 0) cp.epoch = 1;  // 0 tags the cleared buffer
+    ColumnArgs<T, MicRec<T>> a{cp.ncj, cp.nck,     cp.ntj,     cp.ntk,   cp.cols,  cp.order, in,           out,         rec,
+                               cp.exJ, cp.exK,     cp.exSteps, cp.counter, cp.error, cp.base,  cp.epoch,     cp.waitTicks};
+    cp.base += tiles;
+    // the publishing workgroup takes no ticket
+    hipLaunchKernelGGL((columnSweepKernel<T, FWD>), dim3(tiles + (pub.rmax ? 1 : 0)), dim3(COL_LANES * COL_WAVES), 0, st,
+                       a, pub);
     hipCheck(hipGetLastError(), "MIC(0) column sweep launch");
 }
 
@@ -370,21 +356,19 @@ template void cellsFromSlots<float>(const PressureSys &, const ColumnPlan &, con
 template void cellsFromSlots<double>(const PressureSys &, const ColumnPlan &, const double *, double *, hipStream_t);
 
 template <class T>
-static void launchColumnSpmvDot(const ColumnPlan &cp, ColumnMatrix<T> A, const T *x, T *y, double *partial, double *sq,
+static void launchColumnSpmvDot(const ColumnPlan &cp, ColumnMatrix<T> A, const T *x, T *y, double *partial,
                                 hipStream_t st) {
     if (cp.slices == 0) return;
-    const int nb = reduceBlocks(cp.slots());
-    hipLaunchKernelGGL(columnSpmvDotKernel<T>, dim3(nb), dim3(REDUCE_THREADS), 0, st, cp.slots(), cp.links, A, x, y,
-                       partial);
-    reduceFinish(partial, nb, sq, false, st);
+    hipLaunchKernelGGL(columnSpmvDotKernel<T>, dim3(reduceBlocks(cp.slots())), dim3(REDUCE_THREADS), 0, st, cp.slots(),
+                       cp.links, A, x, y, partial);
 }
-void columnSpmvDot(const ColumnPlan &cp, const ColumnSys &C, const double *x, double *y, double *partial, double *sq,
+void columnSpmvDot(const ColumnPlan &cp, const ColumnSys &C, const double *x, double *y, double *partial,
                    hipStream_t st) {
-    launchColumnSpmvDot<double>(cp, ColumnMatrix<double>{C.diag, C.ox, C.oy, C.oz}, x, y, partial, sq, st);
+    launchColumnSpmvDot<double>(cp, ColumnMatrix<double>{C.diag, C.ox, C.oy, C.oz}, x, y, partial, st);
 }
-void columnSpmvDotF(const ColumnPlan &cp, const ColumnSys &C, const float *x, float *y, double *partial, double *sq,
+void columnSpmvDotF(const ColumnPlan &cp, const ColumnSys &C, const float *x, float *y, double *partial,
                     hipStream_t st) {
-    launchColumnSpmvDot<float>(cp, ColumnMatrix<float>{C.fdiag, C.fox, C.foy, C.foz}, x, y, partial, sq, st);
+    launchColumnSpmvDot<float>(cp, ColumnMatrix<float>{C.fdiag, C.fox, C.foy, C.foz}, x, y, partial, st);
 }
 void columnResidual(const ColumnPlan &cp, const ColumnSys &C, const double *b, const double *x, double *r,
                     hipStream_t st) {
@@ -394,11 +378,17 @@ void columnResidual(const ColumnPlan &cp, const ColumnSys &C, const double *b, c
                        ColumnMatrix<double>{C.diag, C.ox, C.oy, C.oz}, b, x, r);
 }
 
-void columnApply(ColumnPlan &cp, const ColumnSys &C, const double *r, double *y, double *z, hipStream_t s) {
-    if (cp.slices > 0) columnSweeps<double>(cp, r, y, z, C.recFwd, C.recBwd, s);
+void columnForward(ColumnPlan &cp, const ColumnSys &C, const double *r, double *y, hipStream_t s, ColumnPublish pub) {
+    if (cp.slices > 0) columnSweepLaunch<double, true>(cp, r, y, C.recFwd, pub, s);
 }
-void columnApplyF(ColumnPlan &cp, const ColumnSys &C, const float *r, float *y, float *z, hipStream_t s) {
-    if (cp.slices > 0) columnSweeps<float>(cp, r, y, z, C.frecFwd, C.frecBwd, s);
+void columnForward(ColumnPlan &cp, const ColumnSys &C, const float *r, float *y, hipStream_t s, ColumnPublish pub) {
+    if (cp.slices > 0) columnSweepLaunch<float, true>(cp, r, y, C.frecFwd, pub, s);
+}
+void columnBackward(ColumnPlan &cp, const ColumnSys &C, const double *y, double *z, hipStream_t s) {
+    if (cp.slices > 0) columnSweepLaunch<double, false>(cp, y, z, C.recBwd, ColumnPublish{}, s);
+}
+void columnBackward(ColumnPlan &cp, const ColumnSys &C, const float *y, float *z, hipStream_t s) {
+    if (cp.slices > 0) columnSweepLaunch<float, false>(cp, y, z, C.frecBwd, ColumnPublish{}, s);
 }
 
 }  // namespace ff

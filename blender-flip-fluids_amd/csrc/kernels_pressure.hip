@@ -241,12 +241,26 @@ __global__ void backwardLevelKernel(const int *nbr, const T *invdiag, const T *l
     z[i] = x * invdiag[i];
 }
 
-// x += a s; r -= a q with a the float-rounded step, and the partial max |r|
+// The value the partials of a reduction stand for, in every thread of the
+// block: the same fold in every block, in the order of the reduction's own
+// second stage, so a kernel that needs the value takes the partials and no
+// launch of one block has to come between (4 us of launch and drain a
+// reduction at any size; a block's fold is about 1.5 us at 1024 partials).
+// Once per OP in a kernel: reduceFold's LDS is not guarded for a second use.
+template <int OP>
+__device__ inline double foldPartials(const double *partial, int nb) {
+    double acc = 0.0;
+    for (int i = threadIdx.x; i < nb; i += REDUCE_THREADS) acc = OP == 0 ? acc + partial[i] : fmax(acc, partial[i]);
+    return reduceFold<OP>(acc);
+}
+
+// x += a s; r -= a q with a = rho / (s . q) the float-rounded step, and the
+// partial max |r|
 template <class TX, class T>
 __global__ __launch_bounds__(REDUCE_THREADS) void pcgStepKernel(TX *x, const T *s, T *r, const T *q, size_t n,
-                                                                const double *num, const double *den,
+                                                                const double *rho, const double *sqPartial, int nsq,
                                                                 double *partial, float *rf) {
-    const double a = *num / *den;
+    const double a = *rho / foldPartials<0>(sqPartial, nsq);
     const float fa = (float)a, fna = (float)(-a);
     const unsigned L = reduceLogicalBlock();
     const size_t span = reduceSpan(n, gridDim.x);
@@ -263,39 +277,23 @@ __global__ __launch_bounds__(REDUCE_THREADS) void pcgStepKernel(TX *x, const T *
     if (threadIdx.x == 0) partial[L] = acc;
 }
 
-// BLAS::addScaled(float alpha, ...) (blaswrapper.h:128-157): the step length
-// is rounded to float before it scales the FP64 vector
-template <class T>
-__global__ void axpyStepKernel(T *y, const T *x, size_t n, const double *num, const double *den,
-                               double sign) {
-    size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= n) return;
-    double a = den ? *num / *den : *num;
-    float fa = (float)(sign * a);
-    y[q] += (T)fa * x[q];
-}
-
-// z = (double)zf + (double)(float)(num/den) * s: the FP32 preconditioner's
-// result widened, then the search-direction update of axpyStepKernel
-__global__ void widenAxpyKernel(double *z, const float *zf, const double *s, size_t n, const double *num,
-                                const double *den) {
-    size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= n) return;
-    const float fa = (float)(*num / *den);
-    double zq = (double)zf[q];
-    zq += (double)fa * s[q];
-    z[q] = zq;
-}
-
-// x += (double)(float)(sign * num/den) * (double)p: the FP64 solution takes
-// the FP32 direction with the same float-rounded step length
-__global__ void axpyMixedKernel(double *x, const float *p, size_t n, const double *num, const double *den,
-                                double sign) {
-    size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= n) return;
-    double a = den ? *num / *den : *num;
-    float fa = (float)(sign * a);
-    x[q] += (double)fa * (double)p[q];
+// the search direction z + (float)(rhoNew / rho) s, into z; rhoNew = z . r from
+// its partials, stored for the next step.  Z: the preconditioner's result,
+// z itself or an FP32 vector that is widened.
+template <class T, class Z>
+__global__ __launch_bounds__(REDUCE_THREADS) void pcgDirectionKernel(T *z, const Z *zin, const T *s, size_t n,
+                                                                     const double *zrPartial, int nzr,
+                                                                     const double *rho, double *rhoNew) {
+    const double num = foldPartials<0>(zrPartial, nzr);
+    const float fa = (float)(num / *rho);
+    const size_t span = reduceSpan(n, gridDim.x);
+    const size_t lo = (size_t)reduceLogicalBlock() * span, hi = lo + span < n ? lo + span : n;
+    for (size_t q = lo + threadIdx.x; q < hi; q += REDUCE_THREADS) {
+        T v = (T)zin[q];
+        v += (T)fa * s[q];
+        z[q] = v;
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) *rhoNew = num;
 }
 
 __global__ void gatherRowsKernel(int m, const int *rows, const double *cells, double *rhs) {
@@ -383,50 +381,44 @@ void mic0ApplyF(const PressureSys &S, const int *hs, const float *r, float *z, h
     micApply<float>(S, hs, S.finvdiag, S.flx, S.fly, S.flz, r, z, s);
 }
 
-void axpyFloatStep(double *y, const double *x, size_t n, const double *num, const double *den,
-                   double sign, hipStream_t s) {
-    if (n == 0) return;
-    hipLaunchKernelGGL(axpyStepKernel<double>, dim3(blocksFor(n, TPB)), dim3(TPB), 0, s, y, x, n, num, den, sign);
-}
-void axpyFloatStepF(float *y, const float *x, size_t n, const double *num, const double *den,
-                    double sign, hipStream_t s) {
-    if (n == 0) return;
-    hipLaunchKernelGGL(axpyStepKernel<float>, dim3(blocksFor(n, TPB)), dim3(TPB), 0, s, y, x, n, num, den, sign);
-}
-
 template <class TX, class T>
-static void launchPcgStep(TX *x, const T *s, T *r, const T *q, size_t n, const double *num, const double *den,
-                          double *partial, double *rmax, hipStream_t st, float *rf = nullptr,
-                          double *rmaxHost = nullptr) {
+static void launchPcgStep(TX *x, const T *s, T *r, const T *q, size_t n, const double *rho, const double *sq, int nsq,
+                          double *rmax, hipStream_t st, float *rf = nullptr) {
     if (n == 0) return;
-    const int nb = reduceBlocks(n);
-    hipLaunchKernelGGL((pcgStepKernel<TX, T>), dim3(nb), dim3(REDUCE_THREADS), 0, st, x, s, r, q, n, num, den,
-                       partial, rf);
-    reduceFinish(partial, nb, rmax, true, st, rmaxHost);
+    hipLaunchKernelGGL((pcgStepKernel<TX, T>), dim3(reduceBlocks(n)), dim3(REDUCE_THREADS), 0, st, x, s, r, q, n, rho,
+                       sq, nsq, rmax, rf);
 }
-void pcgStep(double *x, const double *s, double *r, const double *q, size_t n, const double *num,
-             const double *den, double *partial, double *rmax, hipStream_t st, float *rf, double *rmaxHost) {
-    launchPcgStep<double, double>(x, s, r, q, n, num, den, partial, rmax, st, rf, rmaxHost);
+void pcgStep(double *x, const double *s, double *r, const double *q, size_t n, const double *rho, const double *sq,
+             int nsq, double *rmax, hipStream_t st, float *rf) {
+    launchPcgStep<double, double>(x, s, r, q, n, rho, sq, nsq, rmax, st, rf);
 }
-void pcgStepF(float *x, const float *s, float *r, const float *q, size_t n, const double *num,
-              const double *den, double *partial, double *rmax, hipStream_t st, double *rmaxHost) {
-    launchPcgStep<float, float>(x, s, r, q, n, num, den, partial, rmax, st, nullptr, rmaxHost);
+void pcgStepF(float *x, const float *s, float *r, const float *q, size_t n, const double *rho, const double *sq, int nsq,
+              double *rmax, hipStream_t st) {
+    launchPcgStep<float, float>(x, s, r, q, n, rho, sq, nsq, rmax, st);
 }
-void pcgStepMixed(double *x, const float *s, float *r, const float *q, size_t n, const double *num,
-                  const double *den, double *partial, double *rmax, hipStream_t st, double *rmaxHost) {
-    launchPcgStep<double, float>(x, s, r, q, n, num, den, partial, rmax, st, nullptr, rmaxHost);
+void pcgStepMixed(double *x, const float *s, float *r, const float *q, size_t n, const double *rho, const double *sq,
+                  int nsq, double *rmax, hipStream_t st) {
+    launchPcgStep<double, float>(x, s, r, q, n, rho, sq, nsq, rmax, st);
 }
 
-void widenAxpyStep(double *z, const float *zf, const double *s, size_t n, const double *num, const double *den,
+template <class T, class Z>
+static void launchPcgDirection(T *z, const Z *zin, const T *s, size_t n, const double *zr, int nzr, const double *rho,
+                               double *rhoNew, hipStream_t st) {
+    if (n == 0) return;
+    hipLaunchKernelGGL((pcgDirectionKernel<T, Z>), dim3(reduceBlocks(n)), dim3(REDUCE_THREADS), 0, st, z, zin, s, n, zr,
+                       nzr, rho, rhoNew);
+}
+void pcgDirection(double *z, const double *s, size_t n, const double *zr, int nzr, const double *rho, double *rhoNew,
+                  hipStream_t st) {
+    launchPcgDirection<double, double>(z, z, s, n, zr, nzr, rho, rhoNew, st);
+}
+void pcgDirectionF(float *z, const float *s, size_t n, const double *zr, int nzr, const double *rho, double *rhoNew,
                    hipStream_t st) {
-    if (n == 0) return;
-    hipLaunchKernelGGL(widenAxpyKernel, dim3(blocksFor(n, TPB)), dim3(TPB), 0, st, z, zf, s, n, num, den);
+    launchPcgDirection<float, float>(z, z, s, n, zr, nzr, rho, rhoNew, st);
 }
-
-void axpyMixed(double *x, const float *p, size_t n, const double *num, const double *den, double sign,
-               hipStream_t s) {
-    if (n == 0) return;
-    hipLaunchKernelGGL(axpyMixedKernel, dim3(blocksFor(n, TPB)), dim3(TPB), 0, s, x, p, n, num, den, sign);
+void pcgDirectionWiden(double *z, const float *zf, const double *s, size_t n, const double *zr, int nzr,
+                       const double *rho, double *rhoNew, hipStream_t st) {
+    launchPcgDirection<double, float>(z, zf, s, n, zr, nzr, rho, rhoNew, st);
 }
 
 void gatherRows(const PressureSys &S, const double *cells, double *rhs, hipStream_t s) {

@@ -122,11 +122,8 @@ __global__ __launch_bounds__(RED_THREADS) void reduceStage1(const T *a, const TB
     if (threadIdx.x == 0) partial[L] = acc;
 }
 
-// outHost (optional): a mapped pinned host copy of the result, which the
-// host reads after a stream synchronize instead of copying it back
 template <int OP>
-__global__ __launch_bounds__(RED_THREADS) void reduceStage2(const double *partial, int nb,
-                                                            double *out, double *outHost) {
+__global__ __launch_bounds__(RED_THREADS) void reduceStage2(const double *partial, int nb, double *out) {
     double acc = 0.0;
     for (int i = threadIdx.x; i < nb; i += RED_THREADS) {
         if (OP == 0)
@@ -135,26 +132,39 @@ __global__ __launch_bounds__(RED_THREADS) void reduceStage2(const double *partia
             acc = fmax(acc, partial[i]);
     }
     acc = reduceFold<OP>(acc);
-    if (threadIdx.x == 0) {
-        *out = acc;
-        if (outHost) *outHost = acc;
-    }
+    if (threadIdx.x == 0) *out = acc;
 }
 
 template <class T, int OP, class TB = T>
+void reducePartials(const T *a, const TB *b, size_t n, double *partial, hipStream_t s) {
+    hipLaunchKernelGGL((reduceStage1<T, OP, TB>), dim3(reduceBlocks(n)), dim3(RED_THREADS), 0, s, a, b, n, partial);
+}
+template <class T, int OP, class TB = T>
 void reduce(const T *a, const TB *b, size_t n, double *partial, double *out, hipStream_t s) {
-    int nb = reduceBlocks(n);
-    hipLaunchKernelGGL((reduceStage1<T, OP, TB>), dim3(nb), dim3(RED_THREADS), 0, s, a, b, n, partial);
-    hipLaunchKernelGGL((reduceStage2<OP>), dim3(1), dim3(RED_THREADS), 0, s, partial, nb, out, nullptr);
+    reducePartials<T, OP, TB>(a, b, n, partial, s);
+    hipLaunchKernelGGL((reduceStage2<OP>), dim3(1), dim3(RED_THREADS), 0, s, partial, reduceBlocks(n), out);
+}
+
+// the largest partial, to mapped host memory while other kernels run: the
+// store goes to the host at once
+__global__ __launch_bounds__(RED_THREADS) void publishMaxKernel(const double *partial, int nb, double *host) {
+    publishMax(partial, nb, host);
 }
 
 }  // namespace
 
-void reduceFinish(const double *partial, int nb, double *out, bool isMax, hipStream_t s, double *outHost) {
-    if (isMax)
-        hipLaunchKernelGGL((reduceStage2<1>), dim3(1), dim3(RED_THREADS), 0, s, partial, nb, out, outHost);
-    else
-        hipLaunchKernelGGL((reduceStage2<0>), dim3(1), dim3(RED_THREADS), 0, s, partial, nb, out, outHost);
+void publishMaximum(const double *partial, int nb, double *host, hipStream_t s) {
+    hipLaunchKernelGGL(publishMaxKernel, dim3(1), dim3(RED_THREADS), 0, s, partial, nb, host);
+}
+
+void dotPartials(const double *a, const double *b, size_t n, double *partial, hipStream_t s) {
+    reducePartials<double, 0>(a, b, n, partial, s);
+}
+void dotfPartials(const float *a, const float *b, size_t n, double *partial, hipStream_t s) {
+    reducePartials<float, 0>(a, b, n, partial, s);
+}
+void dotfdPartials(const float *a, const double *b, size_t n, double *partial, hipStream_t s) {
+    reducePartials<float, 0, double>(a, b, n, partial, s);
 }
 
 void dot(const double *a, const double *b, size_t n, double *partial, double *out, hipStream_t s) {

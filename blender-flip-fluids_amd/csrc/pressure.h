@@ -89,6 +89,7 @@ private:
     double *_rowR = nullptr, *_rowY = nullptr, *_rowZ = nullptr;
     float *_rowFR = nullptr, *_rowFY = nullptr, *_rowFZ = nullptr;
     double *_partial = nullptr, *_scal = nullptr;
+    double *_pSq = nullptr, *_pRmax = nullptr, *_pZr = nullptr;  // partials of s . q, |r|_inf and z . r
     double *_hostScal = nullptr, *_hostScalDev = nullptr;  // mapped pinned host slot and its device alias
     std::vector<int> _hLevelStart;
     MicSchedule _ms;
@@ -103,9 +104,14 @@ private:
     int _levelLaunches = 0, _bandLaunches = 0;
     PencilPlan _pp;  // line-pipeline buffers (inside _rowBlock)
     int _sched = 2;
-    // z = M^-1 r with the solver's schedule (y: forward result)
-    void precond(const double *r, double *y, double *z, hipStream_t s);
-    void precondF(const float *r, float *y, float *z, hipStream_t s);
+    // z = M^-1 r with the solver's schedule (y: forward result), whole or in
+    // its two halves
+    template <class T>
+    void precond(const T *r, T *y, T *z, hipStream_t s);
+    template <class T>
+    void precondForward(const T *r, T *y, const double *rmax, hipStream_t s);
+    template <class T>
+    void precondBackward(const T *y, T *z, hipStream_t s);
     int applyLaunches() const { return _sched == 5 ? _bandLaunches : 2; }
     size_t maxRows() const;
     void ensureRowSchedules();
@@ -133,7 +139,8 @@ private:
     void initialGuess(hipStream_t st);
 
     double hostScalar(const double *d, hipStream_t s);
-    double mappedResidual(hipStream_t s);
+    void armResidual();
+    double awaitResidual(hipStream_t s);
     void enqueueTileRanges(bool fp64, hipStream_t s);
     // tile schedule of the preconditioner application for this system
     void buildSchedule(bool fp64, hipStream_t s);
