@@ -17,6 +17,7 @@
 #include <vector>
 
 #include "../../include/ffengine_amd.h"
+#include "host_copy.h"
 #include "kernels.h"
 #include "pressure.h"
 #include "viscosity.h"
@@ -227,8 +228,11 @@ public:
     void getKernelTiming(int id, double *ms, long long *launches) const;
 
 private:
+    void readInterleaved(const float *x, const float *y, const float *z, int start, int end, char *out);
+
     Grid _g;
     hipStream_t _stream = nullptr;
+    HostCopy _hostCopy;
     bool _initialized = false;
     int _currentFrame = 0;
     int _stepNumber = 0;

@@ -900,23 +900,14 @@ void FluidSimulation::removeParticles() {
 
 int FluidSimulation::getNumMarkerParticles() const { return _initialized ? _P.n : 0; }
 
-namespace {
-void interleave(const float *x, const float *y, const float *z, int start, int end, float *out,
-                hipStream_t s) {
-    int n = end - start;
-    if (n <= 0) return;
-    std::vector<float> a(n), b(n), c(n);
-    hipCheck(hipMemcpyAsync(a.data(), x + start, sizeof(float) * n, hipMemcpyDeviceToHost, s), "D2H");
-    hipCheck(hipMemcpyAsync(b.data(), y + start, sizeof(float) * n, hipMemcpyDeviceToHost, s), "D2H");
-    hipCheck(hipMemcpyAsync(c.data(), z + start, sizeof(float) * n, hipMemcpyDeviceToHost, s), "D2H");
-    hipCheck(hipStreamSynchronize(s), "sync");
-    for (int q = 0; q < n; q++) {
-        out[3 * q] = a[q];
-        out[3 * q + 1] = b[q];
-        out[3 * q + 2] = c[q];
-    }
+// three arrays' elements [start, end) into the caller's out, interleaved
+void FluidSimulation::readInterleaved(const float *x, const float *y, const float *z, int start, int end, char *out) {
+    constexpr size_t E = 3 * sizeof(float);
+    _hostCopy.run(out, E * (end - start), _stream, [&](char *dst, size_t lo, size_t n) {
+        const size_t first = start + lo / E;
+        interleave3(x + first, y + first, z + first, n / E, (float *)dst, _stream);
+    });
 }
-}  // namespace
 
 // getMarkerParticleAffine{X,Y,Z}DataRange (fluidsimulation.cpp:3455-3501)
 void FluidSimulation::getMarkerParticleAffineDataRange(int component, int start, int end, char *out) {
@@ -924,21 +915,19 @@ void FluidSimulation::getMarkerParticleAffineDataRange(int component, int start,
         throw std::domain_error("Error: invalid range.\nrange: [" + toString(start) + ", " + toString(end) + "]\n");
     if (!_apic || !_A.a[0])
         throw std::runtime_error("Error: affine data exists with the APIC velocity transfer only.\n");
-    if (end > start)
-        interleave(_A.a[3 * component], _A.a[3 * component + 1], _A.a[3 * component + 2], start, end, (float *)out,
-                   _stream);
+    readInterleaved(_A.a[3 * component], _A.a[3 * component + 1], _A.a[3 * component + 2], start, end, out);
 }
 
 // getMarkerParticle{Position,Velocity}DataRange (fluidsimulation.cpp:3426-3460)
 void FluidSimulation::getMarkerParticlePositionDataRange(int start, int end, char *out) {
     if (start < 0 || end > getNumMarkerParticles() || start > end)
         throw std::domain_error("Error: invalid range.\nrange: [" + toString(start) + ", " + toString(end) + "]\n");
-    if (end > start) interleave(_P.px, _P.py, _P.pz, start, end, (float *)out, _stream);
+    readInterleaved(_P.px, _P.py, _P.pz, start, end, out);
 }
 void FluidSimulation::getMarkerParticleVelocityDataRange(int start, int end, char *out) {
     if (start < 0 || end > getNumMarkerParticles() || start > end)
         throw std::domain_error("Error: invalid range.\nrange: [" + toString(start) + ", " + toString(end) + "]\n");
-    if (end > start) interleave(_P.vx, _P.vy, _P.vz, start, end, (float *)out, _stream);
+    readInterleaved(_P.vx, _P.vy, _P.vz, start, end, out);
 }
 void FluidSimulation::getMarkerParticlePositionData(char *out) {
     getMarkerParticlePositionDataRange(0, getNumMarkerParticles(), out);
@@ -950,8 +939,7 @@ void FluidSimulation::getMarkerParticleVelocityData(char *out) {
 
 void FluidSimulation::getLiquidSDF(float *out) {
     requireInitialized("reading grids");
-    hipCheck(hipMemcpyAsync(out, _phi, sizeof(float) * _phi.n, hipMemcpyDeviceToHost, _stream), "D2H");
-    hipCheck(hipStreamSynchronize(_stream), "sync");
+    _hostCopy.run((char *)out, _phi.p, sizeof(float) * _phi.n, _stream);
 }
 void FluidSimulation::getSolidVelocityField(float *u, float *v, float *w) {
     requireInitialized("getSolidVelocityField");
@@ -960,29 +948,25 @@ void FluidSimulation::getSolidVelocityField(float *u, float *v, float *w) {
     const size_t n[3] = {_u.n, _v.n, _w.n};
     for (int d = 0; d < 3; d++) {
         if (_movingSolid)
-            hipCheck(hipMemcpyAsync(out[d], src[d], sizeof(float) * n[d], hipMemcpyDeviceToHost, _stream), "D2H");
+            _hostCopy.run((char *)out[d], src[d], sizeof(float) * n[d], _stream);
         else
             std::fill(out[d], out[d] + n[d], 0.0f);
     }
-    hipCheck(hipStreamSynchronize(_stream), "solid velocity");
 }
 
 void FluidSimulation::getSolidSDF(float *out) {
     requireInitialized("reading grids");
-    hipCheck(hipMemcpyAsync(out, _solid, sizeof(float) * _solid.n, hipMemcpyDeviceToHost, _stream), "D2H");
-    hipCheck(hipStreamSynchronize(_stream), "sync");
+    _hostCopy.run((char *)out, _solid.p, sizeof(float) * _solid.n, _stream);
 }
 void FluidSimulation::getVelocityField(float *u, float *v, float *w) {
     requireInitialized("reading grids");
-    hipCheck(hipMemcpyAsync(u, _u, sizeof(float) * _u.n, hipMemcpyDeviceToHost, _stream), "D2H");
-    hipCheck(hipMemcpyAsync(v, _v, sizeof(float) * _v.n, hipMemcpyDeviceToHost, _stream), "D2H");
-    hipCheck(hipMemcpyAsync(w, _w, sizeof(float) * _w.n, hipMemcpyDeviceToHost, _stream), "D2H");
-    hipCheck(hipStreamSynchronize(_stream), "sync");
+    _hostCopy.run((char *)u, _u.p, sizeof(float) * _u.n, _stream);
+    _hostCopy.run((char *)v, _v.p, sizeof(float) * _v.n, _stream);
+    _hostCopy.run((char *)w, _w.p, sizeof(float) * _w.n, _stream);
 }
 void FluidSimulation::getPressureGrid(float *out) {
     requireInitialized("reading grids");
-    hipCheck(hipMemcpyAsync(out, _pressure, sizeof(float) * _pressure.n, hipMemcpyDeviceToHost, _stream), "D2H");
-    hipCheck(hipStreamSynchronize(_stream), "sync");
+    _hostCopy.run((char *)out, _pressure.p, sizeof(float) * _pressure.n, _stream);
 }
 void FluidSimulation::getLastPressureSolveStats(int *iterations, double *error, int *success, int *unknowns) {
     *iterations = _lastIters;

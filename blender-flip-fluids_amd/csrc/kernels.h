@@ -275,6 +275,8 @@ void removalFlags(Grid g, const Particles &p, const float *solidNodes, int *keys
                   int *slot, int *offsets, int *perm, int *scanScratch, int maxPerCell,
                   bool extremeRemoval, double maxSpeedSq, int *keep, int *maxCount,
                   hipStream_t s);
+// out[3 q + d] = the d-th of x, y, z at q, q < n (out: device or pinned memory, 16-byte aligned)
+void interleave3(const float *x, const float *y, const float *z, size_t n, float *out, hipStream_t s);
 // stable compaction of the six particle arrays by keep flags (scan in rank)
 void compactParticles(Particles &src, Particles &dst, const int *keep, int *rank,
                       int *scanScratch, hipStream_t s);

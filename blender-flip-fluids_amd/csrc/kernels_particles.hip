@@ -1090,4 +1090,31 @@ void densityAdjoint(Grid g, int np, const float *px, const float *py, const floa
                        xbar);
 }
 
+namespace {
+// A thread stores four floats of the interleaved order in one access, so a
+// wave writes 1 KB of consecutive memory: to pinned host memory the link's
+// rate bounds it (45 MB in 0.83 ms, 54 GB/s; to device memory 0.06 ms).
+__global__ void interleave3Kernel(const float *x, const float *y, const float *z, size_t n, float *out) {
+    const size_t f = 4 * ((size_t)blockIdx.x * blockDim.x + threadIdx.x);
+    if (f >= 3 * n) return;
+    float v[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const size_t e = (f + q) / 3, d = (f + q) % 3;
+        v[q] = e < n ? (d == 0 ? x : d == 1 ? y : z)[e] : 0.0f;
+    }
+    if (f + 4 <= 3 * n) {
+        *(float4 *)(out + f) = make_float4(v[0], v[1], v[2], v[3]);
+    } else {
+        for (int q = 0; f + q < 3 * n; q++) out[f + q] = v[q];
+    }
+}
+}  // namespace
+
+void interleave3(const float *x, const float *y, const float *z, size_t n, float *out, hipStream_t s) {
+    if (n == 0) return;
+    hipLaunchKernelGGL(interleave3Kernel, dim3(blocksFor((3 * n + 3) / 4, TPB)), dim3(TPB), 0, s, x, y, z, n, out);
+    hipCheck(hipGetLastError(), "interleave");
+}
+
 }  // namespace ff

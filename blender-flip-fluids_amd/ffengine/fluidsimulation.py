@@ -20,6 +20,22 @@ GridIndex = collections.namedtuple("GridIndex", "i j k")
 Vector3 = collections.namedtuple("Vector3", "x y z")
 
 
+_PyBytes_FromStringAndSize = ctypes.pythonapi.PyBytes_FromStringAndSize
+_PyBytes_FromStringAndSize.argtypes = [c_char_p, ctypes.c_ssize_t]
+_PyBytes_FromStringAndSize.restype = ctypes.py_object
+_PyBytes_AsString = ctypes.pythonapi.PyBytes_AsString
+_PyBytes_AsString.argtypes = [ctypes.py_object]
+_PyBytes_AsString.restype = c_void_p
+
+
+def _new_bytes(size):
+    """A bytes object with unset contents and the address an entry point fills
+    them at before anyone else sees the object: no cleared buffer and no copy
+    of it."""
+    data = _PyBytes_FromStringAndSize(None, size)
+    return data, _PyBytes_AsString(data)
+
+
 class Vector3_t(ctypes.Structure):
     _fields_ = [("x", c_float), ("y", c_float), ("z", c_float)]
 
@@ -414,12 +430,11 @@ class FluidSimulation(object):
         return _call0(self, "FluidSimulation_get_num_marker_particles", c_int)
 
     def _get_output_data(self, size_name, data_name):
-        size = _call0(self, size_name, c_uint)
-        c_data = (c_char * size)()
+        data, address = _new_bytes(_call0(self, size_name, c_uint))
         f = getattr(lib, data_name)
         pb.init_lib_func(f, [c_void_p, c_void_p, c_void_p], None)
-        pb.execute_lib_func(f, [self(), c_data])
-        return bytes(c_data)
+        pb.execute_lib_func(f, [self(), address])
+        return data
 
     def get_marker_particle_position_data(self):
         return self._get_output_data("FluidSimulation_get_marker_particle_position_data_size",
@@ -430,12 +445,11 @@ class FluidSimulation(object):
                                      "FluidSimulation_get_marker_particle_velocity_data")
 
     def _get_output_data_range(self, name, start_idx, end_idx, size_of_element):
-        n = max(end_idx - start_idx, 0)
-        c_data = (c_char * (n * size_of_element))()
+        data, address = _new_bytes(max(end_idx - start_idx, 0) * size_of_element)
         f = getattr(lib, name)
         pb.init_lib_func(f, [c_void_p, c_int, c_int, c_void_p, c_void_p], None)
-        pb.execute_lib_func(f, [self(), start_idx, end_idx, c_data])
-        return bytes(c_data)
+        pb.execute_lib_func(f, [self(), start_idx, end_idx, address])
+        return data
 
     def get_marker_particle_position_data_range(self, start_idx, end_idx):
         return self._get_output_data_range("FluidSimulation_get_marker_particle_position_data_range",
@@ -478,7 +492,7 @@ class FluidSimulation(object):
 
     # ---- additive read-back (numpy) ----
     def _grid(self, name, shape):
-        a = np.zeros(shape, np.float32)
+        a = np.empty(shape, np.float32)
         f = getattr(lib, name)
         pb.init_lib_func(f, [c_void_p, c_void_p, c_void_p], None)
         pb.execute_lib_func(f, [self(), _fp(a)])
@@ -498,9 +512,9 @@ class FluidSimulation(object):
 
     def get_velocity_field(self):
         i, j, k = self._dims
-        u = np.zeros((k, j, i + 1), np.float32)
-        v = np.zeros((k, j + 1, i), np.float32)
-        w = np.zeros((k + 1, j, i), np.float32)
+        u = np.empty((k, j, i + 1), np.float32)
+        v = np.empty((k, j + 1, i), np.float32)
+        w = np.empty((k + 1, j, i), np.float32)
         f = lib.FluidSimulation_get_velocity_field_data
         pb.init_lib_func(f, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p], None)
         pb.execute_lib_func(f, [self(), _fp(u), _fp(v), _fp(w)])
@@ -510,9 +524,9 @@ class FluidSimulation(object):
         """The solid's face velocities of the last solid rebuild (moving
         obstacles; zero for a static solid)."""
         i, j, k = self._dims
-        u = np.zeros((k, j, i + 1), np.float32)
-        v = np.zeros((k, j + 1, i), np.float32)
-        w = np.zeros((k + 1, j, i), np.float32)
+        u = np.empty((k, j, i + 1), np.float32)
+        v = np.empty((k, j + 1, i), np.float32)
+        w = np.empty((k + 1, j, i), np.float32)
         f = lib.FluidSimulation_get_solid_velocity_field
         pb.init_lib_func(f, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p], None)
         pb.execute_lib_func(f, [self(), _fp(u), _fp(v), _fp(w)])
