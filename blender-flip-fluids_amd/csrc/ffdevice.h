@@ -238,17 +238,6 @@ FF_HD Box boundaryBox(int ni, int nj, int nk, double dx) {
     return b;
 }
 
-// Order-preserving map of a float onto an unsigned key, so that an unsigned
-// min over keys is the float min (used for deterministic LDS min-reductions).
-FF_HD uint32_t floatKey(float f) {
-    uint32_t u = __builtin_bit_cast(uint32_t, f);
-    return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
-}
-FF_HD float keyFloat(uint32_t k) {
-    uint32_t u = (k & 0x80000000u) ? (k & 0x7fffffffu) : ~k;
-    return __builtin_bit_cast(float, u);
-}
-
 // Interpolation::trilinearInterpolate(double p[8], x, y, z) (interpolation.cpp:61-70)
 FF_HD double trilin8(const double *p, double x, double y, double z) {
     return p[0] * (1 - x) * (1 - y) * (1 - z) + p[1] * x * (1 - y) * (1 - z) +
