@@ -44,11 +44,12 @@
 //
 // Measured, one application (both sweeps) FP64 / FP32, against launches over
 // bands of 8 / 12 hyperplanes: 24^3 99 / 86 -> 42 / 35 us, 64^3 237 / 201 ->
-// 110 / 83, 128^3 513 / 441 -> 229 / 171, 256^3 dam break 1267 / 1058 -> 528 /
-// 396.  Two lines a lane and two waves a tile were the fastest of (lines,
+// 108 / 80, 128^3 513 / 441 -> 217 / 162, 256^3 dam break 1267 / 1058 -> 473 /
+// 353.  Two lines a lane and two waves a tile were the fastest of (lines,
 // waves) = (1,4) (2,2) (2,4) (4,1) (4,2) (2,1): 167 / 223 us FP32 / FP64 for a
-// sweep of 96 x 160 x 256, the others 160 / 297 to 199 / 360.  A 16 x 16 tile
-// with an LDS plane and a barrier per step took 0.22 us a step against 0.15.
+// sweep of 96 x 160 x 256, the others 160 / 297 to 199 / 360 (all before the
+// head of the loop matched its steps, see columnSteps).  A 16 x 16 tile with
+// an LDS plane and a barrier per step took 0.22 us a step against 0.15.
 //
 // This header holds only the sweep's body; its includer supplies the hardware
 // operations as macros (see kernels_column.hip).
@@ -193,18 +194,31 @@ FF_CS_DEVICE void columnSteps(const ColumnArgs<T, Rec> &a, const ColumnWave<T> &
         }
         return v;
     };
+    auto store = [&](const T (&v)[R], int u) {
+        unsigned p[R][N];
+#pragma unroll
+        for (int r = 0; r < R; r++) Word::pack(v[r], a.epoch, p[r]);
+        FF_CS_STORE_WORDS(p, w.toJ, w.toJ0 + (unsigned)u * JSTEP);
+        if (LAST) FF_CS_STORE_WORDS(p[FWD ? R - 1 : 0], w.toK, w.toK0 + (unsigned)u * KSTEP);
+        FF_CS_STORE(v, w.out, lane * (unsigned)(R * sizeof(T)) + slice(u) * SLICE);
+    };
     int taken = 0;
     T prev[R];  // the lines' results of the previous step
 #pragma unroll
     for (int r = 0; r < R; r++) prev[r] = T(0);
     Slot ring[PF];
+    // The accesses of the PF steps before the first, in a step's order: stores
+    // that go nowhere, words past the ends.  The counter a wave waits on counts
+    // loads and stores alike, and at the loop's head the compiler takes the
+    // smaller distance of the two ways in: with a head of loads only, every
+    // step waited for all but its last 11 accesses, some of them stores to
+    // memory (96 x 160 x 256: 168 us FP32, 224 us FP64 a sweep; so 151, 205).
 #pragma unroll
     for (int q = 0; q < PF; q++) {
+        store(prev, q - PF);
+        loadJ(ring[(q + PX) % PF].j, q - PF + PX);
+        if (FIRST) loadK(ring[(q + PX) % PF].k, q - PF + PX);
         operands(ring[q], q);
-        if (q < PX) {
-            loadJ(ring[q].j, q);
-            if (FIRST) loadK(ring[q].k, q);
-        }
     }
     T nextK = T(0);
     if (!FIRST) nextK = ringK(0);
@@ -283,12 +297,7 @@ FF_CS_DEVICE void columnSteps(const ColumnArgs<T, Rec> &a, const ColumnWave<T> &
                 FF_CS_WAVE_ORDER();
                 FF_CS_LDS_STORE(&w.own->made, u + 1);
             }
-            unsigned p[R][N];
-#pragma unroll
-            for (int r = 0; r < R; r++) Word::pack(prev[r], a.epoch, p[r]);
-            FF_CS_STORE_WORDS(p, w.toJ, w.toJ0 + (unsigned)u * JSTEP);
-            if (LAST) FF_CS_STORE_WORDS(p[FWD ? R - 1 : 0], w.toK, w.toK0 + (unsigned)u * KSTEP);
-            FF_CS_STORE(prev, w.out, lane * (unsigned)(R * sizeof(T)) + slice(u) * SLICE);
+            store(prev, u);
             loadJ(ring[(q + PX) % PF].j, u + PX);
             if (FIRST) loadK(ring[(q + PX) % PF].k, u + PX);
             operands(ring[q], u + PF);
