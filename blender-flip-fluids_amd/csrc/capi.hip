@@ -614,8 +614,8 @@ void FFAMD_extrapolate(int wi, int wj, int wk, float *field, const unsigned char
         DBuf<uint8_t> vb(n), st(n);
         up(a.p, field, n, sc.s);
         up(vb.p, valid, n, sc.s);
-        ff::extrapolateInit(wi, wj, wk, vb, st, sc.s);
-        for (int l = 0; l < layers; l++) ff::extrapolateLayer(wi, wj, wk, a, st, l, sc.s);
+        const ff::ExtrapolateField f{wi, wj, wk, vb, st, a};
+        ff::extrapolate(&f, 1, layers, sc.s);
         down(field, a.p, n, sc.s);
         sync(sc.s);
     });
@@ -664,8 +664,8 @@ void FFAMD_extrapolate_noalloc(int wi, int wj, int wk, float *field, const unsig
         unsigned char *st = deviceScratch();
         hipStream_t s = (hipStream_t)stream;
         // every status byte is written by the first kernel: nothing to clear
-        ff::extrapolateInit(wi, wj, wk, valid, st, s);
-        for (int l = 0; l < layers; l++) ff::extrapolateLayer(wi, wj, wk, field, st, l, s);
+        const ff::ExtrapolateField f{wi, wj, wk, valid, st, field};
+        ff::extrapolate(&f, 1, layers, s);
         ff::hipCheck(hipGetLastError(), "extrapolation launch");
     });
 }
@@ -683,8 +683,8 @@ void FFAMD_extrapolate_vjp(int wi, int wj, int wk, float *bar, const unsigned ch
         // the status bytes depend on the flags only: run the forward's layers
         // on a scratch field to get them
         ff::hipCheck(hipMemsetAsync(dummy, 0, sizeof(float) * n, sc.s), "memset");
-        ff::extrapolateInit(wi, wj, wk, vb, st, sc.s);
-        for (int l = 0; l < layers; l++) ff::extrapolateLayer(wi, wj, wk, dummy, st, l, sc.s);
+        const ff::ExtrapolateField f{wi, wj, wk, vb, st, dummy};
+        ff::extrapolate(&f, 1, layers, sc.s);
         ff::extrapolateAdjoint(wi, wj, wk, a, st, layers, sc.s);
         down(bar, a.p, n, sc.s);
         sync(sc.s);

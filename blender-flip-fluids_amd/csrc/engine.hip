@@ -669,15 +669,10 @@ void FluidSimulation::step(double dt) {
 
 void FluidSimulation::extrapolate(int layers) {
     const int ni = _g.ni, nj = _g.nj, nk = _g.nk;
-    _timers.begin(T_EXTRAPOLATE, _stream, 3 * layers + 3);
-    extrapolateInit(ni + 1, nj, nk, _vu, _stu, _stream);
-    extrapolateInit(ni, nj + 1, nk, _vv, _stv, _stream);
-    extrapolateInit(ni, nj, nk + 1, _vw, _stw, _stream);
-    for (int l = 0; l < layers; l++) {
-        extrapolateLayer(ni + 1, nj, nk, _u, _stu, l, _stream);
-        extrapolateLayer(ni, nj + 1, nk, _v, _stv, l, _stream);
-        extrapolateLayer(ni, nj, nk + 1, _w, _stw, l, _stream);
-    }
+    _timers.begin(T_EXTRAPOLATE, _stream, layers + 1);
+    const ExtrapolateField f[3] = {{ni + 1, nj, nk, _vu, _stu, _u}, {ni, nj + 1, nk, _vv, _stv, _v},
+                                   {ni, nj, nk + 1, _vw, _stw, _w}};
+    ff::extrapolate(f, 3, layers, _stream);
     _timers.end(T_EXTRAPOLATE, _stream);
 }
 

@@ -282,8 +282,15 @@ void compactParticles(Particles &src, Particles &dst, const int *keep, int *rank
                       int *scanScratch, hipStream_t s);
 
 // ---- grid stencils (kernels_grid.hip) ----
-void extrapolateInit(int wi, int wj, int wk, const uint8_t *valid, uint8_t *stat, hipStream_t s);
-void extrapolateLayer(int wi, int wj, int wk, float *field, uint8_t *stat, int layer, hipStream_t s);
+// the layered extrapolation of up to three fields at once, in place; st
+// receives each face's status
+struct ExtrapolateField {
+    int wi, wj, wk;
+    const uint8_t *valid;
+    uint8_t *st;
+    float *a;
+};
+void extrapolate(const ExtrapolateField *fields, int count, int layers, hipStream_t s);
 // adjoint of the layered extrapolation (for the status the forward's
 // `layers` layers left), in place on the face cotangent bar
 void extrapolateAdjoint(int wi, int wj, int wk, float *bar, const uint8_t *stat, int layers, hipStream_t s);

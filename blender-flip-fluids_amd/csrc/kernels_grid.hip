@@ -1,6 +1,8 @@
 // kernels_grid.hip -- face-array stencils of the FLIP substep: layered
 // velocity extrapolation, body force, solid constraint and the pressure
 // gradient update.
+#include <algorithm>
+
 #include "kernels.h"
 
 namespace ff {
@@ -20,7 +22,20 @@ constexpr uint8_t ST_BORDER = 254, ST_UNKNOWN = 255;
 // gridutils.cpp:120-175).  Faces written in this layer get L+1, which neither
 // the front test (== L) nor the DONE test (<= L) accepts, so one in-place pass
 // per layer is race free.
-__global__ void extrapInitKernel(int wi, int wj, int wk, const uint8_t *valid, uint8_t *st) {
+//
+// What bounds it: the chain of layers, 1 + layers launches, and in each the
+// status bytes (a layer fills few faces).  A launch takes every field of the
+// call, and a thread four faces: it looks at their status and their
+// neighbours' as words, whatever their alignment, and goes on only if one is
+// unknown and one is the front.  Both extrapolations of a substep, against a
+// byte a thread and a launch per field: 24^3 0.24 -> 0.15 ms, 128^3 0.60 -> 0.40,
+// 256^3 3.0 -> 2.5.
+struct ExtrapolateFields {
+    ExtrapolateField f[3];
+};
+__global__ void extrapInitKernel(ExtrapolateFields F) {
+    const ExtrapolateField &D = F.f[blockIdx.y];
+    const int wi = D.wi, wj = D.wj, wk = D.wk;
     size_t f = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     size_t n = (size_t)wi * wj * wk;
     if (f >= n) return;
@@ -29,15 +44,23 @@ __global__ void extrapInitKernel(int wi, int wj, int wk, const uint8_t *valid, u
     if (i == 0 || j == 0 || k == 0 || i == wi - 1 || j == wj - 1 || k == wk - 1)
         s = ST_BORDER;
     else
-        s = valid[f] ? 0 : ST_UNKNOWN;
-    st[f] = s;
+        s = D.valid[f] ? 0 : ST_UNKNOWN;
+    D.st[f] = s;
 }
 
-__global__ void extrapLayerKernel(int wi, int wj, int wk, float *a, uint8_t *st, int L) {
-    size_t f = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    size_t n = (size_t)wi * wj * wk;
-    if (f >= n || st[f] != ST_UNKNOWN) return;
-    const long long nb[6] = {1, -1, wi, -(long long)wi, (long long)wi * wj, -(long long)wi * wj};
+__device__ __forceinline__ uint32_t statusWord(const uint8_t *p) {
+    uint32_t w;
+    __builtin_memcpy(&w, p, 4);  // any alignment
+    return w;
+}
+// not zero if a byte of w is zero
+__device__ __forceinline__ uint32_t zeroBytes(uint32_t w) { return (w - 0x01010101u) & ~w & 0x80808080u; }
+
+__device__ void extrapFace(const ExtrapolateField &D, size_t f, int L) {
+    float *a = D.a;
+    uint8_t *st = D.st;
+    const long long row = D.wi, plane = (long long)D.wi * D.wj;
+    const long long nb[6] = {1, -1, row, -row, plane, -plane};
     uint8_t s[6];
     bool front = false;
 #pragma unroll
@@ -56,6 +79,27 @@ __global__ void extrapLayerKernel(int wi, int wj, int wk, float *a, uint8_t *st,
         }
     a[f] = sum / (float)count;
     st[f] = (uint8_t)(L + 1);
+}
+
+__global__ void extrapLayerKernel(ExtrapolateFields F, int L) {
+    const ExtrapolateField &D = F.f[blockIdx.y];
+    const size_t row = D.wi, plane = (size_t)D.wi * D.wj, n = plane * D.wk;
+    const size_t f = 4 * ((size_t)blockIdx.x * blockDim.x + threadIdx.x);
+    if (f >= n) return;
+    const uint8_t *st = D.st + f;
+    // the words of all four faces' neighbours are in the array (a face of the
+    // first and last plane is border)
+    if (f >= plane && f + 4 + plane <= n) {
+        if (!zeroBytes(~statusWord(st))) return;
+        const uint32_t l = 0x01010101u * (uint32_t)L;
+        if (!(zeroBytes(statusWord(st + 1) ^ l) | zeroBytes(statusWord(st - 1) ^ l) | zeroBytes(statusWord(st + row) ^ l) |
+              zeroBytes(statusWord(st - row) ^ l) | zeroBytes(statusWord(st + plane) ^ l) |
+              zeroBytes(statusWord(st - plane) ^ l)))
+            return;
+    }
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+        if (f + q < n && st[q] == ST_UNKNOWN) extrapFace(D, f + q, L);
 }
 
 // Adjoint of layer L of extrapLayerKernel, given the status bytes the
@@ -210,14 +254,16 @@ __global__ void applyPressureKernel(Grid g, double dt, const float *p, const flo
 
 }  // namespace
 
-void extrapolateInit(int wi, int wj, int wk, const uint8_t *valid, uint8_t *st, hipStream_t s) {
-    size_t n = (size_t)wi * wj * wk;
-    hipLaunchKernelGGL(extrapInitKernel, dim3(blocksFor(n, TPB)), dim3(TPB), 0, s, wi, wj, wk, valid, st);
-}
-
-void extrapolateLayer(int wi, int wj, int wk, float *a, uint8_t *st, int layer, hipStream_t s) {
-    size_t n = (size_t)wi * wj * wk;
-    hipLaunchKernelGGL(extrapLayerKernel, dim3(blocksFor(n, TPB)), dim3(TPB), 0, s, wi, wj, wk, a, st, layer);
+void extrapolate(const ExtrapolateField *fields, int count, int layers, hipStream_t s) {
+    ExtrapolateFields F{};
+    size_t n = 0;
+    for (int d = 0; d < count; d++) {
+        F.f[d] = fields[d];
+        n = std::max(n, (size_t)fields[d].wi * fields[d].wj * fields[d].wk);
+    }
+    hipLaunchKernelGGL(extrapInitKernel, dim3(blocksFor(n, TPB), count), dim3(TPB), 0, s, F);
+    for (int l = 0; l < layers; l++)
+        hipLaunchKernelGGL(extrapLayerKernel, dim3(blocksFor((n + 3) / 4, TPB), count), dim3(TPB), 0, s, F, l);
 }
 
 void extrapolateAdjoint(int wi, int wj, int wk, float *bar, const uint8_t *st, int layers, hipStream_t s) {

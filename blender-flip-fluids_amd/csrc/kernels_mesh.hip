@@ -1029,8 +1029,8 @@ void normalizeSolidVelocity(Grid g, const SolidVelocityData &d, float *us, float
         const size_t nf = faceCount(g, q);
         hipLaunchKernelGGL(normalizeVelocityKernel, dim3(blocksFor(nf, 256)), dim3(256), 0, s, d.f[q], d.w[q], nf,
                            out[q], valid);
-        extrapolateInit(wi[q], wj[q], wk[q], valid, status, s);
-        for (int l = 0; l < layers; l++) extrapolateLayer(wi[q], wj[q], wk[q], out[q], status, l, s);
+        const ExtrapolateField f{wi[q], wj[q], wk[q], valid, status, out[q]};
+        extrapolate(&f, 1, layers, s);
     }
     hipCheck(hipGetLastError(), "normalize solid velocity");
 }

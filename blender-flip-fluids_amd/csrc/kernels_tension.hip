@@ -393,8 +393,8 @@ void curvatureGrid(Grid g, const float *phi, TensionBuffers &B, hipStream_t s) {
     const float upper = (BAND - 1) * g.dx;
     curvatureKernel<<<nbN, TPB, 0, s>>>(D, out, upper, g.dx, B.cv, B.curvature);
     hipCheck(hipGetLastError(), "curvature launch");
-    extrapolateInit(g.ni, g.nj, g.nk, B.cv, B.ext, s);
-    for (int l = 0; l < LAYERS; l++) extrapolateLayer(g.ni, g.nj, g.nk, B.curvature, B.ext, l, s);
+    const ExtrapolateField f{g.ni, g.nj, g.nk, B.cv, B.ext, B.curvature};
+    extrapolate(&f, 1, LAYERS, s);
     B.surface = out;
 }
 

@@ -175,9 +175,9 @@ void Rollout::substep(int k, bool freeze, bool record) {
         off += _nf[d];
     }
     const int wi[3] = {g.ni + 1, g.ni, g.ni}, wj[3] = {g.nj, g.nj + 1, g.nj}, wk[3] = {g.nk, g.nk, g.nk + 1};
-    for (int d = 0; d < 3; d++) extrapolateInit(wi[d], wj[d], wk[d], _valid[d], _st0[d], _s);
-    for (int l = 0; l < _layers; l++)
-        for (int d = 0; d < 3; d++) extrapolateLayer(wi[d], wj[d], wk[d], _u[d], _st0[d], l, _s);
+    ExtrapolateField before[3];
+    for (int d = 0; d < 3; d++) before[d] = ExtrapolateField{wi[d], wj[d], wk[d], _valid[d], _st0[d], _u[d]};
+    extrapolate(before, 3, _layers, _s);
     for (int d = 0; d < 3; d++) copyD(_su[d].p, _u[d].p, sizeof(float) * _nf[d], _s);
     // the body force is a float vector scaled by the double substep length
     // (fluidsimulation.cpp:5837-5876)
@@ -190,9 +190,9 @@ void Rollout::substep(int k, bool freeze, bool record) {
     if (!r.success) throw std::runtime_error("rollout: a pressure solve did not converge");
     applyPressure(g, _st.dt, _pressure, _phi, _wt[0], _wt[1], _wt[2], _u[0], _u[1], _u[2], _valid[0], _valid[1],
                   _valid[2], _s);
-    for (int d = 0; d < 3; d++) extrapolateInit(wi[d], wj[d], wk[d], _valid[d], _st1[d], _s);
-    for (int l = 0; l < _layers; l++)
-        for (int d = 0; d < 3; d++) extrapolateLayer(wi[d], wj[d], wk[d], _u[d], _st1[d], l, _s);
+    ExtrapolateField after[3];
+    for (int d = 0; d < 3; d++) after[d] = ExtrapolateField{wi[d], wj[d], wk[d], _valid[d], _st1[d], _u[d]};
+    extrapolate(after, 3, _layers, _s);
     for (int d = 0; d < 3; d++) {
         copyD(_cu[d].p, _su[d].p, sizeof(float) * _nf[d], _s);
         constrainFaces(_cu[d], _wt[d], _nf[d], _s);
