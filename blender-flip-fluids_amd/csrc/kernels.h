@@ -143,6 +143,19 @@ __device__ inline double reduceFold(double v) {
     for (int q = 1; q < REDUCE_THREADS / 64; q++) acc = OP == 0 ? acc + waves[q] : fmax(acc, waves[q]);
     return acc;
 }
+// The value the partials of a reduction stand for, in every thread of the
+// block: the same fold in every block, in the order of the reduction's own
+// second stage, so a kernel that needs the value takes the partials and no
+// launch of one block has to come between (4 us of launch and drain a
+// reduction at any size; a block's fold is about 1.5 us at 1024 partials).
+// reduceFold's LDS is not guarded for a second use of the same OP in a kernel: a
+// barrier has to come between.
+template <int OP>
+__device__ inline double foldPartials(const double *partial, int nb) {
+    double acc = 0.0;
+    for (int i = threadIdx.x; i < nb; i += REDUCE_THREADS) acc = OP == 0 ? acc + partial[i] : fmax(acc, partial[i]);
+    return reduceFold<OP>(acc);
+}
 // the partials of a dot product only (reduceBlocks(n) of them), for a kernel
 // that folds them itself
 void dotPartials(const double *a, const double *b, size_t n, double *partial, hipStream_t s);
@@ -436,13 +449,9 @@ void pcgStepF(float *x, const float *s, float *r, const float *q, size_t n, cons
               double *rmax, hipStream_t st);
 void pcgStepMixed(double *x, const float *s, float *r, const float *q, size_t n, const double *rho, const double *sq,
                   int nsq, double *rmax, hipStream_t st);
-// *rhoNew = sum zr; z += (float)(rhoNew / rho) * s  (Widen: z = (double)zf + ...)
+// *rhoNew = sum zr; z += (float)(rhoNew / rho) * s
 void pcgDirection(double *z, const double *s, size_t n, const double *zr, int nzr, const double *rho, double *rhoNew,
                   hipStream_t st);
-void pcgDirectionF(float *z, const float *s, size_t n, const double *zr, int nzr, const double *rho, double *rhoNew,
-                   hipStream_t st);
-void pcgDirectionWiden(double *z, const float *zf, const double *s, size_t n, const double *zr, int nzr,
-                       const double *rho, double *rhoNew, hipStream_t st);
 void castToFloat(const double *a, float *b, size_t n, hipStream_t s);
 void addFloatToDouble(double *x, const float *d, size_t n, hipStream_t s);
 void mic0ToFloat(PressureSys &S, hipStream_t s);
@@ -525,6 +534,12 @@ void cellsFromSlots(const PressureSys &S, const ColumnPlan &cp, const double *sl
 void columnSpmvDot(const ColumnPlan &cp, const ColumnSys &C, const double *s, double *q, double *partial,
                    hipStream_t st);
 void columnSpmvDotF(const ColumnPlan &cp, const ColumnSys &C, const float *s, float *q, double *partial, hipStream_t st);
+// the next direction's product: *rhoNew = sum zr, t = z + (float)(rhoNew / rho) s,
+// q = A t and the partials of t . q (z: FP32 beside FP64 vectors is widened)
+template <class T, class Z>
+void columnDirectionSpmvDot(const ColumnPlan &cp, const ColumnSys &C, const Z *z, const T *s, T *t, T *q,
+                            const double *zr, int nzr, const double *rho, double *rhoNew, double *partial,
+                            hipStream_t st);
 // r = b - A x
 void columnResidual(const ColumnPlan &cp, const ColumnSys &C, const double *b, const double *x, double *r,
                     hipStream_t st);

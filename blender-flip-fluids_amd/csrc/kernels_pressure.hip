@@ -241,19 +241,6 @@ __global__ void backwardLevelKernel(const int *nbr, const T *invdiag, const T *l
     z[i] = x * invdiag[i];
 }
 
-// The value the partials of a reduction stand for, in every thread of the
-// block: the same fold in every block, in the order of the reduction's own
-// second stage, so a kernel that needs the value takes the partials and no
-// launch of one block has to come between (4 us of launch and drain a
-// reduction at any size; a block's fold is about 1.5 us at 1024 partials).
-// Once per OP in a kernel: reduceFold's LDS is not guarded for a second use.
-template <int OP>
-__device__ inline double foldPartials(const double *partial, int nb) {
-    double acc = 0.0;
-    for (int i = threadIdx.x; i < nb; i += REDUCE_THREADS) acc = OP == 0 ? acc + partial[i] : fmax(acc, partial[i]);
-    return reduceFold<OP>(acc);
-}
-
 // x += a s; r -= a q with a = rho / (s . q) the float-rounded step, and the
 // partial max |r|
 template <class TX, class T>
@@ -278,21 +265,15 @@ __global__ __launch_bounds__(REDUCE_THREADS) void pcgStepKernel(TX *x, const T *
 }
 
 // the search direction z + (float)(rhoNew / rho) s, into z; rhoNew = z . r from
-// its partials, stored for the next step.  Z: the preconditioner's result,
-// z itself or an FP32 vector that is widened.
-template <class T, class Z>
-__global__ __launch_bounds__(REDUCE_THREADS) void pcgDirectionKernel(T *z, const Z *zin, const T *s, size_t n,
+// its partials, stored for the next step
+__global__ __launch_bounds__(REDUCE_THREADS) void pcgDirectionKernel(double *z, const double *s, size_t n,
                                                                      const double *zrPartial, int nzr,
                                                                      const double *rho, double *rhoNew) {
     const double num = foldPartials<0>(zrPartial, nzr);
     const float fa = (float)(num / *rho);
     const size_t span = reduceSpan(n, gridDim.x);
     const size_t lo = (size_t)reduceLogicalBlock() * span, hi = lo + span < n ? lo + span : n;
-    for (size_t q = lo + threadIdx.x; q < hi; q += REDUCE_THREADS) {
-        T v = (T)zin[q];
-        v += (T)fa * s[q];
-        z[q] = v;
-    }
+    for (size_t q = lo + threadIdx.x; q < hi; q += REDUCE_THREADS) z[q] += (double)fa * s[q];
     if (blockIdx.x == 0 && threadIdx.x == 0) *rhoNew = num;
 }
 
@@ -401,24 +382,11 @@ void pcgStepMixed(double *x, const float *s, float *r, const float *q, size_t n,
     launchPcgStep<double, float>(x, s, r, q, n, rho, sq, nsq, rmax, st);
 }
 
-template <class T, class Z>
-static void launchPcgDirection(T *z, const Z *zin, const T *s, size_t n, const double *zr, int nzr, const double *rho,
-                               double *rhoNew, hipStream_t st) {
-    if (n == 0) return;
-    hipLaunchKernelGGL((pcgDirectionKernel<T, Z>), dim3(reduceBlocks(n)), dim3(REDUCE_THREADS), 0, st, z, zin, s, n, zr,
-                       nzr, rho, rhoNew);
-}
 void pcgDirection(double *z, const double *s, size_t n, const double *zr, int nzr, const double *rho, double *rhoNew,
                   hipStream_t st) {
-    launchPcgDirection<double, double>(z, z, s, n, zr, nzr, rho, rhoNew, st);
-}
-void pcgDirectionF(float *z, const float *s, size_t n, const double *zr, int nzr, const double *rho, double *rhoNew,
-                   hipStream_t st) {
-    launchPcgDirection<float, float>(z, z, s, n, zr, nzr, rho, rhoNew, st);
-}
-void pcgDirectionWiden(double *z, const float *zf, const double *s, size_t n, const double *zr, int nzr,
-                       const double *rho, double *rhoNew, hipStream_t st) {
-    launchPcgDirection<double, float>(z, zf, s, n, zr, nzr, rho, rhoNew, st);
+    if (n == 0) return;
+    hipLaunchKernelGGL(pcgDirectionKernel, dim3(reduceBlocks(n)), dim3(REDUCE_THREADS), 0, st, z, s, n, zr, nzr, rho,
+                       rhoNew);
 }
 
 void gatherRows(const PressureSys &S, const double *cells, double *rhs, hipStream_t s) {

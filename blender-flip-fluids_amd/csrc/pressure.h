@@ -83,8 +83,8 @@ private:
     ColumnPlan _cp;
     ColumnSys _C{};
     // the PCG's vectors, in slots
-    double *_x = nullptr, *_r = nullptr, *_z = nullptr, *_s = nullptr, *_y = nullptr;
-    float *_fr = nullptr, *_fz = nullptr, *_fs = nullptr, *_fd = nullptr, *_fq = nullptr, *_fy = nullptr;
+    double *_x = nullptr, *_r = nullptr, *_z = nullptr, *_s = nullptr, *_y = nullptr, *_t0 = nullptr;
+    float *_fr = nullptr, *_fz = nullptr, *_fs = nullptr, *_fd = nullptr, *_fq = nullptr, *_fy = nullptr, *_ft = nullptr;
     // an application's operands in row order (row-ordered schedules and dots)
     double *_rowR = nullptr, *_rowY = nullptr, *_rowZ = nullptr;
     float *_rowFR = nullptr, *_rowFY = nullptr, *_rowFZ = nullptr;
@@ -139,6 +139,7 @@ private:
     void initialGuess(hipStream_t st);
 
     double hostScalar(const double *d, hipStream_t s);
+    void nextProduct(float *&s, float *&t, bool &first, double *&rho, double *&rhoNew, hipStream_t st);
     void armResidual();
     double awaitResidual(hipStream_t s);
     void enqueueTileRanges(bool fp64, hipStream_t s);

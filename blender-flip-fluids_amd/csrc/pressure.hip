@@ -55,7 +55,7 @@ void PressureSolver::allocate(Grid g) {
     size_t oOrder = b.take(4 * (size_t)_cp.ntj * _cp.ntk);
     size_t oLinks = b.take(sizeof(SliceLinks) * _cp.maxSlices), oSlotRow = b.take(4 * E), oTotal = b.take(4);
     size_t oExJ = b.take(4 * _cp.exJWords), oExK = b.take(4 * _cp.exKWords), oCounter = b.take(4);
-    size_t oC[5], oCF[4], oV[5], oFV[6];
+    size_t oC[5], oCF[4], oV[6], oFV[4];
     for (auto &o : oC) o = b.take(8 * E);
     for (auto &o : oCF) o = b.take(4 * E);
     for (auto &o : oV) o = b.take(8 * E);
@@ -100,8 +100,13 @@ void PressureSolver::allocate(Grid g) {
     _C.frecFwd = (MicRec<float> *)(m + oRec[0]); _C.frecBwd = (MicRec<float> *)(m + oRec[1]);
     _x = (double *)(m + oV[0]); _r = (double *)(m + oV[1]); _z = (double *)(m + oV[2]); _s = (double *)(m + oV[3]);
     _y = (double *)(m + oV[4]);
+    _t0 = (double *)(m + oV[5]);
     _fr = (float *)(m + oFV[0]); _fz = (float *)(m + oFV[1]); _fs = (float *)(m + oFV[2]);
-    _fd = (float *)(m + oFV[3]); _fq = (float *)(m + oFV[4]); _fy = (float *)(m + oFV[5]);
+    _fy = (float *)(m + oFV[3]);
+    // of no use to the modes with FP32 vectors: places of theirs
+    _fd = (float *)_t0;
+    _fq = _fd + E;
+    _ft = (float *)_s;
     _S.ni = g.ni;
     _S.nj = g.nj;
     _S.nk = g.nk;
@@ -584,19 +589,30 @@ bool PressureSolver::pcgFP64(double tolFactor, int maxIter, double resid0, int &
         return false;
     }
     hipCheck(hipMemcpyAsync(_s, _z, sizeof(double) * n, hipMemcpyDeviceToDevice, st), "copy");
-    double *s = _s, *z = _z;
+    // q shares the forward sweep's place: it is read before the sweep
+    double *s = _s, *z = _z, *t = _t0, *q = _y;
     int it;
     for (it = 0; it < maxIter; it++) {
+        // s = z + (float)beta s with beta = rhoNew / rho, and q = A s
         _t->begin(T_SPMV, st);
         if (_refDots > 0) {
-            columnResidual(_cp, _C, nullptr, s, z, st);
-            rowDot(s, z, _pSq, st);
+            if (it > 0) {
+                pcgDirection(z, s, n, _pZr, nb, rho, rhoNew, st);
+                std::swap(s, z);
+                std::swap(rho, rhoNew);
+            }
+            columnResidual(_cp, _C, nullptr, s, q, st);
+            rowDot(s, q, _pSq, st);
+        } else if (it == 0) {
+            columnSpmvDot(_cp, _C, s, q, _pSq, st);
         } else {
-            columnSpmvDot(_cp, _C, s, z, _pSq, st);
+            columnDirectionSpmvDot(_cp, _C, z, s, t, q, _pZr, nb, rho, rhoNew, _pSq, st);
+            std::swap(s, t);
+            std::swap(rho, rhoNew);
         }
         _t->end(T_SPMV, st);
         armResidual();
-        pcgStep(_x, s, _r, z, n, rho, _pSq, nb, _pRmax, st);
+        pcgStep(_x, s, _r, q, n, rho, _pSq, nb, _pRmax, st);
         _t->begin(T_MIC0_APPLY, st, applyLaunches());
         precondForward<double>(_r, _y, _pRmax, st);
         resid = awaitResidual(st);
@@ -610,10 +626,6 @@ bool PressureSolver::pcgFP64(double tolFactor, int maxIter, double resid0, int &
             rowDot(z, _r, _pZr, st);
         else
             dotPartials(z, _r, n, _pZr, st);
-        // beta = rhoNew / rho; z += (float)beta * s; then s <-> z
-        pcgDirection(z, s, n, _pZr, nb, rho, rhoNew, st);
-        std::swap(s, z);
-        std::swap(rho, rhoNew);
     }
     iters = it;
     return false;
@@ -644,14 +656,21 @@ bool PressureSolver::pcgPrecond32(double tolFactor, int maxIter, double resid0, 
     }
     hipCheck(hipMemsetAsync(_s, 0, sizeof(double) * n, st), "memset");
     addFloatToDouble(_s, _fz, n, st);
-    double *s = _s, *z = _z;
+    double *s = _s, *t = _z, *q = _y;
     int it;
     for (it = 0; it < maxIter; it++) {
+        // s = (double)fz + (float)beta s with beta = rhoNew / rho, and q = A s
         _t->begin(T_SPMV, st);
-        columnSpmvDot(_cp, _C, s, z, _pSq, st);
+        if (it == 0) {
+            columnSpmvDot(_cp, _C, s, q, _pSq, st);
+        } else {
+            columnDirectionSpmvDot(_cp, _C, _fz, s, t, q, _pZr, nb, rho, rhoNew, _pSq, st);
+            std::swap(s, t);
+            std::swap(rho, rhoNew);
+        }
         _t->end(T_SPMV, st);
         armResidual();
-        pcgStep(_x, s, _r, z, n, rho, _pSq, nb, _pRmax, st, _fr);
+        pcgStep(_x, s, _r, q, n, rho, _pSq, nb, _pRmax, st, _fr);
         _t->begin(T_MIC0_APPLY, st, applyLaunches());
         precondForward<float>(_fr, _fy, _pRmax, st);
         resid = awaitResidual(st);
@@ -662,13 +681,21 @@ bool PressureSolver::pcgPrecond32(double tolFactor, int maxIter, double resid0, 
         precondBackward<float>(_fy, _fz, st);
         _t->end(T_MIC0_APPLY, st);
         dotfdPartials(_fz, _r, n, _pZr, st);
-        // beta = rhoNew / rho; z = (double)fz + (float)beta * s; then s <-> z
-        pcgDirectionWiden(z, _fz, s, n, _pZr, nb, rho, rhoNew, st);
-        std::swap(s, z);
-        std::swap(rho, rhoNew);
     }
     iters = it;
     return false;
+}
+
+// The FP32 modes' direction s (fz + (float)beta s after the first) and fq = A s.
+void PressureSolver::nextProduct(float *&s, float *&t, bool &first, double *&rho, double *&rhoNew, hipStream_t st) {
+    if (first) {
+        columnSpmvDotF(_cp, _C, s, _fq, _pSq, st);
+        first = false;
+        return;
+    }
+    columnDirectionSpmvDot(_cp, _C, _fz, s, t, _fq, _pZr, reduceBlocks(_cp.slots()), rho, rhoNew, _pSq, st);
+    std::swap(s, t);
+    std::swap(rho, rhoNew);
 }
 
 // FP32 PCG inside FP64 iterative refinement.  The outer loop keeps the FP64
@@ -700,10 +727,11 @@ bool PressureSolver::pcgMixed(double tolFactor, int maxIter, double resid0, doub
         double hrho = hostScalar(rho, st);
         if (hrho == 0 || hrho != hrho) return false;
         hipCheck(hipMemcpyAsync(_fs, _fz, sizeof(float) * n, hipMemcpyDeviceToDevice, st), "copy");
-        float *s = _fs, *z = _fz;
+        float *s = _fs, *t = _ft;
+        bool first = true;
         while (iters < maxIter) {
             _t->begin(T_SPMV, st);
-            columnSpmvDotF(_cp, _C, s, _fq, _pSq, st);
+            nextProduct(s, t, first, rho, rhoNew, st);
             _t->end(T_SPMV, st);
             armResidual();
             pcgStepF(_fd, s, _fr, _fq, n, rho, _pSq, nb, _pRmax, st);
@@ -711,12 +739,9 @@ bool PressureSolver::pcgMixed(double tolFactor, int maxIter, double resid0, doub
             _t->begin(T_MIC0_APPLY, st, applyLaunches());
             precondForward<float>(_fr, _fy, _pRmax, st);
             if (awaitResidual(st) <= innerTol) break;
-            precondBackward<float>(_fy, z, st);
+            precondBackward<float>(_fy, _fz, st);
             _t->end(T_MIC0_APPLY, st);
-            dotfPartials(z, _fr, n, _pZr, st);
-            pcgDirectionF(z, s, n, _pZr, nb, rho, rhoNew, st);
-            std::swap(s, z);
-            std::swap(rho, rhoNew);
+            dotfPartials(_fz, _fr, n, _pZr, st);
         }
         addFloatToDouble(_x, _fd, n, st);
         columnResidual(_cp, _C, _C.rhs, _x, _r, st);
@@ -753,11 +778,12 @@ bool PressureSolver::pcgReliable(double tolFactor, int maxIter, double resid0, d
     double hrho = hostScalar(rho, st);
     if (hrho == 0 || hrho != hrho) return false;
     hipCheck(hipMemcpyAsync(_fs, _fz, sizeof(float) * n, hipMemcpyDeviceToDevice, st), "copy");
-    float *s = _fs, *z = _fz;
+    float *s = _fs, *t = _ft;
+    bool first = true;
     bool trueKnown = true;  // resid holds the true residual of the current x
     while (iters < maxIter) {
         _t->begin(T_SPMV, st);
-        columnSpmvDotF(_cp, _C, s, _fq, _pSq, st);
+        nextProduct(s, t, first, rho, rhoNew, st);
         _t->end(T_SPMV, st);
         armResidual();
         pcgStepMixed(_x, s, _fr, _fq, n, rho, _pSq, nb, _pRmax, st);
@@ -776,12 +802,9 @@ bool PressureSolver::pcgReliable(double tolFactor, int maxIter, double resid0, d
             sinceUpdate = resid;
             precondForward<float>(_fr, _fy, nullptr, st);  // again, from the replaced residual
         }
-        precondBackward<float>(_fy, z, st);
+        precondBackward<float>(_fy, _fz, st);
         _t->end(T_MIC0_APPLY, st);
-        dotfPartials(z, _fr, n, _pZr, st);
-        pcgDirectionF(z, s, n, _pZr, nb, rho, rhoNew, st);
-        std::swap(s, z);
-        std::swap(rho, rhoNew);
+        dotfPartials(_fz, _fr, n, _pZr, st);
     }
     if (!trueKnown) {
         columnResidual(_cp, _C, _C.rhs, _x, _r, st);
