@@ -17,10 +17,11 @@
 #include <thread>
 #include <vector>
 
-#include "ffdevice.h"
-#include "kernels.h"
+#include <hip/hip_runtime_api.h>
 
 namespace ff {
+
+void hipCheck(hipError_t e, const char *what);
 
 class HostCopy {
 public:
@@ -32,10 +33,13 @@ public:
     }
     // out receives `bytes` bytes.  fill(dst, lo, n) enqueues on s what writes
     // bytes [lo, lo + n) of the data to the pinned dst; lo is a multiple of
-    // HALF.  All of them are in out on return.
+    // HALF.  All of them are in out on return.  Several threads may call it at
+    // once (one reads positions, another velocities): they share the pinned
+    // buffer and take turns, as their copies would on the link.
     template <class Fill>
     void run(char *out, size_t bytes, hipStream_t s, Fill fill) {
         if (bytes == 0) return;
+        std::lock_guard<std::mutex> turn(_turn);
         reserve(bytes);
         const int halves = (int)((bytes + HALF - 1) / HALF);
         // a thread's start costs about as much as 256 KB of copying
@@ -143,6 +147,7 @@ private:
         hipCheck(hipHostMalloc((void **)&_pinned, need, hipHostMallocDefault), "read-back buffer");
         _size = need;
     }
+    std::mutex _turn;
     char *_pinned = nullptr;
     size_t _size = 0;
 };

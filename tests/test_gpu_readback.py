@@ -39,3 +39,33 @@ def test_solid_sdf_reads_back_as_set(n3):
     sim.set_solid_phi(phi)
     sim.initialize()
     assert sim.get_solid_sdf().tobytes() == phi.tobytes()
+
+
+def test_read_back_from_two_threads():
+    """Positions in one thread and velocities in another, of one simulation and
+    at once: each gets its own bytes."""
+    import threading
+    n = HALF + 1
+    rng = np.random.default_rng(n)
+    pos = (0.1 + 0.8 * rng.random((n, 3), np.float32)).astype(np.float32)
+    vel = rng.standard_normal((n, 3), np.float32)
+    sim = FluidSimulation(16, 16, 16, 1.0 / 16)
+    for a in range(0, n, 200000):
+        b = min(a + 200000, n)
+        sim.load_marker_particle_data(b - a, pos[a:b].tobytes(), vel[a:b].tobytes())
+    sim.initialize()
+    print("read-back of", n, "by two threads", flush=True)
+    wrong = []
+
+    def read(get, want):
+        for size in (5, 1000, n // 3, n):  # ascending: the pinned buffer grows under way
+            if get(0, size) != want[:size].tobytes():
+                wrong.append((get.__name__, size))
+
+    team = [threading.Thread(target=read, args=a) for a in
+            ((sim.get_marker_particle_position_data_range, pos), (sim.get_marker_particle_velocity_data_range, vel))]
+    for t in team:
+        t.start()
+    for t in team:
+        t.join()
+    assert not wrong
