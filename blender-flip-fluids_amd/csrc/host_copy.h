@@ -40,6 +40,7 @@ public:
     void run(char *out, size_t bytes, hipStream_t s, Fill fill) {
         if (bytes == 0) return;
         std::lock_guard<std::mutex> turn(_turn);
+        const OnDevice on(s);
         reserve(bytes);
         const int halves = (int)((bytes + HALF - 1) / HALF);
         // a thread's start costs about as much as 256 KB of copying
@@ -78,6 +79,29 @@ public:
     static constexpr size_t HALF = (size_t)48 * 350000;
 
 private:
+    // The calling thread is on the stream's device for a while: fill launches a
+    // kernel, and a thread that has chosen no device is on device 0.
+    class OnDevice {
+    public:
+        explicit OnDevice(hipStream_t s) {
+            int device = 0;
+            hipCheck(hipGetDevice(&_before), "hipGetDevice");
+            hipCheck(hipStreamGetDevice(s, &device), "hipStreamGetDevice");
+            if (device == _before) return;
+            hipCheck(hipSetDevice(device), "hipSetDevice");
+            _changed = true;
+        }
+        ~OnDevice() {
+            if (_changed) (void)hipSetDevice(_before);
+        }
+        OnDevice(const OnDevice &) = delete;
+        OnDevice &operator=(const OnDevice &) = delete;
+
+    private:
+        int _before = 0;
+        bool _changed = false;
+    };
+
     // The helper threads of one call.  Half h may be copied once released > h;
     // the destructor ends and joins them whatever happened.
     class Team {

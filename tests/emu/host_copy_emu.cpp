@@ -6,7 +6,8 @@
 // Usage: host_copy_emu <threads>
 // Each thread reads its own arrays back through one HostCopy, of sizes around
 // its halves, ascending (so the pinned buffer is replaced under way), and
-// compares every byte.  Exit status 0: all equal.  Built with a sanitizer.
+// compares every byte; the copies are made on the stream's device, which is not
+// the threads' own.  Exit status 0: all equal.  Built with a sanitizer.
 #include <atomic>
 #include <chrono>
 #include <cstdio>
@@ -25,6 +26,22 @@ void hipCheck(hipError_t e, const char *what) {
 static std::mutex gM;
 static std::vector<std::function<void()>> gQueue;  // the one stream's work
 
+constexpr int STREAM_DEVICE = 3;
+static thread_local int gDevice = 0;
+static std::atomic<int> gElsewhere{0};  // copies asked for on another device
+
+extern "C" hipError_t hipGetDevice(int *d) {
+    *d = gDevice;
+    return hipSuccess;
+}
+extern "C" hipError_t hipSetDevice(int d) {
+    gDevice = d;
+    return hipSuccess;
+}
+extern "C" hipError_t hipStreamGetDevice(hipStream_t, hipDevice_t *d) {
+    *d = STREAM_DEVICE;
+    return hipSuccess;
+}
 extern "C" hipError_t hipHostMalloc(void **p, size_t n, unsigned) {
     *p = std::malloc(n);
     return *p ? hipSuccess : hipErrorOutOfMemory;
@@ -34,6 +51,7 @@ extern "C" hipError_t hipHostFree(void *p) {
     return hipSuccess;
 }
 extern "C" hipError_t hipMemcpyAsync(void *dst, const void *src, size_t n, hipMemcpyKind, hipStream_t) {
+    if (gDevice != STREAM_DEVICE) gElsewhere++;
     std::lock_guard<std::mutex> l(gM);
     gQueue.push_back([=] { std::memcpy(dst, src, n); });
     return hipSuccess;
@@ -60,9 +78,11 @@ int main(int argc, char **argv) {
                 for (size_t q = 0; q < bytes; q++) from[q] = (char)((q * 2654435761u >> 13) + 31 * t);
                 copy.run(to.data() + 1, from.data(), bytes, nullptr);  // an odd address
                 if (to[0] != 'x' || to[bytes + 1] != 'x' || (bytes && std::memcmp(to.data() + 1, from.data(), bytes))) bad++;
+                if (gDevice != 0) bad++;
             }
         });
     for (auto &t : team) t.join();
     if (bad) std::fprintf(stderr, "host_copy_emu: %d read-backs differ\n", (int)bad);
-    return bad ? 1 : 0;
+    if (gElsewhere) std::fprintf(stderr, "host_copy_emu: %d copies on another device\n", (int)gElsewhere);
+    return bad || gElsewhere ? 1 : 0;
 }
