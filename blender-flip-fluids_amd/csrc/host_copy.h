@@ -13,6 +13,7 @@
 #include <condition_variable>
 #include <cstring>
 #include <mutex>
+#include <stdexcept>
 #include <system_error>
 #include <thread>
 #include <vector>
@@ -39,6 +40,7 @@ public:
     template <class Fill>
     void run(char *out, size_t bytes, hipStream_t s, Fill fill) {
         if (bytes == 0) return;
+        if (!out) throw std::domain_error("Error: no buffer to read back into.\n");
         std::lock_guard<std::mutex> turn(_turn);
         const OnDevice on(s);
         reserve(bytes);

@@ -70,6 +70,11 @@ int main(int argc, char **argv) {
     constexpr size_t H = ff::HostCopy::HALF;
     ff::HostCopy copy;
     std::atomic<int> bad{0};
+    try {  // no destination: an error, and nothing written
+        copy.run(nullptr, &copy, 1, nullptr);
+        bad++;
+    } catch (const std::domain_error &) {
+    }
     std::vector<std::thread> team;
     for (int t = 0; t < threads; t++)
         team.emplace_back([&, t] {

@@ -69,3 +69,20 @@ def test_read_back_from_two_threads():
     for t in team:
         t.join()
     assert not wrong
+
+
+def test_a_missing_buffer_is_an_error():
+    """A grid read into no buffer fails with an error, as the copy into it did,
+    and the simulation goes on."""
+    from ctypes import byref, c_int, c_void_p
+    from ffengine.ffengine import ffengine as lib
+    sim = FluidSimulation(16, 16, 16, 1.0 / 16)
+    sim.load_marker_particle_data(1, np.full(3, 0.5, np.float32).tobytes(), np.zeros(3, np.float32).tobytes())
+    sim.initialize()
+    for name in ("pressure_grid", "liquid_sdf", "solid_sdf"):
+        err = c_int(1)
+        f = getattr(lib, "FluidSimulation_get_%s_data" % name)
+        f.argtypes, f.restype = [c_void_p, c_void_p, c_void_p], None
+        f(sim(), None, byref(err))
+        assert err.value == 0, name
+    assert sim.get_pressure_grid().shape == (16, 16, 16)
