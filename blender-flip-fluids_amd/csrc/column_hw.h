@@ -17,10 +17,14 @@
 #define FF_CS_U2F(u) __uint_as_float(u)
 #define FF_CS_D2U(v) ((unsigned long long)__double_as_longlong(v))
 #define FF_CS_U2D(u) __longlong_as_double((long long)(u))
-// LDS accesses that other waves see: in program order, one instruction each
+// LDS accesses that other waves see: one instruction each, volatile, so the
+// compiler keeps their program order
 #define FF_CS_LDS_LOAD(p) ff::ldsLoad(p)
 #define FF_CS_LDS_STORE(p, v) ff::ldsStore((p), (v))
-#define FF_CS_WAVE_ORDER()  // a wave's LDS accesses are performed in order
+#define FF_CS_WAVE_ORDER()  // nothing: the hardware performs a wave's LDS accesses in order
+// what is loaded after it is loaded anew: buffer loads are not volatile (the
+// pipelined ones are to move freely), and a poll without it could be one load
+#define FF_CS_REREAD() asm volatile("" ::: "memory")
 // buffers: accesses outside [0, bytes) load zeros and store nothing
 #define FF_CS_BUFFER ff::ColumnBuffer
 #define FF_CS_MAKE_BUFFER(p, bytes) (ff::ColumnBuffer{(void *)(p), (bytes)})
@@ -49,7 +53,8 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t bufferRsrc(const ColumnBuffer 
     return __builtin_amdgcn_make_buffer_rsrc(b.p, 0, (int)b.bytes, 0x00027000);
 }
 // keeps the offset one register: a bounds check of a base and an immediate
-// would take a negative base out of range
+// would take a negative base out of range.  (It does not make a repeated load
+// of one place a new one: FF_CS_REREAD does.)
 __device__ __forceinline__ int bufferOffset(unsigned off) {
     asm("" : "+v"(off));
     return (int)off;
@@ -102,23 +107,27 @@ __device__ __forceinline__ void bufferStore(const V &v, const ColumnBuffer &b, u
         __builtin_amdgcn_raw_buffer_store_b32(t.d[Q], bufferRsrc(b), bufferOffset(off + 4 * Q), 0, CP);
 }
 
-__device__ __forceinline__ int ldsLoad(int *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); }
-__device__ __forceinline__ float ldsLoad(float *p) {
-    return __uint_as_float(__hip_atomic_load((unsigned *)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
+// (an LDS pointer by type: the compiler leaves a volatile access through a
+// generic one a flat access)
+template <class U>
+using LdsVolatile = volatile __attribute__((address_space(3))) U;
+template <class U>
+__device__ __forceinline__ U ldsLoadBits(void *p) {
+    return __hip_atomic_load((LdsVolatile<U> *)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
+template <class U>
+__device__ __forceinline__ void ldsStoreBits(void *p, U v) {
+    __hip_atomic_store((LdsVolatile<U> *)p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+__device__ __forceinline__ int ldsLoad(int *p) { return ldsLoadBits<int>(p); }
+__device__ __forceinline__ float ldsLoad(float *p) { return __uint_as_float(ldsLoadBits<unsigned>(p)); }
 __device__ __forceinline__ double ldsLoad(double *p) {
-    return __longlong_as_double(
-        (long long)__hip_atomic_load((unsigned long long *)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
+    return __longlong_as_double((long long)ldsLoadBits<unsigned long long>(p));
 }
-__device__ __forceinline__ void ldsStore(int *p, int v) {
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
-__device__ __forceinline__ void ldsStore(float *p, float v) {
-    __hip_atomic_store((unsigned *)p, __float_as_uint(v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
+__device__ __forceinline__ void ldsStore(int *p, int v) { ldsStoreBits<int>(p, v); }
+__device__ __forceinline__ void ldsStore(float *p, float v) { ldsStoreBits<unsigned>(p, __float_as_uint(v)); }
 __device__ __forceinline__ void ldsStore(double *p, double v) {
-    __hip_atomic_store((unsigned long long *)p, (unsigned long long)__double_as_longlong(v), __ATOMIC_RELAXED,
-                       __HIP_MEMORY_SCOPE_WORKGROUP);
+    ldsStoreBits<unsigned long long>(p, (unsigned long long)__double_as_longlong(v));
 }
 
 template <bool FWD>

@@ -52,7 +52,8 @@
 // an LDS plane and a barrier per step took 0.22 us a step against 0.15.
 //
 // This header holds only the sweep's body; its includer supplies the hardware
-// operations as macros (see kernels_column.hip).
+// operations as macros: column_hw.h the GPU's, tests/emu/column_emu.cpp ones
+// that run it on the CPU and grant a ring value no more ordering than asked for.
 #pragma once
 
 #include "column_types.h"
@@ -153,8 +154,10 @@ FF_CS_DEVICE void columnSteps(const ColumnArgs<T, Rec> &a, const ColumnWave<T> &
     auto wait = [&](auto &&ready) {
         const long long start = FF_CS_CLOCK();
         for (;;) {
-            for (int tries = 0; tries < 64; tries++)
+            for (int tries = 0; tries < 64; tries++) {
+                FF_CS_REREAD();
                 if (ready()) return;
+            }
             if (FF_CS_LOAD32(a.error) != 0 || FF_CS_CLOCK() - start > a.waitTicks) {
                 FF_CS_RAISE(a.error);
                 return;
@@ -189,6 +192,7 @@ FF_CS_DEVICE void columnSteps(const ColumnArgs<T, Rec> &a, const ColumnWave<T> &
             if (FF_CS_RARE(made <= x)) {
                 const int want = x + COL_AHEAD < w.lenK ? x + COL_AHEAD : w.lenK;
                 wait([&]() { return (made = FF_CS_UNIFORM(FF_CS_LDS_LOAD(&w.up->made))) >= want; });
+                FF_CS_WAVE_ORDER();  // the entries are read after the count that promised them
             }
             v = FF_CS_LDS_LOAD(&w.up->v[x & (COL_RING - 1)][ringLane]);
         }

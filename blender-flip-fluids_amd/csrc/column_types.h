@@ -1,5 +1,6 @@
 // column_types.h -- plain types of the column layout, shared by the sweep
-// body (column_sweep.h), its host launchers (kernels.h) and CPU builds of it.
+// body (column_sweep.h), its host launchers (kernels.h) and its CPU emulation
+// (tests/emu/column_emu.cpp).
 //
 // A column is 16 x 8 (j, k) lines along i, two lines per lane of a wave: lane
 // j%16 + 16*(k%8/2) holds lines k and k+1.  Its slots are numbered by

@@ -1,0 +1,474 @@
+// column_emu.cpp -- CPU emulation of the column MIC(0) sweeps
+// (blender-flip-fluids_amd/csrc/column_sweep.h), lane by lane.
+//
+// Test infrastructure: it compiles the GPU sweep's own body with g++.  A
+// workgroup is an OS thread and its lanes are fibers of that thread, which meet
+// wherever the kernel moves a value across lanes; the workgroups run at once, so
+// waves do wait for rings and exchange words.  Checked besides the results:
+//   * every buffer the sweep makes lies inside the array it belongs to;
+//   * the ordering the sweep asks for.  Where it states none, a compiler may
+//     move accesses: a value stored to a ring is seen by others from the
+//     writer's next FF_CS_WAVE_ORDER on, and a value loaded from a ring is the
+//     one of the reader's last FF_CS_WAVE_ORDER.
+// The applications run FP64, FP32, FP64 over the same exchange words, so each
+// launch finds the words of the one before.
+//
+// Usage: column_emu <input> <output> <what>
+//   input:  int32 ni, nj, nk, m, then int32 cellRow[N], float64 r[m],
+//           float64 recFwd[m][4], float64 recBwd[m][4]  ({inv, a, b, c})
+//   output: float64 z[m] (FP64), float64 z[m] (FP32)
+//   what:   plain;
+//           pause: while the waves wait, the clock jumps past the limit;
+//           lost: one workgroup is never started and the limit is short (the
+//           launch must end with the error raised; no output)
+#include <algorithm>
+#include <chrono>
+#include <cstdint>
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <memory>
+#include <stdexcept>
+#include <thread>
+#include <unordered_map>
+#include <utility>
+#include <vector>
+
+#include <ucontext.h>
+
+namespace emu {
+
+using Clock = std::chrono::steady_clock;
+enum What { PLAIN, PAUSE, LOST };
+What what = PLAIN;
+Clock::time_point start;  // of the launch
+long long clockNow() {
+    const auto t = Clock::now() - start;
+    long long ns = std::chrono::duration_cast<std::chrono::nanoseconds>(t).count();
+    if (what == PAUSE && t > std::chrono::milliseconds(100)) ns += 100000000000LL;
+    return ns;
+}
+
+constexpr int LANES = 64;
+struct Wave {
+    unsigned phase = 0;
+    int arrived = 0;
+    unsigned long long slot[LANES], seen[LANES];
+};
+struct Fiber {
+    ucontext_t ctx;
+    std::unique_ptr<char[]> stack;
+    bool done = false;
+    unsigned long long order = 0;                             // last FF_CS_WAVE_ORDER
+    std::vector<std::pair<void *, unsigned long long>> made;  // ring values stored since
+};
+struct Group {
+    std::vector<Fiber> fibers;
+    std::vector<Wave> waves;
+    ucontext_t main;
+    int cur = 0, left = 0, barrier = 0;
+    unsigned barrierPhase = 0;
+    // the values each ring place held, by FF_CS_WAVE_ORDER
+    std::unordered_map<void *, std::vector<std::pair<unsigned long long, unsigned long long>>> log;
+    unsigned long long time = 0;
+};
+thread_local Group *g = nullptr;
+
+void yield() {
+    const int from = g->cur;
+    int to = from;
+    do to = (to + 1) % (int)g->fibers.size();
+    while (g->fibers[to].done && to != from);
+    if (to == from) return;
+    g->cur = to;
+    swapcontext(&g->fibers[from].ctx, &g->fibers[to].ctx);
+}
+Fiber &me() { return g->fibers[g->cur]; }
+int lane() { return g->cur % LANES; }
+Wave &wave() { return g->waves[g->cur / LANES]; }
+
+// every lane's value, in seen[] of the wave
+template <class V>
+void meet(V v) {
+    Wave &w = wave();
+    unsigned long long u = 0;
+    std::memcpy(&u, &v, sizeof v);
+    w.slot[lane()] = u;
+    const unsigned phase = w.phase;
+    if (++w.arrived == LANES) {
+        std::memcpy(w.seen, w.slot, sizeof w.seen);
+        w.arrived = 0;
+        w.phase++;
+    } else {
+        while (w.phase == phase) yield();
+    }
+}
+template <class V>
+V from(int l) {
+    V v;
+    std::memcpy(&v, &wave().seen[l], sizeof v);
+    return v;
+}
+template <class V>
+V uniform(V v) {
+    meet(v);
+    return from<V>(0);
+}
+bool any(bool x) {
+    meet((int)x);
+    bool r = false;
+    for (int q = 0; q < LANES; q++) r = r || from<int>(q);
+    return r;
+}
+void barrier() {
+    const unsigned phase = g->barrierPhase;
+    if (++g->barrier == (int)g->fibers.size()) {
+        g->barrier = 0;
+        g->barrierPhase++;
+    } else {
+        while (g->barrierPhase == phase) yield();
+    }
+}
+
+// LDS: counters as they are, ring values as the ordering allows
+int ldsLoad(int *p) {
+    yield();
+    return *p;
+}
+void ldsStore(int *p, int v) { *p = v; }
+template <class V>
+V ldsLoad(V *p) {
+    unsigned long long u = 0;
+    for (const auto &e : g->log[p])
+        if (e.first <= me().order) u = e.second;
+    V v;
+    std::memcpy(&v, &u, sizeof v);
+    return v;
+}
+template <class V>
+void ldsStore(V *p, V v) {
+    unsigned long long u = 0;
+    std::memcpy(&u, &v, sizeof v);
+    me().made.emplace_back(p, u);
+}
+void waveOrder() {
+    meet(0);
+    Fiber &f = me();
+    for (const auto &e : f.made) {
+        auto &l = g->log[e.first];
+        l.emplace_back(g->time + 1, e.second);
+        if (l.size() > 64) l.erase(l.begin());
+    }
+    f.made.clear();
+    f.order = ++g->time;
+    meet(0);
+}
+
+// arrays a buffer may lie in
+std::vector<std::pair<const char *, size_t>> arrays;
+struct Buffer {
+    char *p;
+    unsigned bytes;
+};
+Buffer makeBuffer(const void *p, unsigned bytes) {
+    const char *c = (const char *)p;
+    if (bytes > 0) {
+        bool in = false;
+        for (const auto &a : arrays) in = in || (c >= a.first && c + bytes <= a.first + a.second);
+        if (!in) {
+            std::fprintf(stderr, "column_emu: a buffer outside its array\n");
+            std::abort();
+        }
+    }
+    return Buffer{(char *)p, bytes};
+}
+bool inside(const Buffer &b, unsigned off, unsigned n) { return off < b.bytes && n <= b.bytes - off; }
+template <class V>
+void load(V &v, const Buffer &b, unsigned off) {
+    std::memset((void *)&v, 0, sizeof v);
+    for (unsigned q = 0; q < sizeof v; q += 4)
+        if (inside(b, off + q, 4)) std::memcpy((char *)&v + q, b.p + off + q, 4);
+}
+template <class V>
+void store(const V &v, const Buffer &b, unsigned off) {
+    for (unsigned q = 0; q < sizeof v; q += 4)
+        if (inside(b, off + q, 4)) std::memcpy(b.p + off + q, (const char *)&v + q, 4);
+}
+template <class V>
+void loadWords(V &v, const Buffer &b, unsigned off) {
+    unsigned *w = (unsigned *)&v;
+    for (unsigned q = 0; q < sizeof v / 4; q += 2) {
+        unsigned long long u = 0;
+        if (inside(b, off + 4 * q, 8)) u = __atomic_load_n((unsigned long long *)(b.p + off + 4 * q), __ATOMIC_RELAXED);
+        w[q] = (unsigned)u;
+        w[q + 1] = (unsigned)(u >> 32);
+    }
+}
+template <class V>
+void storeWords(const V &v, const Buffer &b, unsigned off) {
+    const unsigned *w = (const unsigned *)&v;
+    for (unsigned q = 0; q < sizeof v / 4; q += 2)
+        if (inside(b, off + 4 * q, 8))
+            __atomic_store_n((unsigned long long *)(b.p + off + 4 * q), w[q] | ((unsigned long long)w[q + 1] << 32),
+                             __ATOMIC_RELAXED);
+}
+template <bool FWD, class V>
+V rowShift(V v, V ext) {
+    const int l = lane();
+    meet(v);
+    return FWD ? (l % 16 > 0 ? from<V>(l - 1) : ext) : (l % 16 < 15 ? from<V>(l + 1) : ext);
+}
+template <bool FWD, class V>
+V lineShift(V v, V ext) {
+    const int l = lane();
+    meet(v);
+    return FWD ? (l >= 16 ? from<V>(l - 16) : ext) : (l < 48 ? from<V>(l + 16) : ext);
+}
+template <class To, class From>
+To bitCast(From v) {
+    static_assert(sizeof(To) == sizeof(From), "size");
+    To t;
+    std::memcpy(&t, &v, sizeof t);
+    return t;
+}
+
+unsigned firstTicket = 0;  // of the launch
+unsigned ticket(unsigned *p) {
+    const unsigned t = __atomic_fetch_add(p, 1u, __ATOMIC_RELAXED);
+    // the others wait for this one meanwhile
+    if (what == PAUSE && t == firstTicket) std::this_thread::sleep_for(std::chrono::milliseconds(200));
+    return t;
+}
+long long clockMeet() {
+    std::this_thread::yield();
+    return uniform(clockNow());
+}
+
+}  // namespace emu
+
+#define FF_CS_DEVICE inline
+#define FF_CS_SHARED static thread_local
+#define FF_CS_BARRIER() emu::barrier()
+#define FF_CS_LOAD32(p) emu::uniform(__atomic_load_n((p), __ATOMIC_RELAXED))
+#define FF_CS_RAISE(p) __atomic_fetch_or((p), 1, __ATOMIC_RELAXED)
+#define FF_CS_TICKET(p) emu::ticket(p)
+#define FF_CS_CLOCK() emu::clockMeet()
+#define FF_CS_UNIFORM(x) emu::uniform(x)
+#define FF_CS_RARE(x) (x)
+#define FF_CS_ANY(x) emu::any(x)
+#define FF_CS_F2U(v) emu::bitCast<unsigned>(v)
+#define FF_CS_U2F(u) emu::bitCast<float>(u)
+#define FF_CS_D2U(v) emu::bitCast<unsigned long long>(v)
+#define FF_CS_U2D(u) emu::bitCast<double>((unsigned long long)(u))
+#define FF_CS_LDS_LOAD(p) emu::ldsLoad(p)
+#define FF_CS_LDS_STORE(p, v) emu::ldsStore((p), (v))
+#define FF_CS_WAVE_ORDER() emu::waveOrder()
+#define FF_CS_REREAD() emu::yield()
+#define FF_CS_BUFFER emu::Buffer
+#define FF_CS_MAKE_BUFFER(p, n) emu::makeBuffer((p), (n))
+#define FF_CS_LOAD(v, b, off) emu::load((v), (b), (off))
+#define FF_CS_STORE(v, b, off) emu::store((v), (b), (off))
+#define FF_CS_LOAD_WORDS(w, b, off) emu::loadWords((w), (b), (off))
+#define FF_CS_STORE_WORDS(w, b, off) emu::storeWords((w), (b), (off))
+#define FF_CS_ROW_SHIFT(fwd, v, ext) emu::rowShift<fwd>((v), (ext))
+#define FF_CS_LINE_SHIFT(fwd, v, ext) emu::lineShift<fwd>((v), (ext))
+#include "../../blender-flip-fluids_amd/csrc/column_sweep.h"
+
+using namespace ff;
+
+// must match kernels_column.hip
+constexpr int CPF = 6, CPX = 3;
+
+template <class T>
+struct Rec {
+    T inv, a, b, c;
+};
+
+struct System {
+    int ni, nj, nk, m;
+    std::vector<int> cellRow;
+    std::vector<double> r, fwd, bwd;
+};
+// the layout, as columnRanges and columnOrder build it, and what the launches share
+struct Layout {
+    int ncj, nck, ntj, ntk, steps;
+    std::vector<ColumnRange> cols;
+    std::vector<int> slotRow, order;
+    std::vector<unsigned> exJ, exK;
+    unsigned counter = 77, epoch = 0;
+    int error = 0;
+};
+
+static Layout makeLayout(const System &s) {
+    Layout l;
+    auto up = [](int a, int b) { return (a + b - 1) / b; };
+    l.ncj = up(s.nj, COL_J);
+    l.nck = up(s.nk, COL_K);
+    l.ntj = l.ncj;
+    l.ntk = up(l.nck, COL_WAVES);
+    l.steps = s.ni + COL_SKEW;
+    l.cols.assign((size_t)l.ncj * l.nck, ColumnRange{0x3fffffff, -1, 0, 0});
+    auto each = [&](auto &&f) {
+        for (size_t c = 0; c < s.cellRow.size(); c++)
+            if (s.cellRow[c] >= 0) {
+                const int i = (int)(c % s.ni), j = (int)(c / s.ni % s.nj), k = (int)(c / s.ni / s.nj);
+                f(l.cols[j / COL_J + l.ncj * (k / COL_K)], i + j + k, columnPlace(j, k), s.cellRow[c]);
+            }
+    };
+    each([](ColumnRange &r, int h, int, int) {
+        r.lo = std::min(r.lo, h);
+        r.hi = std::max(r.hi, h);
+    });
+    int slices = 0;
+    for (ColumnRange &r : l.cols)
+        if (r.hi >= r.lo) {
+            r.base = COL_SLICE * (slices - r.lo);
+            slices += r.hi - r.lo + 1;
+        }
+    l.slotRow.assign((size_t)COL_SLICE * slices, -1);
+    each([&](ColumnRange &r, int h, int place, int row) { l.slotRow[r.base + COL_SLICE * h + place] = row; });
+    for (int d = 0; d <= l.ntj + l.ntk - 2; d++)
+        for (int pj = 0; pj < l.ntj; pj++)
+            if (d - pj >= 0 && d - pj < l.ntk) l.order.push_back(pj + (d - pj) * l.ntj);
+    // four 32-bit parts: a double's two words
+    l.exJ.assign((size_t)l.ncj * l.ntk * COL_WAVES * l.steps * COL_K * 4, 0);
+    l.exK.assign((size_t)l.ntj * l.ntk * l.steps * COL_J * 4, 0);
+    return l;
+}
+
+template <class F>
+static void workgroup(F body) {
+    constexpr int NT = COL_LANES * COL_WAVES;
+    emu::Group g;
+    emu::g = &g;
+    g.fibers.resize(NT);
+    g.waves.resize(COL_WAVES);
+    g.left = NT;
+    struct Start {
+        F *body;
+        static void run(unsigned lo, unsigned hi) {
+            (*((Start *)(((uintptr_t)hi << 32) | lo))->body)(emu::g->cur);
+            emu::me().done = true;
+            if (--emu::g->left == 0) setcontext(&emu::g->main);
+            emu::yield();
+        }
+    } s{&body};
+    for (emu::Fiber &f : g.fibers) {
+        constexpr size_t STACK = 128 << 10;
+        f.stack.reset(new char[STACK]);
+        getcontext(&f.ctx);
+        f.ctx.uc_stack.ss_sp = f.stack.get();
+        f.ctx.uc_stack.ss_size = STACK;
+        f.ctx.uc_link = nullptr;
+        const uintptr_t p = (uintptr_t)&s;
+        makecontext(&f.ctx, (void (*)())Start::run, 2, (unsigned)p, (unsigned)(p >> 32));
+    }
+    swapcontext(&g.main, &g.fibers[0].ctx);
+    emu::g = nullptr;
+}
+
+template <class T, bool FWD>
+static void sweep(Layout &l, const std::vector<T> &in, std::vector<T> &out, const std::vector<Rec<T>> &rec) {
+    const int tiles = l.ntj * l.ntk;
+    ColumnArgs<T, Rec<T>> a{};
+    a.ncj = l.ncj;
+    a.nck = l.nck;
+    a.ntj = l.ntj;
+    a.ntk = l.ntk;
+    a.cols = l.cols.data();
+    a.order = l.order.data();
+    a.in = in.data();
+    a.out = out.data();
+    a.rec = rec.data();
+    a.exJ = l.exJ.data();
+    a.exK = l.exK.data();
+    a.exSteps = l.steps;
+    a.counter = &l.counter;
+    a.error = &l.error;
+    a.base = l.counter;
+    a.epoch = ++l.epoch;
+    a.waitTicks = emu::what == emu::LOST ? 50000000LL : 20000000000LL;
+    emu::arrays = {{(const char *)in.data(), in.size() * sizeof(T)},
+                   {(const char *)out.data(), out.size() * sizeof(T)},
+                   {(const char *)rec.data(), rec.size() * sizeof(Rec<T>)},
+                   {(const char *)l.exJ.data(), l.exJ.size() * 4},
+                   {(const char *)l.exK.data(), l.exK.size() * 4}};
+    emu::start = emu::Clock::now();
+    emu::firstTicket = l.counter;
+    if (emu::what == emu::LOST) l.counter++;  // the first tile's ticket is gone
+    std::vector<std::thread> groups;
+    for (int w = emu::what == emu::LOST ? 1 : 0; w < tiles; w++)
+        groups.emplace_back([&a] { workgroup([&a](int tid) { columnSweep<T, Rec<T>, CPF, CPX, FWD>(a, tid); }); });
+    for (auto &t : groups) t.join();
+    if (l.counter != a.base + (unsigned)tiles) throw std::runtime_error("ticket count");
+}
+
+template <class T>
+static std::vector<T> apply(const System &s, Layout &l) {
+    const size_t e = l.slotRow.size();
+    std::vector<T> in(e, T(0)), y(e, T(0)), z(e, T(0));
+    std::vector<Rec<T>> rf(e, Rec<T>{}), rb(e, Rec<T>{});
+    for (size_t q = 0; q < e; q++)
+        if (l.slotRow[q] >= 0) {
+            const size_t r = l.slotRow[q];
+            in[q] = (T)s.r[r];
+            rf[q] = Rec<T>{(T)s.fwd[4 * r], (T)s.fwd[4 * r + 1], (T)s.fwd[4 * r + 2], (T)s.fwd[4 * r + 3]};
+            rb[q] = Rec<T>{(T)s.bwd[4 * r], (T)s.bwd[4 * r + 1], (T)s.bwd[4 * r + 2], (T)s.bwd[4 * r + 3]};
+        }
+    sweep<T, true>(l, in, y, rf);
+    sweep<T, false>(l, y, z, rb);
+    std::vector<T> rows(s.m);
+    for (size_t q = 0; q < e; q++) {
+        if (l.slotRow[q] >= 0)
+            rows[l.slotRow[q]] = z[q];
+        else if (y[q] != T(0) || z[q] != T(0))
+            throw std::runtime_error("a slot without a row is not zero");
+    }
+    return rows;
+}
+
+int main(int argc, char **argv) {
+    if (argc != 4) {
+        std::fprintf(stderr, "usage: column_emu <input> <output> <plain|pause|lost>\n");
+        return 2;
+    }
+    emu::what = !std::strcmp(argv[3], "pause") ? emu::PAUSE : !std::strcmp(argv[3], "lost") ? emu::LOST : emu::PLAIN;
+    FILE *f = std::fopen(argv[1], "rb");
+    if (!f) return 2;
+    int hdr[4];
+    if (std::fread(hdr, sizeof(int), 4, f) != 4) return 2;
+    System s{hdr[0], hdr[1], hdr[2], hdr[3], {}, {}, {}, {}};
+    const size_t n = (size_t)s.ni * s.nj * s.nk, m = s.m;
+    s.cellRow.resize(n);
+    s.r.resize(m);
+    s.fwd.resize(4 * m);
+    s.bwd.resize(4 * m);
+    const bool ok = std::fread(s.cellRow.data(), sizeof(int), n, f) == n &&
+                    std::fread(s.r.data(), sizeof(double), m, f) == m &&
+                    std::fread(s.fwd.data(), sizeof(double), 4 * m, f) == 4 * m &&
+                    std::fread(s.bwd.data(), sizeof(double), 4 * m, f) == 4 * m;
+    std::fclose(f);
+    if (!ok) return 2;
+    try {
+        Layout l = makeLayout(s);
+        const std::vector<double> z = apply<double>(s, l);
+        if (emu::what == emu::LOST) return l.error ? 0 : 1;
+        const std::vector<float> zf = apply<float>(s, l);
+        const std::vector<double> again = apply<double>(s, l);
+        if (l.error) throw std::runtime_error("a wait ran out");
+        if (m && std::memcmp(z.data(), again.data(), m * sizeof(double)))
+            throw std::runtime_error("a second application differs");
+        f = std::fopen(argv[2], "wb");
+        if (!f) return 2;
+        std::fwrite(z.data(), sizeof(double), m, f);
+        for (float v : zf) {
+            const double d = v;
+            std::fwrite(&d, sizeof d, 1, f);
+        }
+        std::fclose(f);
+    } catch (const std::exception &e) {
+        std::fprintf(stderr, "column_emu: %s\n", e.what());
+        return 1;
+    }
+    return 0;
+}
