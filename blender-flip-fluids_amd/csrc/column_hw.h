@@ -9,7 +9,6 @@
 #define FF_CS_LOAD32(p) __hip_atomic_load((p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
 #define FF_CS_RAISE(p) __hip_atomic_fetch_or((p), 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
 #define FF_CS_TICKET(p) atomicAdd((p), 1u)
-#define FF_CS_CLOCK() ((long long)wall_clock64())
 #define FF_CS_UNIFORM(x) __builtin_amdgcn_readfirstlane(x)
 #define FF_CS_RARE(x) __builtin_expect(!!(x), 0)
 #define FF_CS_ANY(x) (__ballot(x) != 0)

@@ -32,8 +32,9 @@
 // workgroups took their tickets earlier and are running or done, and a wave
 // waits for the next wave of its tile only while that one holds unread ring
 // entries, so the launch drains for any number of resident workgroups.  Every
-// wait is bounded in wall-clock time: past the limit the wave raises the error
-// word (which every other waiting wave also gives up on) and the launch still
+// wait is bounded, in looks and not by a clock, which would go on while the
+// device runs another process: past the limit the wave raises the error word
+// (which every other waiting wave also gives up on) and the launch still
 // finishes; the host turns the word into an error.
 //
 // Arithmetic.  Every slot performs the reference's operations in its order
@@ -74,10 +75,10 @@ struct ColumnArgs {
     unsigned *exJ, *exK;      // words: column x step x COL_K lines; tile x step x COL_J lines
     int exSteps;              // steps of a column's words (the hyperplanes it can span)
     unsigned *counter;        // ticket counter
-    int *error;               // raised when a wait exceeded waitTicks
+    int *error;               // raised when a wait exceeded waitLooks
     unsigned base;            // counter value when this launch started
     unsigned epoch;           // tag of this launch's published words (never 0)
-    long long waitTicks;      // longest wait, FF_CS_CLOCK() ticks
+    int waitLooks;            // longest wait, looks at what is waited for
 };
 
 // a value's words as four (double) or two (float) 32-bit parts
@@ -149,16 +150,14 @@ FF_CS_DEVICE void columnSteps(const ColumnArgs<T, Rec> &a, const ColumnWave<T> &
     constexpr unsigned JSTEP = COL_K * N * 4, KSTEP = COL_J * N * 4;
     // the backward sweep starts at the last slice
     auto slice = [&](int u) { return (unsigned)(FWD ? u : n - 1 - u); };
-    // looks at the clock and the error word only now and then: both take as
-    // long as a look at what it waits for
+    // looks at the error word only now and then: that takes as long as a look at
+    // what it waits for
     auto wait = [&](auto &&ready) {
-        const long long start = FF_CS_CLOCK();
-        for (;;) {
-            for (int tries = 0; tries < 64; tries++) {
-                FF_CS_REREAD();
-                if (ready()) return;
-            }
-            if (FF_CS_LOAD32(a.error) != 0 || FF_CS_CLOCK() - start > a.waitTicks) {
+#pragma unroll 1
+        for (int looks = 0;; looks++) {
+            FF_CS_REREAD();
+            if (ready()) return;
+            if ((looks & 63) == 63 && (FF_CS_LOAD32(a.error) != 0 || looks >= a.waitLooks)) {
                 FF_CS_RAISE(a.error);
                 return;
             }

@@ -497,9 +497,8 @@ struct ColumnPlan {
     int *slotRow = nullptr;                  // COL_SLICE maxSlices: row of each slot or -1
     unsigned *exJ = nullptr, *exK = nullptr; // exchange words, cleared once
     unsigned *counter = nullptr;             // ticket counter, cleared once
-    int *error = nullptr;                    // raised by a wait past waitTicks
+    int *error = nullptr;                    // raised by a wait past its limit
     unsigned base = 0, epoch = 0;            // counter value and last epoch used
-    long long waitTicks = 0;                 // longest wait in wall-clock ticks
     size_t slots() const { return (size_t)slices * COL_SLICE; }
 };
 // matrix, right-hand side and MIC(0) records in slots (zeros where no row is)

@@ -25,6 +25,9 @@ namespace {
 // 96 x 160 x 256, FP32 / FP64: 6 and 3 151 / 205 us, 6 and 4 - / 210, 8 and 3 151,
 // 8 and 4 155 / 213, 8 and 6 164.
 constexpr int CPF = 6, CPX = 3;
+// A wait's limit.  A look at a ring takes about 0.1 us, one at a word 0.7 us: 2 s
+// and 14 s, where a whole sweep takes 1 ms.
+constexpr int WAIT_LOOKS = 20000000;
 constexpr int EMPTY_LO = 0x3fffffff;
 
 int ceilDiv(int a, int b) { return (a + b - 1) / b; }
@@ -313,7 +316,7 @@ void columnSweepLaunch(ColumnPlan &cp, const T *in, T *out, const MicRec<T> *rec
     const unsigned tiles = (unsigned)cp.ntj * cp.ntk;
     if (++cp.epoch == 0) cp.epoch = 1;  // 0 tags the cleared buffer
     ColumnArgs<T, MicRec<T>> a{cp.ncj, cp.nck,     cp.ntj,     cp.ntk,   cp.cols,  cp.order, in,           out,         rec,
-                               cp.exJ, cp.exK,     cp.exSteps, cp.counter, cp.error, cp.base,  cp.epoch,     cp.waitTicks};
+                               cp.exJ, cp.exK,     cp.exSteps, cp.counter, cp.error, cp.base,  cp.epoch,     WAIT_LOOKS};
     cp.base += tiles;
     // the publishing workgroup takes no ticket
     hipLaunchKernelGGL((columnSweepKernel<T, FWD>), dim3(tiles + (pub.rmax ? 1 : 0)), dim3(COL_LANES * COL_WAVES), 0, st,

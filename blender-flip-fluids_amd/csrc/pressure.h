@@ -103,6 +103,7 @@ private:
     KernelTimers _noTimers;
     int _levelLaunches = 0, _bandLaunches = 0;
     PencilPlan _pp;  // line-pipeline buffers (inside _rowBlock)
+    long long _waitTicks = 0;  // the row-ordered schedules' longest wait, wall-clock ticks
     int _sched = 2;
     // z = M^-1 r with the solver's schedule (y: forward result), whole or in
     // its two halves

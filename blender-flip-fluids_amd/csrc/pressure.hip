@@ -132,7 +132,7 @@ void PressureSolver::allocate(Grid g) {
     int dev = 0, wallKHz = 0;
     hipCheck(hipGetDevice(&dev), "hipGetDevice");
     hipCheck(hipDeviceGetAttribute(&wallKHz, hipDeviceAttributeWallClockRate, dev), "device attribute");
-    _cp.waitTicks = 2000LL * std::max(wallKHz, 1);  // 2 s
+    _waitTicks = 2000LL * std::max(wallKHz, 1);  // 2 s
 }
 
 size_t PressureSolver::maxRows() const {
@@ -185,7 +185,7 @@ void PressureSolver::ensureRowSchedules() {
     _ms.counter = (int *)(m + oCounter);
     _ms.error = _cp.error;
     _ms.grid = std::max(cus, 1);
-    _ms.waitTicks = _cp.waitTicks;
+    _ms.waitTicks = _waitTicks;
     _S.levelFill = (int *)(m + oLf);
     _S.levelRows = (int *)(m + oLr);
     double *d[6];
@@ -206,7 +206,7 @@ void PressureSolver::ensureRowSchedules() {
     _pp.ex = (unsigned long long *)(m + oPEx);
     _pp.counter = (unsigned *)(m + oPCounter);
     _pp.error = _cp.error;
-    _pp.waitTicks = _cp.waitTicks;
+    _pp.waitTicks = _waitTicks;
     _pp.base = _pp.epoch = 0;
     hipCheck(hipMemset(_pp.ex, 0, 8 * exWords), "clear exchange words");
     hipCheck(hipMemset(_pp.counter, 0, 4), "clear ticket counter");
@@ -259,7 +259,7 @@ void PressureSolver::checkError(hipStream_t s) {
     int e = 0;
     hipCheck(hipMemcpyAsync(&e, _cp.error, sizeof(int), hipMemcpyDeviceToHost, s), "D2H error word");
     hipCheck(hipStreamSynchronize(s), "sync");
-    if (e) throw std::runtime_error("MIC(0) preconditioner: a wait for a neighbour's results exceeded its time limit");
+    if (e) throw std::runtime_error("MIC(0) preconditioner: a wait for a neighbour's results exceeded its limit");
 }
 
 void PressureSolver::setSchedule(int schedule) {

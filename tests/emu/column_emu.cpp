@@ -10,6 +10,8 @@
 //     move accesses: a value stored to a ring is seen by others from the
 //     writer's next FF_CS_WAVE_ORDER on, and a value loaded from a ring is the
 //     one of the reader's last FF_CS_WAVE_ORDER.
+// There is no clock here: a wait that goes by one, which counts the time another
+// process has the device, does not build.
 // The applications run FP64, FP32, FP64 over the same exchange words, so each
 // launch finds the words of the one before.
 //
@@ -17,12 +19,9 @@
 //   input:  int32 ni, nj, nk, m, then int32 cellRow[N], float64 r[m],
 //           float64 recFwd[m][4], float64 recBwd[m][4]  ({inv, a, b, c})
 //   output: float64 z[m] (FP64), float64 z[m] (FP32)
-//   what:   plain;
-//           pause: while the waves wait, the clock jumps past the limit;
-//           lost: one workgroup is never started and the limit is short (the
-//           launch must end with the error raised; no output)
+//   what:   plain, or lost: one workgroup is never started and the limit is short
+//           (the launch must end with the error raised; no output)
 #include <algorithm>
-#include <chrono>
 #include <cstdint>
 #include <cstdio>
 #include <cstdlib>
@@ -38,16 +37,8 @@
 
 namespace emu {
 
-using Clock = std::chrono::steady_clock;
-enum What { PLAIN, PAUSE, LOST };
+enum What { PLAIN, LOST };
 What what = PLAIN;
-Clock::time_point start;  // of the launch
-long long clockNow() {
-    const auto t = Clock::now() - start;
-    long long ns = std::chrono::duration_cast<std::chrono::nanoseconds>(t).count();
-    if (what == PAUSE && t > std::chrono::milliseconds(100)) ns += 100000000000LL;
-    return ns;
-}
 
 constexpr int LANES = 64;
 struct Wave {
@@ -232,16 +223,10 @@ To bitCast(From v) {
     return t;
 }
 
-unsigned firstTicket = 0;  // of the launch
-unsigned ticket(unsigned *p) {
-    const unsigned t = __atomic_fetch_add(p, 1u, __ATOMIC_RELAXED);
-    // the others wait for this one meanwhile
-    if (what == PAUSE && t == firstTicket) std::this_thread::sleep_for(std::chrono::milliseconds(200));
-    return t;
-}
-long long clockMeet() {
+// looked at between the looks of a wait
+int errorWord(const int *p) {
     std::this_thread::yield();
-    return uniform(clockNow());
+    return uniform(__atomic_load_n(p, __ATOMIC_RELAXED));
 }
 
 }  // namespace emu
@@ -249,10 +234,9 @@ long long clockMeet() {
 #define FF_CS_DEVICE inline
 #define FF_CS_SHARED static thread_local
 #define FF_CS_BARRIER() emu::barrier()
-#define FF_CS_LOAD32(p) emu::uniform(__atomic_load_n((p), __ATOMIC_RELAXED))
+#define FF_CS_LOAD32(p) emu::errorWord(p)
 #define FF_CS_RAISE(p) __atomic_fetch_or((p), 1, __ATOMIC_RELAXED)
-#define FF_CS_TICKET(p) emu::ticket(p)
-#define FF_CS_CLOCK() emu::clockMeet()
+#define FF_CS_TICKET(p) __atomic_fetch_add((p), 1u, __ATOMIC_RELAXED)
 #define FF_CS_UNIFORM(x) emu::uniform(x)
 #define FF_CS_RARE(x) (x)
 #define FF_CS_ANY(x) emu::any(x)
@@ -387,14 +371,12 @@ static void sweep(Layout &l, const std::vector<T> &in, std::vector<T> &out, cons
     a.error = &l.error;
     a.base = l.counter;
     a.epoch = ++l.epoch;
-    a.waitTicks = emu::what == emu::LOST ? 50000000LL : 20000000000LL;
+    a.waitLooks = emu::what == emu::LOST ? 100 : 1 << 30;
     emu::arrays = {{(const char *)in.data(), in.size() * sizeof(T)},
                    {(const char *)out.data(), out.size() * sizeof(T)},
                    {(const char *)rec.data(), rec.size() * sizeof(Rec<T>)},
                    {(const char *)l.exJ.data(), l.exJ.size() * 4},
                    {(const char *)l.exK.data(), l.exK.size() * 4}};
-    emu::start = emu::Clock::now();
-    emu::firstTicket = l.counter;
     if (emu::what == emu::LOST) l.counter++;  // the first tile's ticket is gone
     std::vector<std::thread> groups;
     for (int w = emu::what == emu::LOST ? 1 : 0; w < tiles; w++)
@@ -429,10 +411,10 @@ static std::vector<T> apply(const System &s, Layout &l) {
 
 int main(int argc, char **argv) {
     if (argc != 4) {
-        std::fprintf(stderr, "usage: column_emu <input> <output> <plain|pause|lost>\n");
+        std::fprintf(stderr, "usage: column_emu <input> <output> <plain|lost>\n");
         return 2;
     }
-    emu::what = !std::strcmp(argv[3], "pause") ? emu::PAUSE : !std::strcmp(argv[3], "lost") ? emu::LOST : emu::PLAIN;
+    emu::what = !std::strcmp(argv[3], "lost") ? emu::LOST : emu::PLAIN;
     FILE *f = std::fopen(argv[1], "rb");
     if (!f) return 2;
     int hdr[4];

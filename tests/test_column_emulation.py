@@ -73,3 +73,11 @@ def _check(emulator, tmp_path, n3, kind, what):
     for kind in ("full", "scattered", "islands", "layer")])
 def test_column_sweeps_emulated_bitexact(emulator, tmp_path, n3, kind):
     _check(emulator, tmp_path, n3, kind, "plain")
+
+
+def test_a_lost_workgroup_ends_the_launch(emulator, tmp_path):
+    """A wait for a workgroup that never runs ends at the limit: the launch
+    finishes with the error raised."""
+    n3 = (9, 40, 33)
+    sysm, r = _system("full", n3)
+    _run(emulator, tmp_path, n3, sysm, r, "lost")
