@@ -3,6 +3,8 @@
 // Every entry point converts exceptions into *err = 0 plus one process-wide
 // message buffer, like the reference's safe_execute_* wrappers
 // (c_bindings/cbindings.h:48-155, cbindings.cpp:35-43).
+#include <algorithm>
+#include <cmath>
 #include <cstring>
 #include <exception>
 #include <memory>
@@ -1298,18 +1300,25 @@ int FFAMD_mic0_apply(int ni, int nj, int nk, double dx, double dt, const float *
                                     std::to_string(m) + " rows");
         DBuf<double> dr(m), dz(m);
         up(dr.p, r, m, sc.s);
-        if (precision == 0) {
-            ps.applyPreconditioner(dr, dz, schedule, sc.s);
-        } else {
-            DBuf<float> fr(m), fz(m);
-            ff::castToFloat(dr, fr, m, sc.s);
-            ps.applyPreconditionerF(fr, fz, schedule, sc.s);
-            ff::hipCheck(hipMemsetAsync(dz, 0, sizeof(double) * m, sc.s), "memset");
-            ff::addFloatToDouble(dz, fz, m, sc.s);
+        const auto apply = [&](int how) {
+            if (precision == 0) {
+                ps.applyPreconditioner(dr, dz, how, sc.s);
+            } else {
+                DBuf<float> fr(m), fz(m);
+                ff::castToFloat(dr, fr, m, sc.s);
+                ps.applyPreconditionerF(fr, fz, how, sc.s);
+                ff::hipCheck(hipMemsetAsync(dz, 0, sizeof(double) * m, sc.s), "memset");
+                ff::addFloatToDouble(dz, fz, m, sc.s);
+                sync(sc.s);
+            }
+            down(z, dz.p, m, sc.s);
             sync(sc.s);
-        }
-        down(z, dz.p, m, sc.s);
-        sync(sc.s);
+        };
+        apply(schedule);
+        // The columns' result is exact where all values are finite.  An infinity
+        // or a NaN on the way reaches z, and rows that do not depend on it: the
+        // bands, which leave missing neighbours out, answer such a call.
+        if (schedule == 2 && !std::all_of(z, z + m, [](double v) { return std::isfinite(v); })) apply(5);
         ps.checkError(sc.s);
         return (int)m;
     });

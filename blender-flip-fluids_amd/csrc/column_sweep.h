@@ -41,7 +41,8 @@
 // (forward: subtract the -z, -y, -x terms, then scale by invdiag; backward:
 // +x, +y, +z).  A missing neighbour's coefficient and value are zero, so its
 // term subtracts +0 and leaves every bit.  (Values must be finite: an infinity
-// times a missing coefficient is NaN.  PCG's dot products spread either.)
+// times a missing coefficient is NaN.  PCG's dot products spread either;
+// FFAMD_mic0_apply answers such a call in bands.)
 //
 // Measured, one application (both sweeps) FP64 / FP32, against launches over
 // bands of 8 / 12 hyperplanes: 24^3 99 / 86 -> 42 / 35 us, 64^3 237 / 201 ->

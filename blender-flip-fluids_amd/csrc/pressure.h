@@ -69,7 +69,9 @@ public:
     // schedule 0 = one launch per hyperplane, 1 = tile wavefront (switched
     // off: raises an error), 2 = columns (the solver's), 3 = bands of
     // hyperplanes with the tile ranges checked on the device, 4 = the line
-    // pipeline.
+    // pipeline, 5 = bands of the tiles the host lists.  0, 3 and 5 leave the term
+    // of a missing neighbour out; 2 and 4 subtract 0 times it, the same for finite
+    // values only.
     void applyPreconditioner(const double *r, double *z, int schedule, hipStream_t s);
     void applyPreconditionerF(const float *r, float *z, int schedule, hipStream_t s);
     // throws when a preconditioner launch gave up waiting (waits for the stream)

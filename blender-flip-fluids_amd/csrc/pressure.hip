@@ -395,7 +395,7 @@ void PressureSolver::applyPreconditioner(const double *r, double *z, int schedul
     } else if (schedule == 1) {
         buildSchedule(true, s);
         micApplyTiles(_S, _ms, r, z, s);
-    } else if (schedule == 3) {
+    } else if (schedule == 3 || schedule == 5) {
         mic0ApplyBands(_g, _S, _plan, _tileLo, _tileHi, r, _rowY, z, s);
     } else {
         mic0Apply(_S, _hLevelStart.data(), r, z, s);
@@ -416,7 +416,7 @@ void PressureSolver::applyPreconditionerF(const float *r, float *z, int schedule
     } else if (schedule == 1) {
         buildSchedule(false, s);
         micApplyTilesF(_S, _ms, r, z, s);
-    } else if (schedule == 3) {
+    } else if (schedule == 3 || schedule == 5) {
         mic0ApplyBandsF(_g, _S, _plan, _tileLo, _tileHi, r, _rowFY, z, s);
     } else {
         mic0ApplyF(_S, _hLevelStart.data(), r, z, s);

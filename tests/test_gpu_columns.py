@@ -48,3 +48,41 @@ def test_column_sweeps_bitexact(n3, kind):
     f = K.mic0_apply(n3, dx, dt, uvw, weights, phi, r, precision=1, schedule=2)
     # the call adds the widened FP32 result to zeros: -0 comes back as +0
     assert same_bits(f.astype(np.float32), _mic_sweeps(sysm, n3, r, np.float32) + np.float32(0))
+
+
+@pytest.mark.parametrize("schedule", [2, 3, 0], ids=["columns", "bands-device-check", "hyperplanes"])
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan, 1e300])
+@pytest.mark.parametrize("n3", [(9, 16, 33), (31, 15, 47), (40, 40, 70)])
+def test_non_finite_values_stay_in_their_body(n3, value, schedule):
+    """A value that is, or in the sweeps or as a float becomes, infinite or NaN
+    changes the rows that depend on it and no others: the other of two bodies of
+    liquid, a cell apart along the lines they share, keeps its bits, and in its
+    own body it goes where the serial sweeps take it."""
+    ni, nj, nk = n3
+    rng = np.random.default_rng(sum(n3))
+    k, j, i = np.meshgrid(np.arange(nk), np.arange(nj), np.arange(ni), indexing="ij")
+    phi = np.where(i != ni // 2, np.float32(-0.4), np.float32(0.3)).astype(np.float32) / max(n3)
+    weights = O.face_weights(n3, O.solid_box_phi(n3, 1.0 / max(n3)))
+    uvw = [rng.standard_normal(s).astype(np.float32) for s in ((nk, nj, ni + 1), (nk, nj + 1, ni), (nk + 1, nj, ni))]
+    args = n3, 1.0 / max(n3), 1.0 / 120.0, uvw, weights, phi
+    sysm = O.pressure_system(*args)
+    m = len(sysm["rows"])
+
+    def agree(got, want):
+        finite = np.isfinite(want)
+        assert np.array_equal(np.isfinite(got), finite)
+        assert np.array_equal(got, want, equal_nan=True)
+        assert same_bits(got[finite], want[finite])
+
+    for at in (0, m - 1):  # in the one body, ahead of the other in the forward sweep, and in the other one
+        r = rng.standard_normal(m)
+        r[at] = value
+        say(f"row {at} of {m} is {value}, {n3} schedule {schedule}")
+        want = O.apply_mic0(sysm, r)
+        assert np.isfinite(want).sum() >= m // 3
+        agree(K.mic0_apply(*args, r, precision=0, schedule=schedule), want)
+        with np.errstate(all="ignore"):
+            want = _mic_sweeps(sysm, n3, r, np.float32) + np.float32(0)
+            got = K.mic0_apply(*args, r, precision=1, schedule=schedule).astype(np.float32)
+        assert m // 3 <= np.isfinite(want).sum() < m
+        agree(got, want)
