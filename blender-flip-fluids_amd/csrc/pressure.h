@@ -115,7 +115,12 @@ private:
     void precondForward(const T *r, T *y, const double *rmax, hipStream_t s);
     template <class T>
     void precondBackward(const T *y, T *z, hipStream_t s);
-    int applyLaunches() const { return _sched == 5 ? _bandLaunches : 2; }
+    // launches of its halves: the row-ordered schedules convert before and after,
+    // and publish in a launch of its own
+    int forwardLaunches(bool publish) const { return _sched == 2 ? 1 : publish ? 2 : 1; }
+    int applyLaunches(bool publish) const {
+        return forwardLaunches(publish) + (_sched == 2 ? 1 : (_sched == 5 ? _bandLaunches : 2) + 1);
+    }
     size_t maxRows() const;
     void ensureRowSchedules();
     void prepareRowSchedule(int schedule, bool fp64, hipStream_t s);

@@ -374,7 +374,7 @@ void PressureSolver::precondBackward(const T *y, T *z, hipStream_t s) {
 }
 template <class T>
 void PressureSolver::precond(const T *r, T *y, T *z, hipStream_t s) {
-    _t->begin(T_MIC0_APPLY, s, applyLaunches());
+    _t->begin(T_MIC0_APPLY, s, applyLaunches(false));
     precondForward<T>(r, y, nullptr, s);
     precondBackward<T>(y, z, s);
     _t->end(T_MIC0_APPLY, s);
@@ -613,10 +613,11 @@ bool PressureSolver::pcgFP64(double tolFactor, int maxIter, double resid0, int &
         _t->end(T_SPMV, st);
         armResidual();
         pcgStep(_x, s, _r, q, n, rho, _pSq, nb, _pRmax, st);
-        _t->begin(T_MIC0_APPLY, st, applyLaunches());
+        _t->begin(T_MIC0_APPLY, st, applyLaunches(true));
         precondForward<double>(_r, _y, _pRmax, st);
         resid = awaitResidual(st);
         if (resid <= std::min(tol, 1.0)) {
+            _t->end(T_MIC0_APPLY, st, forwardLaunches(true));
             iters = it + 1;
             return true;
         }
@@ -671,10 +672,11 @@ bool PressureSolver::pcgPrecond32(double tolFactor, int maxIter, double resid0, 
         _t->end(T_SPMV, st);
         armResidual();
         pcgStep(_x, s, _r, q, n, rho, _pSq, nb, _pRmax, st, _fr);
-        _t->begin(T_MIC0_APPLY, st, applyLaunches());
+        _t->begin(T_MIC0_APPLY, st, applyLaunches(true));
         precondForward<float>(_fr, _fy, _pRmax, st);
         resid = awaitResidual(st);
         if (resid <= std::min(tol, 1.0)) {
+            _t->end(T_MIC0_APPLY, st, forwardLaunches(true));
             iters = it + 1;
             return true;
         }
@@ -736,9 +738,12 @@ bool PressureSolver::pcgMixed(double tolFactor, int maxIter, double resid0, doub
             armResidual();
             pcgStepF(_fd, s, _fr, _fq, n, rho, _pSq, nb, _pRmax, st);
             iters++;
-            _t->begin(T_MIC0_APPLY, st, applyLaunches());
+            _t->begin(T_MIC0_APPLY, st, applyLaunches(true));
             precondForward<float>(_fr, _fy, _pRmax, st);
-            if (awaitResidual(st) <= innerTol) break;
+            if (awaitResidual(st) <= innerTol) {
+                _t->end(T_MIC0_APPLY, st, forwardLaunches(true));
+                break;
+            }
             precondBackward<float>(_fy, _fz, st);
             _t->end(T_MIC0_APPLY, st);
             dotfPartials(_fz, _fr, n, _pZr, st);
@@ -789,10 +794,11 @@ bool PressureSolver::pcgReliable(double tolFactor, int maxIter, double resid0, d
         pcgStepMixed(_x, s, _fr, _fq, n, rho, _pSq, nb, _pRmax, st);
         iters++;
         trueKnown = false;
-        _t->begin(T_MIC0_APPLY, st, applyLaunches());
+        _t->begin(T_MIC0_APPLY, st, applyLaunches(true));
         precondForward<float>(_fr, _fy, _pRmax, st);
         const double rf = awaitResidual(st);
         if (rf <= delta * sinceUpdate || rf <= tol) {
+            _t->end(T_MIC0_APPLY, st, forwardLaunches(true));
             columnResidual(_cp, _C, _C.rhs, _x, _r, st);
             absMax(_r, n, _partial, rn, st);
             resid = hostScalar(rn, st);
@@ -800,6 +806,7 @@ bool PressureSolver::pcgReliable(double tolFactor, int maxIter, double resid0, d
             if (resid <= tol) return true;
             castToFloat(_r, _fr, n, st);
             sinceUpdate = resid;
+            _t->begin(T_MIC0_APPLY, st, applyLaunches(false));
             precondForward<float>(_fr, _fy, nullptr, st);  // again, from the replaced residual
         }
         precondBackward<float>(_fy, _fz, st);

@@ -53,11 +53,12 @@ public:
         _launches[id] = launches;
         (void)hipEventRecord(_cur[id], s);
     }
-    void end(int id, hipStream_t s) {
+    // launches: those since begin(), where that could not know
+    void end(int id, hipStream_t s, int launches = 0) {
         if (!_on) return;
         hipEvent_t e = take();
         (void)hipEventRecord(e, s);
-        _pending.push_back(Pending{id, _cur[id], e, _launches[id]});
+        _pending.push_back(Pending{id, _cur[id], e, launches > 0 ? launches : _launches[id]});
     }
     // wait for all recorded pairs and accumulate
     void collect() {

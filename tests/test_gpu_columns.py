@@ -86,3 +86,31 @@ def test_non_finite_values_stay_in_their_body(n3, value, schedule):
             got = K.mic0_apply(*args, r, precision=1, schedule=schedule).astype(np.float32)
         assert m // 3 <= np.isfinite(want).sum() < m
         agree(got, want)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32-preconditioner", "mixed", "mixed-reliable"])
+def test_every_sweep_is_timed(precision):
+    """The kernel timing of the MIC(0) application counts every sweep of a solve:
+    two an iteration and two before the first, but for a solve's last iteration
+    (mixed: each inner solve's), which runs the forward one; a replaced residual
+    (mixed-reliable) runs the forward one again."""
+    from ctypes import byref, c_double, c_int, c_longlong, c_void_p
+    from ffengine import scenes
+    from ffengine.ffengine import ffengine as lib
+    from test_gpu_engine import make_gpu
+    lib.FluidSimulation_enable_kernel_timing.argtypes = [c_void_p, c_int, c_void_p]
+    lib.FluidSimulation_get_kernel_timing.argtypes = [c_void_p, c_int, c_void_p, c_void_p, c_void_p]
+    sim = make_gpu(24, scenes.dam_break_particles(24, seed=3), precision=precision, tol=1e-8)
+    ok = c_int()
+    lib.FluidSimulation_enable_kernel_timing(sim(), 1, byref(ok))
+    assert ok.value
+    sim.step(1.0 / 240.0)
+    its = sim.get_last_pressure_solve_stats()["iterations"]
+    ms, launches = c_double(), c_longlong()
+    lib.FluidSimulation_get_kernel_timing(sim(), 7, byref(ms), byref(launches), byref(ok))
+    say(f"{precision}: {its} iterations, {launches.value} sweeps")
+    assert ok.value and its > 1 and ms.value > 0
+    if precision in ("fp64", "fp32-preconditioner"):
+        assert launches.value == 2 * its + 1
+    else:
+        assert 2 * its + 1 < launches.value <= 4 * its
