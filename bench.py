@@ -164,7 +164,8 @@ def algorithmic_bytes(name, n, P, M_total, launches_per_sub, substeps, iters_tot
     if name == "p2g":
         return substeps * (28 * P + 4 * N + 5 * F)          # 28 B/particle, 4 B/cell, 5 B/face
     if name == "spmv":
-        per = 24 if mode in ("mixed", "mixed-reliable") else 48  # 4 coefficients + x read + y write per row
+        # 4 coefficients, z and s read, the direction and its product written per row (z in FP32 beside FP64 vectors)
+        per = 32 if mode in ("mixed", "mixed-reliable") else 64 if mode == "fp64" else 60
         return per * M_total
     if name == "mic0_apply":
         per = 96 if mode == "fp64" else 48                    # both sweeps: r, invdiag, 3 L, z per row
@@ -180,9 +181,25 @@ def algorithmic_bytes(name, n, P, M_total, launches_per_sub, substeps, iters_tot
     return None
 
 
-def sweep_kernel_name(fp64):
-    """Template name of the MIC(0) sweep kernel the library runs for one precision (forward and backward launches)."""
-    return "columnSweepKernel<%s>" % ("double" if fp64 else "float")
+def sweep_kernel_name(fp64, schedule):
+    """The MIC(0) sweep kernel the library runs for one precision and schedule, with the shape it was built for
+    (columns: forward and backward launches; lines along j and k of a column, columns of a workgroup)."""
+    from ctypes import byref, c_int, c_void_p
+    from ffengine import pybindings as pb
+    from ffengine.ffengine import ffengine as lib
+    word = "double" if fp64 else "float"
+    a, b, c = c_int(), c_int(), c_int()
+    if schedule == 2:
+        f = lib.FFAMD_mic0_column_shape
+        pb.init_lib_func(f, [c_void_p] * 4, None)
+        pb.execute_lib_func(f, [byref(a), byref(b), byref(c)])
+        return "columnSweepKernel<%s> %dx%dx%d" % (word, a.value, b.value, c.value)
+    if schedule == 5:
+        f = lib.FFAMD_mic0_band_shape
+        pb.init_lib_func(f, [c_int, c_void_p, c_void_p, c_void_p], None)
+        pb.execute_lib_func(f, [1 if fp64 else 0, byref(a), byref(b)])
+        return "micBandKernel<%s, %d, %d>" % (word, a.value, b.value)
+    return "pencilSweepKernel<%s>" % word
 
 
 def measured_traffic(kernel):
@@ -754,7 +771,7 @@ def main():
     launches = max(kt[dom]["launches"], 1)
     traffic, kname = None, dom
     if dom == "mic0_apply":
-        kname = sweep_kernel_name(main_mode == "fp64")
+        kname = sweep_kernel_name(main_mode == "fp64", args.schedule or 2)
         traffic = measured_traffic(kname)
     # algorithmic HBM bytes / time of every kernel group that has a byte model
     # (SpMV, the transfers, the preconditioner, ...), as a fraction of 8 TB/s

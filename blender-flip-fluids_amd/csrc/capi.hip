@@ -1272,6 +1272,14 @@ void FFAMD_mic0_band_shape(int fp64, int *levels, int *tile, int *err) {
     });
 }
 
+void FFAMD_mic0_column_shape(int *linesJ, int *linesK, int *columns, int *err) {
+    guarded(err, [&] {
+        *linesJ = ff::COL_J;
+        *linesK = ff::COL_K;
+        *columns = ff::COL_WAVES;
+    });
+}
+
 int FFAMD_mic0_apply(int ni, int nj, int nk, double dx, double dt, const float *u, const float *v,
                      const float *w, const float *wu, const float *wv, const float *ww, const float *phi,
                      int precision, int schedule, int n, const double *r, double *z, int *err) {

@@ -535,6 +535,9 @@ int FFAMD_projection_vjp(int isize, int jsize, int ksize, double dx, double dt, 
  * the reference): hyperplanes per launch and tile side in lines, for the FP64
  * (fp64 = 1) or the FP32 factor. */
 void FFAMD_mic0_band_shape(int fp64, int *levels, int *tile, int *err);
+/* And of its column schedule: lines of a column along j and along k, columns
+ * of a workgroup. */
+void FFAMD_mic0_column_shape(int *lines_j, int *lines_k, int *columns, int *err);
 void FFAMD_sample_velocity(int isize, int jsize, int ksize, double dx, const float *u,
                            const float *v, const float *w, int np, const float *pos, float *out,
                            int *err);
