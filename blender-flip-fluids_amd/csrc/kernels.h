@@ -127,7 +127,7 @@ __device__ inline unsigned reduceLogicalBlock() {
 }
 // fold one double per thread of a REDUCE_THREADS block, OP 0 sum, 1 max, in a
 // fixed order: a wave64 butterfly (every lane ends with the same bits), then
-// the four wave results in wave order.  The result is valid in thread 0.
+// the four wave results in wave order, in every thread.
 template <int OP>
 __device__ inline double reduceFold(double v) {
     __shared__ double waves[REDUCE_THREADS / 64];
@@ -149,7 +149,7 @@ __device__ inline double reduceFold(double v) {
 // launch of one block has to come between (4 us of launch and drain a
 // reduction at any size; a block's fold is about 1.5 us at 1024 partials).
 // reduceFold's LDS is not guarded for a second use of the same OP in a kernel: a
-// barrier has to come between.
+// barrier has to come between.  (columnDirectionSpmvDotKernel has one.)
 template <int OP>
 __device__ inline double foldPartials(const double *partial, int nb) {
     double acc = 0.0;

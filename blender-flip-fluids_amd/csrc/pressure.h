@@ -126,16 +126,11 @@ private:
     void prepareRowSchedule(int schedule, bool fp64, hipStream_t s);
     void factor(bool fp64, hipStream_t st);
     void rowDot(const double *a, const double *b, double *out, hipStream_t st);
-    // schedule 5: executable graphs of the band launches for the (r, z)
-    // pairs of the current solve's applications (the PCG's z alternates
-    // between two buffers), dropped when a new system is assembled
-    struct BandGraph {
-        const void *r = nullptr, *z = nullptr;
-        hipGraphExec_t exec = nullptr;
-    };
-    BandGraph _graphs[2];
-    int _graphNext = 0;
-    void dropGraphs();
+    // schedule 5: the band launches of an application as an executable graph,
+    // recorded at the first application of a system (every application of it
+    // has the same operands), dropped when a new system is prepared
+    hipGraphExec_t _graph = nullptr;
+    void dropGraph();
     template <class T>
     void graphApply(const T *r, T *y, T *z, hipStream_t s);
     int _refDots = 0;  // thread count of the reference's dot order, or 0 for the tree reductions

@@ -12,7 +12,7 @@ namespace ff {
 void hipCheck(hipError_t e, const char *what);
 
 PressureSolver::~PressureSolver() {
-    dropGraphs();
+    dropGraph();
     if (_block) (void)hipFree(_block);
     if (_rowBlock) (void)hipFree(_rowBlock);
     if (_hostScal) (void)hipHostFree(_hostScal);
@@ -269,29 +269,19 @@ void PressureSolver::setSchedule(int schedule) {
     _sched = schedule;
 }
 
-void PressureSolver::dropGraphs() {
-    for (BandGraph &b : _graphs) {
-        if (b.exec) (void)hipGraphExecDestroy(b.exec);
-        b = BandGraph{};
-    }
-    _graphNext = 0;
+void PressureSolver::dropGraph() {
+    if (_graph) (void)hipGraphExecDestroy(_graph);
+    _graph = nullptr;
 }
 
 // The band launches of one application are the same for every application
-// of a solve (same plan, same buffers), so they are recorded once per (r, z)
-// pair by stream capture and replayed with one hipGraphLaunch.  The capture
-// holds kernel launches only.
+// of a solve (same plan, same buffers), so they are recorded once by stream
+// capture and replayed with one hipGraphLaunch.  The capture holds kernel
+// launches only.
 template <class T>
 void PressureSolver::graphApply(const T *r, T *y, T *z, hipStream_t s) {
     if (_S.m == 0) return;
-    BandGraph *slot = nullptr;
-    for (BandGraph &b : _graphs)
-        if (b.exec && b.r == r && b.z == z) slot = &b;
-    if (!slot) {
-        slot = &_graphs[_graphNext];
-        _graphNext = (_graphNext + 1) % 2;
-        if (slot->exec) (void)hipGraphExecDestroy(slot->exec);
-        *slot = BandGraph{};
+    if (!_graph) {
         hipGraph_t graph = nullptr;
         hipCheck(hipStreamBeginCapture(s, hipStreamCaptureModeRelaxed), "begin capture");
         try {
@@ -305,13 +295,12 @@ void PressureSolver::graphApply(const T *r, T *y, T *z, hipStream_t s) {
             throw;
         }
         hipCheck(hipStreamEndCapture(s, &graph), "end capture");
-        const hipError_t e = hipGraphInstantiate(&slot->exec, graph, nullptr, nullptr, 0);
+        const hipError_t e = hipGraphInstantiate(&_graph, graph, nullptr, nullptr, 0);
         (void)hipGraphDestroy(graph);
+        if (e != hipSuccess) _graph = nullptr;
         hipCheck(e, "instantiate the band graph");
-        slot->r = r;
-        slot->z = z;
     }
-    hipCheck(hipGraphLaunch(slot->exec, s), "launch the band graph");
+    hipCheck(hipGraphLaunch(_graph, s), "launch the band graph");
 }
 
 // the row-ordered schedules' operands of the current factor
@@ -329,7 +318,7 @@ void PressureSolver::prepareRowSchedule(int schedule, bool fp64, hipStream_t s) 
                      host ? _hTileHi.data() : nullptr, _plan);
         _bandLaunches = (int)_plan.l0.size();
     }
-    dropGraphs();  // recorded with the previous system's plan
+    dropGraph();  // recorded with the previous system's plan
 }
 
 // An application in two halves.  The forward half also publishes the largest
