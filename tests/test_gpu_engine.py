@@ -296,10 +296,10 @@ def test_removal_rules_match_oracle():
 
 @pytest.mark.parametrize("precision", ["fp64", "mixed", "fp32-preconditioner"])
 def test_preconditioner_schedules_give_the_same_bits(precision):
-    """Schedule 2 (one launch per band), 4 (the line pipeline) and 5 (the
-    bands recorded once per solve as a HIP graph and replayed) apply the same
-    operations to the same operands, so two frames of a dam break come out
-    bit for bit the same under each, in each PCG mode."""
+    """Schedule 2 (columns, one launch per sweep), 4 (the line pipeline) and 5
+    (bands of hyperplanes recorded once per solve as a HIP graph and replayed)
+    apply the same operations to the same operands, so two frames of a dam break
+    come out bit for bit the same under each, in each PCG mode."""
     n = 32
     pos = scenes.dam_break_particles(n, seed=3)
     out = {}

@@ -239,17 +239,40 @@ def _check_mic0_apply(n, schedule):
     assert same_bits(g32.astype(np.float32), _mic_sweeps(sysm, n3, r, np.float32))
 
 
-@pytest.mark.parametrize("schedule", [4, 2, 3, 0], ids=["line-pipeline", "bands", "bands-device-check",
+@pytest.mark.parametrize("schedule", [4, 2, 3, 0], ids=["line-pipeline", "columns", "bands-device-check",
                                                      "hyperplanes"])
 @pytest.mark.parametrize("n", CASES + [70])
 def test_mic0_apply_bitexact(n, schedule):
     """The preconditioner application as a line pipeline (pencils of lines
-    along i, one launch per sweep), in bands of hyperplanes (also with the tile
-    check on the device, the path of grids whose tiles outnumber a launch's
-    tile mask) and one launch per hyperplane, against the oracle's serial
-    sweeps (FP64) and a hyperplane-vectorised FP32 restatement (mixed
-    mode)."""
+    along i, one launch per sweep), in columns (the solver's: 16 x 8 lines, one
+    launch per sweep), in bands of hyperplanes with the tile check on the device
+    (the path of grids whose tiles outnumber a launch's tile mask) and one launch
+    per hyperplane, against the oracle's serial sweeps (FP64) and a
+    hyperplane-vectorised FP32 restatement (mixed mode).  Bands of tiles that the
+    host lists: test_band_schedule_bitexact."""
     _check_mic0_apply(n, schedule=schedule)
+
+
+@pytest.mark.parametrize("n", CASES + [70])
+def test_band_schedule_bitexact(n):
+    """Bands of the tiles that the host lists (solver schedule 5 runs them from a
+    graph): FFAMD_mic0_apply takes them where the columns' result is not finite
+    throughout.  Here a drop of one cell, alone in the far corner, holds an
+    infinity: all other rows are as without it."""
+    n3, dx, dt, uvw, weights, phi = _pressure_inputs(n)
+    assert (phi[n - 4:, n - 4:, n - 4:] > 0).all()
+    phi[n - 2, n - 2, n - 2] = -0.3 * dx
+    sysm = O.pressure_system(n3, dx, dt, uvw, weights, phi)
+    m = len(sysm["rows"])
+    r = np.random.default_rng(n).standard_normal(m)
+    r[-1] = np.inf
+    say(f"mic0_apply in bands n={n} rows={m}")
+    g64 = K.mic0_apply(n3, dx, dt, uvw, weights, phi, r, precision=0, schedule=2)
+    assert same_bits(g64[:-1], O.apply_mic0(sysm, r)[:-1]) and g64[-1] == np.inf
+    g32 = K.mic0_apply(n3, dx, dt, uvw, weights, phi, r, precision=1, schedule=2).astype(np.float32)
+    # the call adds the widened FP32 result to zeros: -0 comes back as +0
+    assert same_bits(g32[:-1], _mic_sweeps(sysm, n3, r, np.float32)[:-1] + np.float32(0)) and g32[-1] == np.inf
+    assert np.isfinite(g64[:-1]).all() and np.isfinite(g32[:-1]).all()
 
 
 @pytest.mark.skip(reason="tile-wavefront MIC(0) kernel switched off: under test it never finished (the compiled "
