@@ -1300,8 +1300,10 @@ int FFAMD_mic0_apply(int ni, int nj, int nk, double dx, double dt, const float *
         up(dphi.p, phi, N, sc.s);
         ff::PressureSolver ps;
         ps.allocate(g);
-        // one PCG iteration builds the system and the factor
-        ps.solve(dt, du, dv, dw, a, b, c, dphi, 1e-300, 1, precision, 1e-4, dp, scan, sc.s, nullptr);
+        // one PCG iteration builds the system and the factor; a zero right-hand
+        // side is not solved
+        if (ps.solve(dt, du, dv, dw, a, b, c, dphi, 1e-300, 1, precision, 1e-4, dp, scan, sc.s, nullptr).iterations == 0)
+            ps.factorSystem(precision == 0, sc.s);
         size_t m = (size_t)ps.system().m;
         if ((size_t)n != m)
             throw std::domain_error("r and z hold " + std::to_string(n) + " values; the system has " +
@@ -1350,8 +1352,9 @@ int FFAMD_pressure_system(int ni, int nj, int nk, double dx, double dt, const fl
         ff::PressureSolver ps;
         ps.allocate(g);
         // one PCG iteration builds the system and the factor; the tolerance is
-        // irrelevant for the system itself
-        ps.solve(dt, du, dv, dw, a, b, c, dphi, 1e-300, 1, 0, 1e-4, dp, scan, sc.s, nullptr);
+        // irrelevant for the system itself.  A zero right-hand side is not solved.
+        if (ps.solve(dt, du, dv, dw, a, b, c, dphi, 1e-300, 1, 0, 1e-4, dp, scan, sc.s, nullptr).iterations == 0)
+            ps.factorSystem(true, sc.s);
         const ff::PressureSys &S = ps.system();
         size_t m = (size_t)S.m;
         down(rows, S.rows, m, sc.s);

@@ -64,6 +64,9 @@ public:
     void setSchedule(int schedule);
     int schedule() const { return _sched; }
     const std::vector<int> &levelTable() const { return _hLevelStart; }
+    // the MIC(0) factor of the last solve()'s system, which a solve that had
+    // nothing to solve did not need
+    void factorSystem(bool fp64, hipStream_t s);
     // one preconditioner application z = (L L^T)^-1 r on the current factor
     // (after solve()); FP64 or the FP32 copy; r and z in row order.
     // schedule 0 = one launch per hyperplane, 1 = tile wavefront (switched

@@ -548,6 +548,10 @@ void PressureSolver::factor(bool fp64, hipStream_t st) {
     _t->end(T_MIC0_FACTOR, st);
 }
 
+void PressureSolver::factorSystem(bool fp64, hipStream_t s) {
+    if (_S.m > 0) factor(fp64, s);
+}
+
 // a . b in the reference's summation order: over the rows
 void PressureSolver::rowDot(const double *a, const double *b, double *out, hipStream_t st) {
     ensureRowSchedules();

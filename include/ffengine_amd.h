@@ -484,8 +484,7 @@ int FFAMD_pressure_system(int isize, int jsize, int ksize, double dx, double dt,
  * error, 2 = columns of 16 x 8 lines along i, one launch per triangular sweep
  * (the solver's), 3 = bands of hyperplanes with each workgroup reading its
  * tile's hyperplane range on the device, 4 = the line pipeline (pencils of
- * 16 x 16 lines along i, one launch per triangular sweep).  The inputs must give a non-zero
- * divergence.  Returns M. */
+ * 16 x 16 lines along i, one launch per triangular sweep).  Returns M. */
 int FFAMD_mic0_apply(int isize, int jsize, int ksize, double dx, double dt, const float *u,
                      const float *v, const float *w, const float *wu, const float *wv,
                      const float *ww, const float *liquid_phi, int precision, int schedule,

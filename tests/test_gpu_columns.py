@@ -88,6 +88,28 @@ def test_non_finite_values_stay_in_their_body(n3, value, schedule):
         agree(got, want)
 
 
+def test_a_system_without_divergence_has_its_factor():
+    """The matrix and its factor do not depend on the velocities: with none, so
+    that there is nothing to solve, the factor and its application are the
+    oracle's all the same."""
+    n3, dx = (20, 18, 19), 1.0 / 20
+    rng = np.random.default_rng(1)
+    phi = _liquid("scattered", n3, rng)
+    weights = O.face_weights(n3, O.solid_box_phi(n3, dx))
+    ni, nj, nk = n3
+    uvw = [np.zeros(s, np.float32) for s in ((nk, nj, ni + 1), (nk, nj + 1, ni), (nk + 1, nj, ni))]
+    args = n3, dx, 1.0 / 120.0, uvw, weights, phi
+    sysm = O.pressure_system(*args)
+    r = rng.standard_normal(len(sysm["rows"]))
+    say(f"no divergence: {len(r)} rows")
+    assert not sysm["rhs"].any()
+    assert same_bits(K.pressure_system(*args)["invdiag"], sysm["invdiag"])
+    for schedule in (2, 4, 3, 0):
+        assert same_bits(K.mic0_apply(*args, r, precision=0, schedule=schedule), O.apply_mic0(sysm, r))
+        got = K.mic0_apply(*args, r, precision=1, schedule=schedule).astype(np.float32)
+        assert same_bits(got, _mic_sweeps(sysm, n3, r, np.float32) + np.float32(0))
+
+
 @pytest.mark.parametrize("precision", ["fp64", "fp32-preconditioner", "mixed", "mixed-reliable"])
 def test_every_sweep_is_timed(precision):
     """The kernel timing of the MIC(0) application counts every sweep of a solve:
