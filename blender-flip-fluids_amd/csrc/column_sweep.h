@@ -47,11 +47,16 @@
 // Measured, one application (both sweeps) FP64 / FP32, against launches over
 // bands of 8 / 12 hyperplanes: 24^3 99 / 86 -> 42 / 35 us, 64^3 237 / 201 ->
 // 108 / 80, 128^3 513 / 441 -> 217 / 162, 256^3 dam break 1267 / 1058 -> 473 /
-// 353.  Two lines a lane and two waves a tile were the fastest of (lines,
-// waves) = (1,4) (2,2) (2,4) (4,1) (4,2) (2,1): 167 / 223 us FP32 / FP64 for a
-// sweep of 96 x 160 x 256, the others 160 / 297 to 199 / 360 (all before the
-// head of the loop matched its steps, see columnSteps).  A 16 x 16 tile with
-// an LDS plane and a barrier per step took 0.22 us a step against 0.15.
+// 353.  A forward sweep FP32 / FP64 by (lines a lane, waves a tile), us:
+//              24^3       64^3       100^3       96x160x256
+//   (2, 2)  20.0/26.5  52.3/70.5   85.3/114.3   151/204   taken
+//   (2, 1)  18.8/34.9  48.9/95.9   79.9/147.9   142/264
+//   (2, 4)  20.8/27.9  53.4/85.7   86.6/137.4   153/238
+//   (1, 2)  19.6/23.6  53.4/64.3   87.1/102.1   165/198
+//   (1, 4)  20.5/25.3  55.1/66.2   91.3/105.4   169/199
+// One shape serves both precisions, since FP64 vectors and FP32 sweeps share a
+// layout; (4, 1) and (4, 2) were slower still.  A 16 x 16 tile with an LDS plane
+// and a barrier per step took 0.22 us a step against 0.15.
 //
 // This header holds only the sweep's body; its includer supplies the hardware
 // operations as macros: column_hw.h the GPU's, tests/emu/column_emu.cpp ones

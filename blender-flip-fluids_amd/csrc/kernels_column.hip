@@ -21,9 +21,15 @@ namespace ff {
 
 namespace {
 
-// Steps whose operands, and whose neighbours' words, are in flight.  A sweep of
-// 96 x 160 x 256, FP32 / FP64: 6 and 3 151 / 205 us, 6 and 4 - / 210, 8 and 3 151,
-// 8 and 4 155 / 213, 8 and 6 164.
+// Steps whose operands, and whose neighbours' words, are in flight.  A forward
+// sweep FP32 / FP64, us:
+//             24^3       64^3      96x160x256
+//    6, 3  20.0/26.4  52.4/70.4   151/203   taken (the fewest registers)
+//    6, 2  23.3/27.2  60.5/71.9   160/198
+//    6, 4  19.9/27.0  52.0/72.0   153/210
+//    8, 3  19.6/26.0  51.4/69.4   150/202
+//    8, 4  19.9/26.8  52.4/71.8   154/211
+//   12, 3  21.5/28.4  53.6/72.5   151/205
 constexpr int CPF = 6, CPX = 3;
 // A wait's limit.  A look at a ring takes about 0.1 us, one at a word 0.7 us: 2 s
 // and 14 s, where a whole sweep takes 1 ms.
