@@ -136,3 +136,32 @@ def test_every_sweep_is_timed(precision):
         assert launches.value == 2 * its + 1
     else:
         assert 2 * its + 1 < launches.value <= 4 * its
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_two_simulations_at_once(precision):
+    """Two threads, each with a simulation of its own: their sweeps wait on the
+    device for their own tiles only, and each frame is the one it is alone."""
+    import threading
+    from ffengine import scenes
+    from test_gpu_engine import gpu_particles, make_gpu
+    sizes = (33, 48)
+
+    def run(n, out):
+        sim = make_gpu(n, scenes.dam_break_particles(n, seed=n), precision=precision, tol=1e-8)
+        for _ in range(3):
+            sim.update(1.0 / 60.0)
+        out[n] = [a.copy() for a in gpu_particles(sim)]
+
+    alone, together = {}, {}
+    for n in sizes:
+        run(n, alone)
+    say(f"{precision}: two simulations at once")
+    team = [threading.Thread(target=run, args=(n, together)) for n in sizes]
+    for t in team:
+        t.start()
+    for t in team:
+        t.join()
+    for n in sizes:
+        for a, b in zip(alone[n], together[n]):
+            assert np.array_equal(a.view(np.uint32), b.view(np.uint32)), n
