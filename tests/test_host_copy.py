@@ -27,4 +27,7 @@ def emulator(tmp_path_factory):
 
 @pytest.mark.parametrize("threads", [1, 3])
 def test_read_back_from_threads(emulator, threads):
-    subprocess.run([emulator, str(threads)], check=True, timeout=300)
+    done = subprocess.run([emulator, str(threads)], capture_output=True, text=True, timeout=300)
+    if "unexpected memory mapping" in done.stderr:
+        pytest.skip("ThreadSanitizer does not run with this kernel's address layout")
+    assert done.returncode == 0, done.stderr
