@@ -31,8 +31,8 @@ namespace {
 //    8, 4  19.9/26.8  52.4/71.8   154/211
 //   12, 3  21.5/28.4  53.6/72.5   151/205
 constexpr int CPF = 6, CPX = 3;
-// A wait's limit.  A look at a ring takes about 0.1 us, one at a word 0.7 us: 2 s
-// and 14 s, where a whole sweep takes 1 ms.
+// A wait's limit.  A look takes the latency of LDS (a ring) or of device memory (a
+// word), some 0.05 to 0.7 us: 1 s at least, where a whole sweep takes 1 ms.
 constexpr int WAIT_LOOKS = 20000000;
 constexpr int EMPTY_LO = 0x3fffffff;
 

@@ -229,8 +229,8 @@ int FluidSimulation_get_pressure_solver_warm_start(FluidSimulation *obj, int *er
  * the row order, recorded once per solve as a HIP graph and replayed.  All give
  * the same bits; 4 and 5 convert between the solver's layout and the row order
  * around each application.  In 2 and 4 workgroups wait for each other's results
- * on the device; a wait past its limit (2: 20 million looks, some seconds of
- * device time; 4: 2 seconds) makes the call fail with an error. */
+ * on the device; a wait past its limit (2: 20 million looks, a second of
+ * device time or more; 4: 2 seconds) makes the call fail with an error. */
 void FluidSimulation_set_pressure_solver_preconditioner_schedule(FluidSimulation *obj, int schedule,
                                                                  int *err);
 int FluidSimulation_get_pressure_solver_preconditioner_schedule(FluidSimulation *obj, int *err);
